@@ -9,13 +9,18 @@
 // [B, H, U, V]). One pass over the pair tensor z replaces the reference's LayerNorm
 // output, linear output and permuted copy.
 //
-// Layout: eight lanes per pixel (a wave holds 8 consecutive pixels of the flattened
-// [B, U, V] grid), lane j of a pixel loading the 16-byte channel chunks j, j + 8, ... of its
-// row, so a wave's loads cover 8 whole contiguous pixel rows. Mean and variance are reduced
-// over the 8 lanes with xor shuffles (two passes over the registers). The projection
-// weights sit in LDS as fp32 [H][Zc]; each lane forms its channels' partial dot product for
-// a head, the 8 partials meet through three xor shuffles, and lane h % 8 stores head h.
-// The kernel is HBM-bound (Zc * e bytes read per pixel against H * e written).
+// Layout: a wave takes 32 consecutive pixels of the flattened [B, U, V] grid. Their rows are
+// one contiguous range of z, read in memory order (whole lines per instruction; reading the
+// fragments straight from memory takes 32 bytes of each of 32 lines per instruction, and the
+// lines fall out of L1 before their other parts are used) and passed through a wave-private LDS
+// tile into the MFMA's B fragment: two lanes per pixel, lane half g holding the 8-channel chunks
+// 16 kk + 8 g (k = channel, column = pixel). Mean and variance are one exchange between the two
+// lanes, and the projection is [32 heads][Zc] x [Zc][32 pixels] with the weights as A fragments
+// (heads past H repeat the last one and are not stored; chunks past Zc are zero on both sides).
+// The result has a pixel per lane, so each head's 32 values leave as one run. Bound by HBM
+// (Zc * e bytes read per pixel against H * e written). The matrix unit replaced eight-lane dot
+// products on the vector ALU (H * Zc / 8 FMAs with an LDS read each and three shuffles per head
+// and lane): 54 -> 18.4 us at 384 x 384 pixels, Zc = 128, H = 16, bf16.
 //
 // Also here: the gate and output projection of attention with pair bias (apb_gate_out_kernel,
 // below), the part of the op after the attention itself.
@@ -28,105 +33,148 @@ namespace gnn {
 
 namespace {
 
-constexpr int PB_THREADS = 256;              // 4 waves
-constexpr int PB_PIX = PB_THREADS / 8;       // pixels per workgroup iteration
-constexpr int PB_MAX_CHUNKS = 4;             // Zc <= 256
-constexpr int PB_MAX_W = 8192;               // H * Zc <= 8192 (32 KB of fp32 weights)
+constexpr int PB_MAX_ZC = 256;
+constexpr int PB_MAX_W = 8192;               // H * Zc <= 8192
 
+// 8 consecutive elements: one vector load where the array is 16-byte aligned, else scalar loads
 template <typename T>
-__global__ __launch_bounds__(PB_THREADS) void pair_bias_proj_kernel(const gnn_pair_bias_args a) {
-  __shared__ float ws[PB_MAX_W];
-  __shared__ float gs[PB_MAX_CHUNKS * 64];
-  const int Zc = (int)a.Zc, H = (int)a.H, V = (int)a.V, U = (int)a.U;
-  const int tid = threadIdx.x;
-  for (int i = tid; i < H * Zc; i += PB_THREADS) ws[i] = TypeOps<T>::to_f32(((const T*)a.proj_w)[i]);
-  for (int i = tid; i < Zc; i += PB_THREADS)
-    gs[i] = a.ln_w ? TypeOps<T>::to_f32(((const T*)a.ln_w)[i]) : 1.0f;
-  __syncthreads();
+__device__ __forceinline__ typename TypeOps<T>::V8 load8_any(const T* p, bool aligned) {
+  if (aligned) return load8(p);
+  typename TypeOps<T>::V8 v;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = p[e];
+  return v;
+}
 
-  const int j = tid & 7;
-  const int nch = Zc / 8;
-  const int64_t npix = a.B * (int64_t)U * V;
+// KS k-steps of 16 channels (Zc <= 16 * KS); waves per workgroup such that the LDS tiles of
+// 32 padded rows each take at most 36 KB
+template <typename T, int KS>
+struct PairBiasCfg {
+  static constexpr int PITCH = 16 * KS * (int)sizeof(T) + 16;  // bytes
+  static constexpr int NW = PITCH * 32 <= 9 * 1024 ? 4 : PITCH * 32 <= 18 * 1024 ? 2 : 1;
+  static constexpr int CHUNKS = KS * (int)sizeof(T) / 2;       // 16-byte chunks per lane
+};
+
+template <typename T, int KS>
+__global__ __launch_bounds__((64 * PairBiasCfg<T, KS>::NW), (sizeof(T) == 2 && KS <= 8 ? 4 : 1)) void pair_bias_proj_kernel(const gnn_pair_bias_args a) {
+  typedef typename TypeOps<T>::V8 V8;
+  typedef PairBiasCfg<T, KS> Cfg;
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  constexpr int PREC = sizeof(T) == 4 ? PREC_IEEE : PREC_NATIVE;
+  __shared__ __align__(16) unsigned char tiles[Cfg::NW * 32 * Cfg::PITCH];
+  const int Zc = (int)a.Zc, H = (int)a.H;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5, wave = threadIdx.x >> 6;
+  unsigned char* tile = tiles + wave * 32 * Cfg::PITCH;
+  const int64_t npix = a.B * a.U * a.V;
+  const int64_t p0 = ((int64_t)blockIdx.x * Cfg::NW + wave) * 32, p = p0 + l32;
+  const bool ok = p < npix;
+
+  // the 32 rows in memory order; rows past the last pixel repeat the last chunk
+  const int cpr = Zc * (int)sizeof(T) / 16;  // 16-byte chunks per row
+  const int64_t left = (npix - (p0 < npix ? p0 : npix - 1)) * cpr - 1;
+  const u32x4_t* src = (const u32x4_t*)a.z + (p0 < npix ? p0 : npix - 1) * cpr;
+  u32x4_t raw[Cfg::CHUNKS];
+#pragma unroll
+  for (int i = 0; i < Cfg::CHUNKS; ++i) {
+    const int c = 64 * i + lane;
+    raw[i] = src[c < left ? c : left];
+  }
+  // the first 32 heads' weights, requested before the rows are waited for
+  const bool wal = ((uintptr_t)a.proj_w & 15) == 0;
+  V8 w[KS];
+  auto weights = [&](int h0) {
+    const T* wrow = (const T*)a.proj_w + (int64_t)(h0 + l32 < H ? h0 + l32 : H - 1) * Zc + 8 * g;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) w[kk] = 16 * kk + 8 * g < Zc ? load8_any(wrow + 16 * kk, wal) : zero8<T>();
+  };
+  weights(0);
+#pragma unroll
+  for (int i = 0; i < Cfg::CHUNKS; ++i) {
+    const int c = 64 * i + lane;
+    const int r = Zc == 16 * KS ? c / (KS * (int)sizeof(T)) : c / cpr;
+    if (r < 32) *reinterpret_cast<u32x4_t*>(tile + r * Cfg::PITCH + (c - r * cpr) * 16) = raw[i];
+  }
+  // Each pass over the row reads it from LDS again (the compiler would otherwise keep the
+  // fp32 copies of all channels live and spill)
+  auto chunk = [&](int kk) {
+    return 16 * kk + 8 * g < Zc ? load8((const T*)(tile + l32 * Cfg::PITCH) + 16 * kk + 8 * g) : zero8<T>();
+  };
+  auto next_pass = [] {
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+  };
+  next_pass();
   const float inv_zc = 1.0f / (float)Zc;
-  for (int64_t p0 = (int64_t)blockIdx.x * PB_PIX; p0 < npix; p0 += (int64_t)gridDim.x * PB_PIX) {
-    const int64_t p = p0 + (tid >> 3);
-    const bool ok = p < npix;
-    const T* row = (const T*)a.z + (ok ? p : 0) * Zc;
-    f32x8 x[PB_MAX_CHUNKS];
-    float s = 0.f;
+  float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
-      const int ch = j + 8 * c;
-      if (ch < nch) {
-        x[c] = TypeOps<T>::to_f32(load8(row + 8 * ch));
+  for (int kk = 0; kk < KS; ++kk) {
+    const f32x8 v = TypeOps<T>::to_f32(chunk(kk));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s += x[c][e];
-      }
+    for (int e = 0; e < 8; ++e) s += v[e];
+  }
+  const float mean = pair_sum(s) * inv_zc;
+  next_pass();
+  float q = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) {
+    const f32x8 v = TypeOps<T>::to_f32(chunk(kk));
+    float t = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t += (v[e] - mean) * (v[e] - mean);
+    q += 16 * kk + 8 * g < Zc ? t : 0.f;
+  }
+  const float rstd = 1.0f / sqrtf(pair_sum(q) * inv_zc + a.eps);
+  next_pass();
+  // normalised, gamma-scaled and rounded to the input dtype (F.layer_norm's output)
+  const T* gam = (const T*)a.ln_w;
+  const bool gal = ((uintptr_t)gam & 15) == 0;
+  V8 x[KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) {
+    const int ch = 16 * kk + 8 * g;
+    x[kk] = zero8<T>();
+    if (ch < Zc) {
+      f32x8 v = TypeOps<T>::to_f32(chunk(kk));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (v[e] - mean) * rstd;
+      if (gam) v *= TypeOps<T>::to_f32(load8_any(gam + ch, gal));
+      x[kk] = TypeOps<T>::from_f32(v);
     }
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    s += __shfl_xor(s, 4);
-    const float mean = s * inv_zc;
-    float q = 0.f;
+  }
+
+  const uint32_t V = (uint32_t)a.V, U = (uint32_t)a.U;
+  const uint64_t r = (uint64_t)(ok ? p : 0) / V;
+  const uint32_t v0 = (uint32_t)((uint64_t)(ok ? p : 0) - r * V);
+  T* orow = (T*)a.out + (int64_t)(r / U) * a.out_stride[0] + (int64_t)(r % U) * a.out_stride[2] + v0;
+  for (int h0 = 0; h0 < H; h0 += 32) {
+    if (h0 > 0) weights(h0);
+    f32x16 acc;
 #pragma unroll
-    for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
-      if (j + 8 * c < nch) {
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float d = x[c][e] - mean;
-          q += d * d;
-        }
-      }
-    }
-    q += __shfl_xor(q, 1);
-    q += __shfl_xor(q, 2);
-    q += __shfl_xor(q, 4);
-    const float rstd = 1.0f / sqrtf(q * inv_zc + a.eps);
-    // normalised, gamma-scaled and rounded to the input dtype (F.layer_norm's output)
+    for (int kk = 0; kk < KS; ++kk) Mma<T, PREC>::step(acc, w[kk], x[kk]);
 #pragma unroll
-    for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
-      const int ch = j + 8 * c;
-      if (ch < nch) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          x[c][e] = TypeOps<T>::to_f32(TypeOps<T>::from_f32((x[c][e] - mean) * rstd * gs[8 * ch + e]));
-      }
-    }
-    int64_t b = 0, u = 0, v = 0;
-    if (ok) {
-      v = p % V;
-      const int64_t r = p / V;
-      u = r % U;
-      b = r / U;
-    }
-    T* orow = (T*)a.out + b * a.out_stride[0] + u * a.out_stride[2] + v;
-    for (int h = 0; h < H; ++h) {
-      const float* wh = ws + h * Zc;
-      float acc = 0.f;
-#pragma unroll
-      for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
-        const int ch = j + 8 * c;
-        if (ch < nch) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(x[c][e], wh[8 * ch + e], acc);
-        }
-      }
-      acc += __shfl_xor(acc, 1);
-      acc += __shfl_xor(acc, 2);
-      acc += __shfl_xor(acc, 4);
-      if (ok && (h & 7) == j) orow[h * a.out_stride[1]] = TypeOps<T>::from_f32(acc);
+    for (int i = 0; i < 16; ++i) {
+      const int h = h0 + 8 * (i / 4) + 4 * g + i % 4;
+      if (ok && h < H) orow[h * a.out_stride[1]] = TypeOps<T>::from_f32(acc[i]);
     }
   }
 }
 
+template <typename T, int KS>
+int launch_pb(const gnn_pair_bias_args& a, hipStream_t stream) {
+  constexpr int pix = 32 * PairBiasCfg<T, KS>::NW;
+  const int64_t grid = (a.B * a.U * a.V + pix - 1) / pix;
+  if (grid >= ((int64_t)1 << 31)) return set_error(GNN_ERR_UNSUPPORTED, "pair_bias_proj: too many pixels");
+  hipLaunchKernelGGL((pair_bias_proj_kernel<T, KS>), dim3((uint32_t)grid), dim3(2 * pix), 0, stream, a);
+  return (int)hipGetLastError();
+}
+// the channel loops unroll over 64, 128 or 256 channels
 template <typename T>
 int launch_pb(const gnn_pair_bias_args& a, hipStream_t stream) {
-  const int64_t npix = a.B * a.U * a.V;
-  const int64_t want = (npix + PB_PIX - 1) / PB_PIX;
-  const int grid = (int)std::min<int64_t>(want, (int64_t)persistent_grid((const void*)pair_bias_proj_kernel<T>,
-                                                                          PB_THREADS, 0) * 4);
-  hipLaunchKernelGGL(pair_bias_proj_kernel<T>, dim3(grid < 1 ? 1 : grid), dim3(PB_THREADS), 0, stream, a);
-  return (int)hipGetLastError();
+  if (a.Zc <= 64) return launch_pb<T, 4>(a, stream);
+  if (a.Zc <= 128) return launch_pb<T, 8>(a, stream);
+  return launch_pb<T, 16>(a, stream);
 }
 
 // ---- gate and output projection ------------------------------------------------------
@@ -346,7 +394,7 @@ int apb_gate_out(const gnn_apb_gate_out_args& a, hipStream_t stream) {
 }
 
 int pair_bias_proj(const gnn_pair_bias_args& a, hipStream_t stream) {
-  if (a.Zc % 8 != 0 || a.Zc > 8 * PB_MAX_CHUNKS * 8)
+  if (a.Zc % 8 != 0 || a.Zc > PB_MAX_ZC)
     return set_error(GNN_ERR_UNSUPPORTED, "pair_bias_proj: c_z must be a multiple of 8 and at most 256");
   if (a.H * a.Zc > PB_MAX_W)
     return set_error(GNN_ERR_UNSUPPORTED, "pair_bias_proj: heads * c_z must be at most 8192");
