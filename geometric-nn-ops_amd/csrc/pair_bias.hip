@@ -180,29 +180,28 @@ int launch_pb(const gnn_pair_bias_args& a, hipStream_t stream) {
 // ---- gate and output projection ------------------------------------------------------
 //   out = ( T(o) * T(sigmoid(T(s Wg^T + bg))) ) Wo^T + bo,
 // each product's result rounded to T as the reference's F.linear / torch.sigmoid / multiply
-// return it (attention_pair_bias.py:86-89). One workgroup (4 waves) per GT = 32 tokens:
+// return it (attention_pair_bias.py:86-89). One workgroup (NW waves) per GT = 32 tokens:
 // the tile's s rows and its o rows (the attention output, heads merged) are staged in LDS;
-// gate pre-activations run on MFMA in passes of 128 channels (wave w: channels 32 w ..,
+// gate pre-activations run on MFMA in passes of 32 NW channels (wave w: channels 32 w ..,
 // A = Wg rows from global memory, fetched a chunk of k-steps ahead, B = s fragments from
 // LDS), and each lane writes o * g over
 // the o values it read, so the gated tile never leaves LDS; the output product then reads it
 // as its B operand and its results leave through an LDS staging tile as 16-byte rows. No
 // intermediate (g, o * g) reaches memory.
 constexpr int GT = 32;       // tokens per workgroup
-constexpr int GOC = 128;     // output channels per pass (4 waves x 32)
-constexpr int GO_THREADS = 256;
 
 struct GateOutLds {
-  size_t s, og, y, bias, total;
+  size_t s, og, y, bias;
 };
+// goc: output channels per pass, 32 per wave
 template <typename T>
-__host__ __device__ inline GateOutLds gate_out_lds(int64_t Cs, int64_t D) {
+__host__ __device__ inline GateOutLds gate_out_lds(int64_t Cs, int64_t D, int goc) {
   constexpr int pad = 16 / (int)sizeof(T);
   GateOutLds L;
   L.s = 0;
   L.og = L.s + (size_t)GT * (Cs + pad) * sizeof(T);
   L.y = L.og + (size_t)GT * (D + pad) * sizeof(T);
-  L.bias = L.y + (size_t)GT * (GOC + pad) * sizeof(T);
+  L.bias = L.y + (size_t)GT * (goc + pad) * sizeof(T);
   return L;
 }
 // the biases follow as fp32 [D] and [Co]
@@ -246,16 +245,17 @@ __device__ __forceinline__ void gate_out_gemm(f32x16& acc, const T* __restrict__
   else gate_out_gemm<T, PREC, 2>(acc, wrow, nk, tile, ld, l32, g);  // widths are multiples of 32: nk is even
 }
 
-template <typename T, int PREC>
-__global__ __launch_bounds__(GO_THREADS) void apb_gate_out_kernel(const gnn_apb_gate_out_args a) {
+template <typename T, int PREC, int NW>
+__global__ __launch_bounds__(64 * NW) void apb_gate_out_kernel(const gnn_apb_gate_out_args a) {
   typedef typename TypeOps<T>::V8 V8;
   typedef typename TypeOps<T>::V4 V4;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr int pad = 16 / (int)sizeof(T);
   constexpr int EPC = 16 / (int)sizeof(T);  // elements per 16-byte chunk
+  constexpr int GO_THREADS = 64 * NW, GOC = 32 * NW;
   const int Cs = (int)a.Cs, D = (int)a.D, Co = (int)a.Co;
   const int SR = Cs + pad, OR = D + pad, YR = GOC + pad;
-  const GateOutLds L = gate_out_lds<T>(Cs, D);
+  const GateOutLds L = gate_out_lds<T>(Cs, D, GOC);
   T* ss = reinterpret_cast<T*>(smem_raw + L.s);
   T* og = reinterpret_cast<T*>(smem_raw + L.og);
   T* ys = reinterpret_cast<T*>(smem_raw + L.y);
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(GO_THREADS) void apb_gate_out_kernel(const gnn_apb_
 
   // stage s [GT][Cs] and o [GT][D] (16-byte chunks, zeros past the last token), SB chunks
   // per thread loaded before any is stored, so their latencies overlap
-  constexpr int SB = 8;
+  constexpr int SB = NW == 4 ? 8 : 2;
   typedef typename std::conditional<sizeof(T) == 2, V8, V4>::type Vc;  // 16 bytes of T
   auto stage = [&](const T* src, int64_t ld, int C, T* dst, int R) {
     const int cpr = C / EPC, n = GT * cpr;
@@ -362,14 +362,32 @@ __global__ __launch_bounds__(GO_THREADS) void apb_gate_out_kernel(const gnn_apb_
   }
 }
 
-template <typename T, int PREC>
-int launch_gate_out(const gnn_apb_gate_out_args& a, hipStream_t stream) {
-  const size_t smem = gate_out_lds_total(gate_out_lds<T>(a.Cs, a.D), a.D, a.Co);
-  const void* fn = (const void*)apb_gate_out_kernel<T, PREC>;
+template <typename T, int PREC, int NW>
+int launch_gate_out(const gnn_apb_gate_out_args& a, hipStream_t stream, size_t smem) {
+  const void* fn = (const void*)apb_gate_out_kernel<T, PREC, NW>;
   if (smem > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-  hipLaunchKernelGGL((apb_gate_out_kernel<T, PREC>), dim3((uint32_t)((a.M + GT - 1) / GT)), dim3(GO_THREADS), smem,
+  hipLaunchKernelGGL((apb_gate_out_kernel<T, PREC, NW>), dim3((uint32_t)((a.M + GT - 1) / GT)), dim3(64 * NW), smem,
                      stream, a);
   return (int)hipGetLastError();
+}
+
+constexpr size_t GO_MAX_LDS = 160 * 1024;
+
+// Waves per workgroup. A call has one workgroup per 32 tokens, so few that most CUs stay idle
+// and its time is one workgroup's chain of weight loads and MFMAs per pass of 32 channels a
+// wave: widths above 128 take as many waves as the registers allow (16; 8 for fp32, whose
+// fragments are twice as wide), so that D = 384 is one pass instead of three; narrower ones
+// and widths whose tiles would not fit in LDS beside the wider output pass take 4.
+// 384 tokens, c_s = D = 384, bf16: 25.6 -> 21.9 us.
+template <typename T, int PREC>
+int launch_gate_out(const gnn_apb_gate_out_args& a, hipStream_t stream) {
+  constexpr int NW = sizeof(T) == 2 ? 16 : 8;
+  const size_t wide = gate_out_lds_total(gate_out_lds<T>(a.Cs, a.D, 32 * NW), a.D, a.Co);
+  if ((a.D > 128 || a.Co > 128) && wide <= GO_MAX_LDS) return launch_gate_out<T, PREC, NW>(a, stream, wide);
+  const size_t smem = gate_out_lds_total(gate_out_lds<T>(a.Cs, a.D, 128), a.D, a.Co);
+  if (smem > GO_MAX_LDS)
+    return set_error(GNN_ERR_UNSUPPORTED, "apb_gate_out: c_s + attention width too large for the LDS tiles");
+  return launch_gate_out<T, PREC, 4>(a, stream, smem);
 }
 
 }  // namespace
@@ -377,11 +395,6 @@ int launch_gate_out(const gnn_apb_gate_out_args& a, hipStream_t stream) {
 int apb_gate_out(const gnn_apb_gate_out_args& a, hipStream_t stream) {
   if (a.Cs % 32 != 0 || a.D % 32 != 0 || a.Co % 32 != 0)
     return set_error(GNN_ERR_UNSUPPORTED, "apb_gate_out: c_s, the attention width and c_out must be multiples of 32");
-  const size_t e = a.dtype == GNN_F32 ? 4 : 2;
-  const size_t lds = gate_out_lds_total(e == 2 ? gate_out_lds<bf16>(a.Cs, a.D) : gate_out_lds<float>(a.Cs, a.D), a.D,
-                                        a.Co);
-  if (lds > 160 * 1024)
-    return set_error(GNN_ERR_UNSUPPORTED, "apb_gate_out: c_s + attention width too large for the LDS tiles");
   if (a.M >= ((int64_t)1 << 31) * GT) return set_error(GNN_ERR_UNSUPPORTED, "apb_gate_out: too many tokens");
   switch (a.dtype) {
     case GNN_BF16: return launch_gate_out<bf16, PREC_NATIVE>(a, stream);

@@ -46,3 +46,23 @@ def test_pair_bias_projection_tiles(Zc, H, U, V, dtype):
     got = pair_bias_projection_hip(z.to(DEV), None, w.to(DEV), 1e-5)
     want = O.pair_bias_projection(to_np(z), to_np(torch.ones(Zc)), to_np(w), 1e-5)
     assert O.rel_fro(to_np(got), want) <= TOL[dtype]
+
+
+@DTYPES
+@pytest.mark.parametrize(("M", "Cs", "D", "Co"), [(1, 32, 128, 128), (33, 64, 160, 32), (31, 384, 384, 384),
+                                                  (40, 96, 544, 576), (32, 1024, 1024, 64)])
+def test_gate_out_widths(M, Cs, D, Co, dtype):
+    """Widths at and past one pass of four waves and of the wide workgroup, and the largest tiles,
+    which leave no LDS for the wide output pass."""
+    from geometric_nn_ops_torch.triangle._kernels.attention_pair_bias import gate_out_hip
+
+    if dtype == torch.float32 and Cs + D > 1024:
+        Cs = D = 512
+    g = gen(200 + D)
+    r = lambda *shape, scale=1.0: (torch.randn(*shape, generator=g) * scale).to(dtype)  # noqa: E731
+    s, o, gw, ow = r(M, Cs), r(M, D), r(D, Cs, scale=Cs ** -0.5), r(Co, D, scale=D ** -0.5)
+    gb, ob = r(D, scale=0.3), r(Co, scale=0.3)
+    got = gate_out_hip(*(t.to(DEV) for t in (s, o, gw, gb, ow, ob)))
+    q = to_np
+    want = O.linear(q(o) * O.sigmoid(O.linear(q(s), q(gw), q(gb))), q(ow), q(ob))
+    assert O.rel_fro(to_np(got), want) <= TOL[dtype]
