@@ -1569,20 +1569,28 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_pp_kernel(const gnn_trimul
 }
 
 // ============================== stage 2: per-channel contraction ==========================
-template <typename T>
+// fp32 under ieee: BM x BM output tiles, 4 waves of BM / 2 x BM / 2, one stage of 32 k held in
+// registers while the previous one multiplies. Columns N .. NP - 1 of a and b are zeros, so the
+// loads run to NP without a tail. Bound by the fp32 matrix rate (64 cycles per 32x32x2), so the
+// tile edge is chosen for the least padding: 64 where ceil(N / 64) is odd and at most 7 (128
+// planes, N = 64: 10.1 -> 4.9 us, 131: 30.0 -> 21.0, 300: 116 -> 90, 430: 270 -> 229), 128 otherwise
+// (half the cache bytes per flop at the same padded area; N = 690, 11 tiles of 64: 835 against 843).
+template <typename T, int BM_>
 struct ContractCfg {
-  static constexpr int BM = 128, BN = 128;
-  static constexpr int BK = sizeof(T) == 2 ? 64 : 32;  // 128 B of k per row per stage
+  static constexpr int BM = BM_, BN = BM_;
+  static constexpr int BK = 32;  // 128 B of k per row per stage
   static constexpr int ROW = BK + lds_pad<T>();
+  static constexpr int WT = BM / 64;  // 32 x 32 tiles per wave and dimension
 };
 
-template <typename T, int PREC>
+template <typename T, int PREC, int BM>
 __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restrict__ A,
                                                                 const T* __restrict__ Bm,
                                                                 T* __restrict__ O, int N,
                                                                 int64_t NP) {
   typedef typename TypeOps<T>::V8 V8;
-  typedef ContractCfg<T> Cfg;
+  typedef ContractCfg<T, BM> Cfg;
+  constexpr int WT = Cfg::WT;
   __shared__ __align__(16) T as[Cfg::BM * Cfg::ROW];
   __shared__ __align__(16) T bs[Cfg::BN * Cfg::ROW];
 
@@ -1611,18 +1619,9 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restr
       const int r = c / CPR, kc = k0 + (c % CPR) * 8;
       ra[i] = zero8<T>();
       rb[i] = zero8<T>();
-      if (kc < N) {
-        if (kc + 8 <= N) {
-          if (i0 + r < N) ra[i] = load8(Ap + (int64_t)(i0 + r) * NP + kc);
-          if (j0 + r < N) rb[i] = load8(Bp + (int64_t)(j0 + r) * NP + kc);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (kc + e < N) {
-              if (i0 + r < N) ra[i][e] = Ap[(int64_t)(i0 + r) * NP + kc + e];
-              if (j0 + r < N) rb[i][e] = Bp[(int64_t)(j0 + r) * NP + kc + e];
-            }
-        }
+      if (kc < NP) {
+        if (i0 + r < N) ra[i] = load8(Ap + (int64_t)(i0 + r) * NP + kc);
+        if (j0 + r < N) rb[i] = load8(Bp + (int64_t)(j0 + r) * NP + kc);
       }
     }
   };
@@ -1636,11 +1635,11 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restr
     }
   };
 
-  f32x16 acc[2][2];
+  f32x16 acc[WT][WT];
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+  for (int x = 0; x < WT; ++x)
 #pragma unroll
-    for (int y = 0; y < 2; ++y)
+    for (int y = 0; y < WT; ++y)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[x][y][r] = 0.f;
 
@@ -1653,33 +1652,33 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restr
     if (has_next) load((kt + 1) * Cfg::BK);
 #pragma unroll
     for (int kk = 0; kk < Cfg::BK / 16; ++kk) {
-      V8 af[2], bf[2];
+      V8 af[WT], bf[WT];
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
-        af[x] = load8(&as[(64 * wm + 32 * x + l32) * Cfg::ROW + 16 * kk + 8 * g]);
+      for (int x = 0; x < WT; ++x)
+        af[x] = load8(&as[(32 * WT * wm + 32 * x + l32) * Cfg::ROW + 16 * kk + 8 * g]);
 #pragma unroll
-      for (int y = 0; y < 2; ++y)
-        bf[y] = load8(&bs[(64 * wn + 32 * y + l32) * Cfg::ROW + 16 * kk + 8 * g]);
+      for (int y = 0; y < WT; ++y)
+        bf[y] = load8(&bs[(32 * WT * wn + 32 * y + l32) * Cfg::ROW + 16 * kk + 8 * g]);
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int x = 0; x < WT; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) Mma<T, PREC>::step(acc[x][y], af[x], bf[y]);
+        for (int y = 0; y < WT; ++y) Mma<T, PREC>::step(acc[x][y], af[x], bf[y]);
     }
     __syncthreads();
     if (has_next) store();
     __syncthreads();
   }
 
-  // acc[x][y][r] = o[i0 + 64wm + 32x + 8(r/4) + 4g + r%4][j0 + 64wn + 32y + l32]
+  // acc[x][y][r] = o[i0 + (BM/2)wm + 32x + 8(r/4) + 4g + r%4][j0 + (BM/2)wn + 32y + l32]
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+  for (int x = 0; x < WT; ++x)
 #pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      const int j = j0 + 64 * wn + 32 * y + l32;
+    for (int y = 0; y < WT; ++y) {
+      const int j = j0 + 32 * WT * wn + 32 * y + l32;
       if (j >= N) continue;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int i = i0 + 64 * wm + 32 * x + 8 * (r / 4) + 4 * g + (r % 4);
+        const int i = i0 + 32 * WT * wm + 32 * x + 8 * (r / 4) + 4 * g + (r % 4);
         if (i < N) Op[(int64_t)i * NP + j] = TypeOps<T>::from_f32(acc[x][y][r]);
       }
     }
@@ -2672,17 +2671,21 @@ int launch_contract(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t
     if (a.N >= GNN_CONTRACT_BM256_N) return launch_contract_dma<T, 256>(a, L, st, NP);
     return launch_contract_dma<T, 128>(a, L, st, NP);
   }
-  typedef ContractCfg<T> Cfg;
-  const int64_t nblk = a.B * a.Ch * ((a.N + Cfg::BM - 1) / Cfg::BM) * ((a.N + Cfg::BN - 1) / Cfg::BN);
-  unsigned char* ws = (unsigned char*)a.workspace;
   if constexpr (sizeof(T) == 4 && PREC == PREC_BF16X3) {
     return launch_contract_x3(a, L, st, NP);
-  } else {
-    hipLaunchKernelGGL((trimul_contract_kernel<T, PREC>), dim3((uint32_t)nblk), dim3(NT), 0, st,
-                       (const T*)(ws + L.off_a), (const T*)(ws + L.off_b), (T*)(ws + L.off_o), (int)a.N,
-                       NP);
+  } else if constexpr (sizeof(T) == 4) {
+    unsigned char* ws = (unsigned char*)a.workspace;
+    auto run = [&](auto bm) {
+      constexpr int BM = decltype(bm)::value;
+      const int64_t nt = (a.N + BM - 1) / BM;
+      hipLaunchKernelGGL((trimul_contract_kernel<T, PREC, BM>), dim3((uint32_t)(a.B * a.Ch * nt * nt)), dim3(NT), 0,
+                         st, (const T*)(ws + L.off_a), (const T*)(ws + L.off_b), (T*)(ws + L.off_o), (int)a.N, NP);
+      return (int)hipGetLastError();
+    };
+    if (a.N <= 448 && (a.N + 63) / 64 % 2 == 1) return run(std::integral_constant<int, 64>{});
+    return run(std::integral_constant<int, 128>{});
   }
-  return (int)hipGetLastError();
+  return GNN_OK;
 }
 
 template <typename T, int PREC, int CK, int CHK>

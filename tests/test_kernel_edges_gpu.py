@@ -5,7 +5,7 @@ fp32 2^-24 relative), and the bounds below allow for the two or three roundings 
 import pytest
 import torch
 
-from helpers import gen, to_np
+from helpers import gen, np_weights, pair_input, to_np, trimul_weights
 from oracle import triangle_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +66,38 @@ def test_gate_out_widths(M, Cs, D, Co, dtype):
     q = to_np
     want = O.linear(q(o) * O.sigmoid(O.linear(q(s), q(gw), q(gb))), q(ow), q(ob))
     assert O.rel_fro(to_np(got), want) <= TOL[dtype]
+
+
+# --------------------------------------------------------------- multiplicative update, forward
+def _trimul_forward_error(N, C, Ch, dtype, direction, B=1):
+    """Worst relative error of the forward over sampled rows and columns (first, last and the ones
+    at tile edges)."""
+    from geometric_nn_ops_torch.triangle import triangle_multiplicative_update
+
+    w = trimul_weights(C, Ch, dtype, seed=N, biases=True, ln_random=True)
+    x, mask = pair_input(B, N, C, dtype, seed=N + 1)
+    with torch.no_grad():
+        got = triangle_multiplicative_update(x.to(DEV), direction, mask.to(DEV), **{k: v.to(DEV) for k, v in w.items()})
+    at = sorted({i for i in (0, 31, 32, 63, 64, 127, 128, 191, N - 1) if i < N})
+    want = O.trimul_grid(to_np(x), direction, to_np(mask), at, at, **np_weights(w))
+    return O.rel_fro(to_np(got[:, at][:, :, at]), want)
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+@pytest.mark.parametrize("N", [1, 33, 64, 65, 129, 192, 193, 449])
+def test_fp32_contraction_tiles(N, direction):
+    """Both tile edges of the full-precision contraction, at and past their multiples."""
+    assert _trimul_forward_error(N, 32, 32, torch.float32, direction) <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+@pytest.mark.parametrize(("dtype", "N", "C", "Ch", "B"), [
+    # one to four workgroups on a tile (256 compute units over N ceil(N / 64) B tiles)
+    (torch.float32, 3, 128, 128, 1), (torch.float32, 64, 128, 128, 1), (torch.float32, 45, 128, 128, 2),
+    (torch.float32, 40, 256, 96, 1), (torch.float32, 64, 64, 32, 1), (torch.bfloat16, 33, 256, 128, 1),
+    (torch.bfloat16, 64, 96, 160, 1), (torch.float16, 63, 32, 256, 2),
+    # full-precision weights held in registers: both widths, c_hidden below c_z, row tails
+    (torch.float32, 130, 128, 128, 1), (torch.float32, 91, 128, 128, 2), (torch.float32, 131, 128, 64, 1),
+    (torch.float32, 135, 64, 128, 1)])
+def test_projection_dispatch(dtype, N, C, Ch, B, direction):
+    assert _trimul_forward_error(N, C, Ch, dtype, direction, B) <= TOL[dtype]
