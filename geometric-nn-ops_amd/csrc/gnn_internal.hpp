@@ -10,6 +10,9 @@ namespace gnn {
 // Records `msg` as this thread's last error and returns `code`.
 int set_error(int code, const char* msg);
 
+// Compute units of the current device, at least 1.
+int compute_units();
+
 // Resident workgroups of a persistent kernel on the current device: occupancy x CU count,
 // at least 1.
 int persistent_grid(const void* fn, int threads, size_t smem);

@@ -259,7 +259,8 @@ struct LnWidth {
 // Chunks of x per thread that the tile load must hold: ceil(C / 64), rounded up to 2, 4, 8.
 __host__ __device__ inline int proj_xm(int64_t C) { return C <= 128 ? 2 : C <= 256 ? 4 : 8; }
 
-template <typename T, int PREC, int XM>
+// SPLIT: gridDim.y workgroups share a tile's units (proj_split)
+template <typename T, int PREC, int XM, bool SPLIT>
 __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_args a, int64_t NP,
                                                              size_t off_a, size_t off_b,
                                                              size_t off_g) {
@@ -375,6 +376,8 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_ar
   // ---- projections of one tile
   const int nk = C / 16;
   const int npg = 2 * Ch / 32, ngo = C / 32;
+  constexpr int PGRP = PSUB / SPT;  // passes of a projection unit over the tile
+  const int split = SPLIT ? (int)gridDim.y : 1, part = SPLIT ? (int)blockIdx.y : 0;
   T* __restrict__ a_cm = (T*)((unsigned char*)a.workspace + off_a);
   T* __restrict__ b_cm = (T*)((unsigned char*)a.workspace + off_b);
   T* __restrict__ gout = (T*)(a.gate ? (unsigned char*)a.gate : (unsigned char*)a.workspace + off_g);
@@ -388,7 +391,18 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_ar
   auto compute = [&](const Tile& tl) {
     // gated projection units: acc = [pixel][channel], row = pixel 32s + 8(r/4) + 4g + r%4,
     // col = channel 32u + l32; staged as [channel][pixel] for 128-byte row stores
-    for (int u = wave; u < npg; u += PW) {
+    for (int j = 0;; ++j) {
+      int u, s0;  // unit, first sub-tile
+      if constexpr (!SPLIT) {
+        u = wave + PW * (j / PGRP);
+        s0 = SPT * (j % PGRP);
+        if (u >= npg) break;
+      } else {
+        const int it = part + split * (wave + PW * j);
+        if (it >= npg * PGRP) break;
+        u = it % npg;
+        s0 = SPT * (it / npg);
+      }
       const int ch = 32 * u + l32;
       const T* wprow = wp + (int64_t)ch * C + 8 * g;
       const T* wgrow = wg + (int64_t)ch * C + 8 * g;
@@ -406,64 +420,65 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_ar
         if (nk <= KCH) load_w(0);
         wp_unit = u;
       }
-      for (int s0 = 0; s0 < PSUB; s0 += SPT) {
 #pragma unroll
-        for (int s2 = 0; s2 < SPT; ++s2) {
-          const int s = s0 + s2;
-          f32x16 accp, accg;
+      for (int s2 = 0; s2 < SPT; ++s2) {
+        const int s = s0 + s2;
+        f32x16 accp, accg;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            accp[r] = bp;
-            accg[r] = bg;
-          }
-          for (int kc = 0; kc < nk; kc += KCH) {
-            if (nk > KCH) load_w(kc);
+        for (int r = 0; r < 16; ++r) {
+          accp[r] = bp;
+          accg[r] = bg;
+        }
+        for (int kc = 0; kc < nk; kc += KCH) {
+          if (nk > KCH) load_w(kc);
 #pragma unroll
-            for (int j = 0; j < KCH; ++j) {
-              if (kc + j >= nk) break;
-              const V8 zf = load8(&zs[(32 * s + l32) * ZR + 16 * (kc + j) + 8 * g]);
-              Mma<T, PREC>::step(accp, zf, wpf[j]);
-              Mma<T, PREC>::step(accg, zf, wgf[j]);
-            }
-          }
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            const int pt = 8 * rg + 4 * g;  // pixel within the sub-tile
-            const f32x4 m4 = *reinterpret_cast<const f32x4*>(&mk[32 * s + pt]);
-            f32x4 v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = accp[4 * rg + e] * sigmoid_acc(accg[4 * rg + e]) * m4[e];
-            store4(&ebuf[l32 * ER + 32 * s2 + pt], TypeOps<T>::from_f32(v));
+          for (int j = 0; j < KCH; ++j) {
+            if (kc + j >= nk) break;
+            const V8 zf = load8(&zs[(32 * s + l32) * ZR + 16 * (kc + j) + 8 * g]);
+            Mma<T, PREC>::step(accp, zf, wpf[j]);
+            Mma<T, PREC>::step(accg, zf, wgf[j]);
           }
         }
-        wave_lds_sync();
-        // 16-byte stores, 4 * SPT lanes per channel row of 32 * SPT pixels
 #pragma unroll
-        for (int i = 0; i < 2 * SPT; ++i) {
-          const int c = lane + 64 * i;
-          const int crow = c / (4 * SPT), p0 = (c % (4 * SPT)) * 8;
-          const int chg = 32 * u + crow;
-          T* dst = chg < Ch ? a_cm : b_cm;
-          const int chh = chg < Ch ? chg : chg - Ch;
-          const int pl = 32 * s0 + p0;
-          T* drow = dst + ab_offset<T>((int64_t)tl.b * Ch + chh, tl.row, tl.c0 + pl, N, NP);
-          const V8 val = load8(&ebuf[crow * ER + p0]);
-          if (tl.c0 + pl + 8 <= N) {
-            store8(drow, val);
-          } else if (tl.c0 + pl < NP) {  // row tail: pixels N .. NP-1 are written as zeros
-            V8 v = val;
+        for (int rg = 0; rg < 4; ++rg) {
+          const int pt = 8 * rg + 4 * g;  // pixel within the sub-tile
+          const f32x4 m4 = *reinterpret_cast<const f32x4*>(&mk[32 * s + pt]);
+          f32x4 v;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (tl.c0 + pl + e >= N) v[e] = TypeOps<T>::from_f32(0.f);
-            store8(drow, v);
-          }
+          for (int e = 0; e < 4; ++e) v[e] = accp[4 * rg + e] * sigmoid_acc(accg[4 * rg + e]) * m4[e];
+          store4(&ebuf[l32 * ER + 32 * s2 + pt], TypeOps<T>::from_f32(v));
         }
-        wave_lds_sync();
       }
+      wave_lds_sync();
+      // 16-byte stores, 4 * SPT lanes per channel row of 32 * SPT pixels
+#pragma unroll
+      for (int i = 0; i < 2 * SPT; ++i) {
+        const int c = lane + 64 * i;
+        const int crow = c / (4 * SPT), p0 = (c % (4 * SPT)) * 8;
+        const int chg = 32 * u + crow;
+        T* dst = chg < Ch ? a_cm : b_cm;
+        const int chh = chg < Ch ? chg : chg - Ch;
+        const int pl = 32 * s0 + p0;
+        T* drow = dst + ab_offset<T>((int64_t)tl.b * Ch + chh, tl.row, tl.c0 + pl, N, NP);
+        const V8 val = load8(&ebuf[crow * ER + p0]);
+        if (tl.c0 + pl + 8 <= N) {
+          store8(drow, val);
+        } else if (tl.c0 + pl < NP) {  // row tail: pixels N .. NP-1 are written as zeros
+          V8 v = val;
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (tl.c0 + pl + e >= N) v[e] = TypeOps<T>::from_f32(0.f);
+          store8(drow, v);
+        }
+      }
+      wave_lds_sync();
     }
     // output-gate items (unit uo, sub-tile s): acc = [channel][pixel], row = channel
     // 32uo + 8(r/4) + 4g + r%4, col = pixel 32s + l32; staged as [pixel][channel]
-    for (int it = wave; it < ngo * PSUB; it += PW) {
+    for (int j = 0;; ++j) {
+      const int it = SPLIT ? part + split * (wave + PW * j) - npg * PGRP : wave + PW * j;
+      if (SPLIT && it < 0) continue;
+      if (it >= ngo * PSUB) break;
       const int uo = it % ngo, s = it / ngo;
       const int c00 = 32 * uo;
       const T* wrow = wgo + (int64_t)(c00 + l32) * C + 8 * g;
@@ -539,16 +554,62 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_ar
   }
 }
 
-// ---- stage 1, fp32 under bf16x3: C = CK in {64, 128}, c_hidden <= 128 ---------------------
-// The generic kernel's tile walk, two-barrier LayerNorm and epilogues, with every MFMA
-// operand split into bf16 hi / lo halves once instead of at each product: z where the
-// LayerNorm writes it to LDS (two bf16 planes), a wave's projection weights (its one unit:
-// 32 rows of p_in and of g_in, 2 Ch / 32 <= PW) when the launch starts (registers, for the
-// whole launch) and the output-gate weights when the workgroup starts (two bf16 planes in
-// LDS). The MFMA loops then only read fragments; a product is lo*hi + hi*lo + hi*hi in fp32
-// accumulators. Accumulators start at zero and the biases join after the product.
+// ---- stage 1, fp32: C = CK in {64, 128}, c_hidden <= 128 -----------------------------------
+// The generic kernel's tile walk, two-barrier LayerNorm and epilogues, with every weight read
+// once per launch: a wave's projection weights (its one unit: 32 rows of p_in and of g_in,
+// 2 Ch / 32 <= PW; 128 registers at CK = 128) stay in registers and the output-gate weights in
+// LDS. The MFMA loops then only read LDS fragments. The generic kernel fetches the weights of
+// four k-steps at a time inside its products, and each of those waits (the memory counter is in
+// order) also waits for the next tile's x and for the stores of the previous unit; ieee at
+// c_z = c_hidden = 128: N = 201 124 -> 99 us, N = 384 281 -> 206 us, where the matrix unit
+// alone needs 154 (64 cycles per fp32 32x32x2).
+// X3 (bf16x3): every operand is split into bf16 hi / lo halves once instead of at each product,
+// z where the LayerNorm writes it to LDS (two bf16 planes), the weights where they are loaded; a
+// product is lo*hi + hi*lo + hi*hi in fp32 accumulators. Otherwise (ieee) z and the gate weights
+// are fp32 planes of at most the same size. Accumulators start at zero and the biases join after
+// the product.
+template <bool X3>
+struct F32Frag;  // 8 consecutive k of one row
+template <>
+struct F32Frag<true> {
+  bf16x8 h, l;
+  __device__ __forceinline__ void split(const f32x8& v) { split_bf16(v, h, l); }
+};
+template <>
+struct F32Frag<false> {
+  f32x8 v;
+  __device__ __forceinline__ void split(const f32x8& x) { v = x; }
+};
+// A plane of rows in LDS: hi / lo bf16 planes `lo` bytes apart, or one fp32 plane
+template <bool X3, int CK>
+struct F32Plane {
+  static constexpr int ROW = X3 ? CK + 8 : CK + 4;  // elements per row (16 B of padding)
+  unsigned char* base;
+  size_t lo;
+  __device__ __forceinline__ F32Frag<X3> get(int row, int k) const {
+    F32Frag<X3> f;
+    if constexpr (X3) {
+      f.h = load8((const bf16*)base + row * ROW + k);
+      f.l = load8((const bf16*)(base + lo) + row * ROW + k);
+    } else {
+      f.v = load8((const float*)base + row * ROW + k);
+    }
+    return f;
+  }
+  __device__ __forceinline__ void put(int row, int k, const f32x8& v) const {
+    if constexpr (X3) {
+      bf16x8 h, l;
+      split_bf16(v, h, l);
+      store8((bf16*)base + row * ROW + k, h);
+      store8((bf16*)(base + lo) + row * ROW + k, l);
+    } else {
+      store8((float*)base + row * ROW + k, v);
+    }
+  }
+};
+
 template <int CK>
-struct ProjX3Lds {
+struct ProjF32Lds {
   static constexpr int ZB = CK + 8;  // bf16 per z / gate-weight row (16 B of padding)
   static constexpr int ER = 32 + 4;  // fp32 per staging row
   static constexpr size_t zh = 0;
@@ -574,19 +635,17 @@ __device__ __forceinline__ f32x16 mfma_bf16(const bf16x8& a, const bf16x8& b, co
 // lanes past the row, so no memory access sits in a branch: with one, the compiler's
 // memory-counter waits at the join count the path without it, and the waits for the next
 // tile's loads also wait for the stores issued after them.
-template <int CK, bool FIXED>
-__global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul_args a, int64_t NP,
+template <int CK, bool FIXED, bool X3>
+__global__ __launch_bounds__(PNT, 1) void trimul_proj_f32_kernel(const gnn_trimul_args a, int64_t NP,
                                                                 size_t off_a, size_t off_b, size_t off_g) {
-  typedef ProjX3Lds<CK> S;
+  typedef ProjF32Lds<CK> S;
+  typedef F32Frag<X3> Frag;
   constexpr int XM = CK / 64;  // 8-channel chunks of x per thread
   constexpr int NK = CK / 16;  // k-steps
-  constexpr int ZB = S::ZB, ER = S::ER;
+  constexpr int ER = S::ER;
   constexpr int NGO = CK / 32;  // output-gate units
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  bf16* zh = reinterpret_cast<bf16*>(smem_raw + S::zh);
-  bf16* zl = reinterpret_cast<bf16*>(smem_raw + S::zl);
-  bf16* woh = reinterpret_cast<bf16*>(smem_raw + S::woh);
-  bf16* wol = reinterpret_cast<bf16*>(smem_raw + S::wol);
+  const F32Plane<X3, CK> zs{smem_raw + S::zh, S::zl - S::zh}, wos{smem_raw + S::woh, S::wol - S::woh};
   float2* red = reinterpret_cast<float2*>(smem_raw + S::red);
   float* lnw = reinterpret_cast<float*>(smem_raw + S::lnw);
   float* lnb = reinterpret_cast<float*>(smem_raw + S::lnb);
@@ -601,7 +660,7 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul
   const bool outgoing = a.outgoing != 0;
   const int64_t ntiles = (int64_t)a.B * N * ((N + PTP - 1) / PTP);
 
-  // ---- once per workgroup: LayerNorm parameters, gate-out weights (split) and biases
+  // ---- once per workgroup: LayerNorm parameters, gate-out weights and biases
   for (int c = tid; c < CK; c += PNT) {
     lnw[c] = ld_or<float>(a.ln_in_w, c, 1.f);
     lnb[c] = ld_or<float>(a.ln_in_b, c, 0.f);
@@ -609,17 +668,14 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul
   }
   for (int c = tid; c < CK * CK / 8; c += PNT) {
     const int row = c / (CK / 8), k0 = (c % (CK / 8)) * 8;
-    bf16x8 hi, lo;
-    split_bf16(load8((const float*)a.g_out_w + (int64_t)row * CK + k0), hi, lo);
-    store8(&woh[row * ZB + k0], hi);
-    store8(&wol[row * ZB + k0], lo);
+    wos.put(row, k0, load8((const float*)a.g_out_w + (int64_t)row * CK + k0));
   }
-  // ---- once per wave: its projection unit's weights, split (B operand: column = channel
+  // ---- once per wave: its projection unit's weights (B operand: column = channel
   // 32 * wave + l32, k = 16 kk + 8 g + e)
   static_assert(!FIXED || (CK == 128 && NGO * PSUB == PW), "FIXED: one unit and one gate item per wave");
   const int npg = 2 * Ch / 32;
   const bool has_unit = FIXED || wave < npg;  // uniform over the wave
-  bf16x8 wph[NK], wpl[NK], wgh[NK], wgl[NK];
+  Frag wpf[NK], wgf[NK];
   float bp = 0.f, bg = 0.f;
   {
     const int ch = has_unit ? 32 * wave + l32 : 0;
@@ -627,8 +683,8 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul
     const float* wgrow = (const float*)a.g_in_w + (int64_t)ch * CK + 8 * g;
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
-      split_bf16(load8(wprow + 16 * k), wph[k], wpl[k]);
-      split_bf16(load8(wgrow + 16 * k), wgh[k], wgl[k]);
+      wpf[k].split(load8(wprow + 16 * k));
+      wgf[k].split(load8(wgrow + 16 * k));
     }
     bp = ld_or<float>(a.p_in_b, ch, 0.f);
     bg = ld_or<float>(a.g_in_b, ch, 0.f);
@@ -695,10 +751,7 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul
         v[e] = (xr[j][e] - mean_r) * rstd * w0[e] + b0[e];
         v[e + 4] = (xr[j][e + 4] - mean_r) * rstd * w1[e] + b1[e];
       }
-      bf16x8 hi, lo;
-      split_bf16(v, hi, lo);
-      store8(&zh[xpl * ZB + 8 * ci], hi);
-      store8(&zl[xpl * ZB + 8 * ci], lo);
+      zs.put(xpl, 8 * ci, v);
     }
     if (tid < PTP) mk[tid] = mreg.value();
   };
@@ -719,14 +772,21 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul
         if (FIXED) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int k = 0; k < NK; ++k) {
-          const int o = (32 * s + l32) * ZB + 16 * k + 8 * g;
-          const bf16x8 h = load8(&zh[o]), l = load8(&zl[o]);
-          accp = mfma_bf16(l, wph[k], accp);
-          accg = mfma_bf16(l, wgh[k], accg);
-          accp = mfma_bf16(h, wpl[k], accp);
-          accg = mfma_bf16(h, wgl[k], accg);
-          accp = mfma_bf16(h, wph[k], accp);
-          accg = mfma_bf16(h, wgh[k], accg);
+          const Frag z = zs.get(32 * s + l32, 16 * k + 8 * g);
+          if constexpr (X3) {
+            accp = mfma_bf16(z.l, wpf[k].h, accp);
+            accg = mfma_bf16(z.l, wgf[k].h, accg);
+            accp = mfma_bf16(z.h, wpf[k].l, accp);
+            accg = mfma_bf16(z.h, wgf[k].l, accg);
+            accp = mfma_bf16(z.h, wpf[k].h, accp);
+            accg = mfma_bf16(z.h, wgf[k].h, accg);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              accp = __builtin_amdgcn_mfma_f32_32x32x2f32(z.v[e], wpf[k].v[e], accp, 0, 0, 0);
+              accg = __builtin_amdgcn_mfma_f32_32x32x2f32(z.v[e], wgf[k].v[e], accg, 0, 0, 0);
+            }
+          }
         }
         if (FIXED) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
@@ -794,18 +854,20 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_x3_kernel(const gnn_trimul
     for (int it = wave; FIXED || it < NGO * PSUB; it += PW) {  // FIXED: item `wave`, always
       const int uo = it % NGO, s = it / NGO;
       const int c00 = 32 * uo;
-      f32x16 accx, acch;  // cross terms, hi * hi
+      f32x16 accx, acch;  // X3: cross terms, hi * hi
 #pragma unroll
       for (int r = 0; r < 16; ++r) accx[r] = acch[r] = 0.f;
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
-        const int ow = (c00 + l32) * ZB + 16 * k + 8 * g;
-        const int oz = (32 * s + l32) * ZB + 16 * k + 8 * g;
-        const bf16x8 whf = load8(&woh[ow]), wlf = load8(&wol[ow]);
-        const bf16x8 zhf = load8(&zh[oz]), zlf = load8(&zl[oz]);
-        accx = mfma_bf16(wlf, zhf, accx);
-        acch = mfma_bf16(whf, zhf, acch);
-        accx = mfma_bf16(whf, zlf, accx);
+        const Frag w = wos.get(c00 + l32, 16 * k + 8 * g), z = zs.get(32 * s + l32, 16 * k + 8 * g);
+        if constexpr (X3) {
+          accx = mfma_bf16(w.l, z.h, accx);
+          acch = mfma_bf16(w.h, z.h, acch);
+          accx = mfma_bf16(w.h, z.l, accx);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acch = __builtin_amdgcn_mfma_f32_32x32x2f32(w.v[e], z.v[e], acch, 0, 0, 0);
+        }
       }
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
@@ -2525,19 +2587,6 @@ size_t out_smem(const gnn_trimul_args& a) {
   return out_lds_bytes(a.Ch, sizeof(T));
 }
 
-template <typename T, int PREC, int XM>
-int launch_proj_xm(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st) {
-  const int64_t NP = round_up(a.N, 32);
-  const int64_t ntiles = a.B * a.N * ((a.N + PTP - 1) / PTP);
-  const size_t smem = proj_lds<T>(a.C).total;
-  const void* fn = (const void*)trimul_proj_kernel<T, PREC, XM>;
-  if (smem > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-  const int64_t grid = std::min<int64_t>(ntiles, persistent_grid(fn, PNT, smem));
-  hipLaunchKernelGGL((trimul_proj_kernel<T, PREC, XM>), dim3((uint32_t)grid), dim3(PNT), smem, st, a, NP,
-                     L.off_a, L.off_b, L.off_g);
-  return (int)hipGetLastError();
-}
-
 template <typename T, int CK, int CHK>
 int launch_proj_fast(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st) {
   const int64_t NP = round_up(a.N, 32);
@@ -2567,17 +2616,45 @@ int launch_proj_pp(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t 
   return (int)hipGetLastError();
 }
 
-template <int CK, bool FIXED>
-int launch_proj_x3(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st) {
+template <int CK, bool FIXED, bool X3>
+int launch_proj_f32(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st) {
   const int64_t NP = round_up(a.N, 32);
   const int64_t ntiles = a.B * a.N * ((a.N + PTP - 1) / PTP);
-  constexpr size_t smem = ProjX3Lds<CK>::total;
-  const void* fn = (const void*)trimul_proj_x3_kernel<CK, FIXED>;
+  constexpr size_t smem = ProjF32Lds<CK>::total;
+  const void* fn = (const void*)trimul_proj_f32_kernel<CK, FIXED, X3>;
   (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   const int64_t grid = std::min<int64_t>(ntiles, persistent_grid(fn, PNT, smem));
-  hipLaunchKernelGGL((trimul_proj_x3_kernel<CK, FIXED>), dim3((uint32_t)grid), dim3(PNT), smem, st, a, NP,
+  hipLaunchKernelGGL((trimul_proj_f32_kernel<CK, FIXED, X3>), dim3((uint32_t)grid), dim3(PNT), smem, st, a, NP,
                      L.off_a, L.off_b, L.off_g);
   return (int)hipGetLastError();
+}
+
+// Workgroups that share a tile of the generic kernel: few tiles leave most CUs idle while each
+// workgroup multiplies for long (fp32 above all: 64 cycles per 32x32x2), so up to 4 workgroups
+// split a tile's units then, as long as all of them still have a CU to themselves. Each
+// normalises the tile for itself. fp32, N = 64, c_z = c_hidden = 128: 34 -> 17 us.
+int64_t proj_split(const gnn_trimul_args& a) {
+  const int64_t ntiles = a.B * a.N * ((a.N + PTP - 1) / PTP);
+  return std::max<int64_t>(1, std::min<int64_t>(4, compute_units() / ntiles));
+}
+
+template <typename T, int PREC, int XM, bool SPLIT>
+int launch_proj_xm(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st, int64_t split) {
+  const int64_t NP = round_up(a.N, 32);
+  const int64_t ntiles = a.B * a.N * ((a.N + PTP - 1) / PTP);
+  const size_t smem = proj_lds<T>(a.C).total;
+  const void* fn = (const void*)trimul_proj_kernel<T, PREC, XM, SPLIT>;
+  if (smem > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  const int64_t grid = std::min<int64_t>(ntiles, persistent_grid(fn, PNT, smem));
+  hipLaunchKernelGGL((trimul_proj_kernel<T, PREC, XM, SPLIT>), dim3((uint32_t)grid, (uint32_t)split), dim3(PNT), smem,
+                     st, a, NP, L.off_a, L.off_b, L.off_g);
+  return (int)hipGetLastError();
+}
+template <typename T, int PREC, int XM>
+int launch_proj_xm(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st) {
+  const int64_t split = proj_split(a);
+  return split > 1 ? launch_proj_xm<T, PREC, XM, true>(a, L, st, split)
+                   : launch_proj_xm<T, PREC, XM, false>(a, L, st, 1);
 }
 
 #ifndef GNN_PROJX3_FIXED
@@ -2585,13 +2662,15 @@ int launch_proj_x3(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t 
 #endif
 template <typename T, int PREC>
 int launch_proj(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st) {
-  if constexpr (sizeof(T) == 4 && PREC == PREC_BF16X3) {
-    if (2 * a.Ch <= 32 * PW) {  // one projection unit per wave
+  if constexpr (sizeof(T) == 4) {
+    constexpr bool X3 = PREC == PREC_BF16X3;
+    // one projection unit per wave; under ieee a launch of few tiles is split instead
+    if (2 * a.Ch <= 32 * PW && (X3 || proj_split(a) == 1)) {
       // c_hidden = 128 takes buffer stores over ranges of 32 channel planes (128 N NP bytes)
       if (GNN_PROJX3_FIXED && a.C == 128 && a.Ch == 128 && 128 * a.N * round_up(a.N, 32) < ((int64_t)1 << 31))
-        return launch_proj_x3<128, true>(a, L, st);
-      if (a.C == 128) return launch_proj_x3<128, false>(a, L, st);
-      if (a.C == 64) return launch_proj_x3<64, false>(a, L, st);
+        return launch_proj_f32<128, true, X3>(a, L, st);
+      if (a.C == 128) return launch_proj_f32<128, false, X3>(a, L, st);
+      if (a.C == 64) return launch_proj_f32<64, false, X3>(a, L, st);
     }
   }
   if constexpr (sizeof(T) == 2) {
