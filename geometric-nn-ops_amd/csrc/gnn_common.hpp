@@ -166,6 +166,17 @@ __device__ __forceinline__ void buffer_store(const V& v, __amdgpu_buffer_rsrc_t 
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, off, 0, 0);
 }
 
+// ---- transposed LDS fragment reads beside LDS DMA -----------------------------------------
+// ds_read_b64_tr_b16: each 16-lane group receives a 4 (rows) x 16 (columns) block of 16-bit values
+// transposed, 4 consecutive rows of one column per lane; `base` is the lane's LDS byte address.
+// Written in assembly, with the wait for their data in the same block: in front of the builtin the
+// compiler waits for every global_load_lds in flight (vmcnt(0)), which undoes a pipeline whose
+// later stages are meant to be in flight across the reads (ordinary LDS loads get no such wait).
+// The caller has waited for the DMA of the stage that it reads (vmcnt, then a barrier).
+__device__ __forceinline__ uint32_t lds_addr(const unsigned char* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
+}
+
 // ---- 32x32 tile, one K=16 step ----------------------------------------------------------
 // acc[row, col] += sum_k A[row, k] * B[k, col] over the 16 k of this step, with both
 // operands given as fragments (see the file comment).
