@@ -289,6 +289,58 @@ int gnn_trimul_contract_bwd(const gnn_trimul_contract_bwd_args* args, void* stre
   return hip_status((hipError_t)rc, "trimul_contract_bwd");
 }
 
+static int check_rows_product(const gnn_rows_product_args* args, bool pointers) {
+  if (!args) return set_error(GNN_ERR_ARG, "rows_product: args is NULL");
+  const gnn_rows_product_args& a = *args;
+  if (a.dtype != GNN_BF16 && a.dtype != GNN_F16 && a.dtype != GNN_F32)
+    return set_error(GNN_ERR_ARG, "rows_product: unknown dtype");
+  if (a.count < 1 || a.count > GNN_ROWS_PRODUCT_MAX || a.rows < 1)
+    return set_error(GNN_ERR_ARG, "rows_product: rows must be positive and count in 1 .. GNN_ROWS_PRODUCT_MAX");
+  for (int i = 0; i < a.count; ++i) {
+    const gnn_rows_product_item& p = a.p[i];
+    if (p.O < 8 || p.I < 8 || p.O % 8 || p.I % 8 || p.O > (1 << 20) || p.I > (1 << 20))
+      return set_error(GNN_ERR_ARG, "rows_product: O and I must be multiples of 8, at most 2^20");
+    if (!pointers) continue;
+    if (!p.d || !p.t || !p.partial) return set_error(GNN_ERR_ARG, "rows_product: d, t and partial are required");
+    if (p.d_ld < p.O || p.t_ld < p.I || p.d_ld % 8 || p.t_ld % 8)
+      return set_error(GNN_ERR_ARG, "rows_product: row pitches must cover the rows and be multiples of 8");
+    if (!aligned(p.d, 16) || !aligned(p.t, 16) || !aligned(p.partial, 4))
+      return set_error(GNN_ERR_ARG, "rows_product: d and t must be 16-byte aligned");
+  }
+  return GNN_OK;
+}
+
+int64_t gnn_rows_product_slices(const gnn_rows_product_args* args) {
+  return check_rows_product(args, false) ? 0 : rows_product_slices(*args);
+}
+
+int gnn_rows_product(const gnn_rows_product_args* args, void* stream) {
+  if (int rc = check_rows_product(args, true)) return rc;
+  int rc = rows_product(*args, (hipStream_t)stream);
+  if (rc < 0) return rc;
+  return hip_status((hipError_t)rc, "rows_product");
+}
+
+int gnn_reduce_parts(const gnn_reduce_args* args, void* stream) {
+  if (!args) return set_error(GNN_ERR_ARG, "reduce_parts: args is NULL");
+  const gnn_reduce_args& a = *args;
+  if (a.count < 1 || a.count > GNN_REDUCE_MAX)
+    return set_error(GNN_ERR_ARG, "reduce_parts: count must be in 1 .. GNN_REDUCE_MAX");
+  for (int i = 0; i < a.count; ++i) {
+    const gnn_reduce_segment& s = a.seg[i];
+    if (!s.src || !s.dst || s.parts < 1 || s.n < 1 || (s.parts > 1 && s.stride < s.n))
+      return set_error(GNN_ERR_ARG, "reduce_parts: src, dst, parts, n and a stride of at least n are required");
+    const bool f32 = s.dtype == GNN_F32;
+    if (!f32 && s.dtype != GNN_BF16 && s.dtype != GNN_F16)
+      return set_error(GNN_ERR_ARG, "reduce_parts: unknown dtype");
+    if (!aligned(s.src, 4) || !aligned(s.dst, f32 ? 4 : 2))
+      return set_error(GNN_ERR_ARG, "reduce_parts: src and dst must be aligned to their elements");
+  }
+  int rc = reduce_parts(a, (hipStream_t)stream);
+  if (rc < 0) return rc;
+  return hip_status((hipError_t)rc, "reduce_parts");
+}
+
 int gnn_trimul_relayout(const gnn_trimul_relayout_args* args, void* stream) {
   if (!args) return set_error(GNN_ERR_ARG, "trimul_relayout: args is NULL");
   const gnn_trimul_relayout_args& a = *args;

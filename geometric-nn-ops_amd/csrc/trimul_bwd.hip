@@ -37,6 +37,7 @@ constexpr int LN_ROWS = LN_THREADS / 32;
 constexpr int LN_MAX_K = 512;
 constexpr int LN_UNROLL = 4;                    // rows per half-wave step
 constexpr int LN_MAX_GRID = 4096;               // partial rows of the weight gradients
+constexpr int LN_MIN_GRID = 1024;               // workgroups before each takes several steps
 
 template <typename T>
 __device__ __forceinline__ float ld1(const void* p, int64_t i, float dflt) {
@@ -1000,7 +1001,10 @@ int trimul_out_bwd(const gnn_trimul_out_bwd_args& a, hipStream_t st) {
 int64_t layernorm_partials(int64_t rows, int64_t K) {
   (void)K;
   const int64_t want = (rows + LN_ROWS * LN_UNROLL - 1) / (LN_ROWS * LN_UNROLL);
-  return want < 1 ? 1 : (want > LN_MAX_GRID ? LN_MAX_GRID : want);
+  // past LN_MIN_GRID workgroups (which fill the CUs) each takes up to 8 steps: fewer partial rows
+  // to add up afterwards (147456 rows of 128: 1024 instead of 4096, 27.2 -> 24.1 us)
+  const int64_t most = std::min<int64_t>(LN_MAX_GRID, std::max<int64_t>(LN_MIN_GRID, want / 8));
+  return std::max<int64_t>(1, std::min(want, most));
 }
 
 int layernorm_rows(const gnn_layernorm_args& a, hipStream_t st) {

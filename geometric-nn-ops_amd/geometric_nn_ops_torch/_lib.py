@@ -313,6 +313,57 @@ class TrimulRelayoutArgs(ctypes.Structure):
     ]
 
 
+class RowsProductItem(ctypes.Structure):
+    """Mirror of ``gnn_rows_product_item``."""
+
+    _fields_ = [
+        ("d", ctypes.c_void_p),
+        ("t", ctypes.c_void_p),
+        ("partial", ctypes.c_void_p),
+        ("d_ld", ctypes.c_int64),
+        ("t_ld", ctypes.c_int64),
+        ("O", ctypes.c_int64),
+        ("I", ctypes.c_int64),
+    ]
+
+
+ROWS_PRODUCT_MAX = 4
+
+
+class RowsProductArgs(ctypes.Structure):
+    """Mirror of ``gnn_rows_product_args``."""
+
+    _fields_ = [
+        ("p", RowsProductItem * ROWS_PRODUCT_MAX),
+        ("rows", ctypes.c_int64),
+        ("count", ctypes.c_int32),
+        ("dtype", ctypes.c_int32),
+    ]
+
+
+class ReduceSegment(ctypes.Structure):
+    """Mirror of ``gnn_reduce_segment``."""
+
+    _fields_ = [
+        ("src", ctypes.c_void_p),
+        ("dst", ctypes.c_void_p),
+        ("parts", ctypes.c_int64),
+        ("stride", ctypes.c_int64),
+        ("n", ctypes.c_int64),
+        ("dtype", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+    ]
+
+
+REDUCE_MAX = 16
+
+
+class ReduceArgs(ctypes.Structure):
+    """Mirror of ``gnn_reduce_args``."""
+
+    _fields_ = [("seg", ReduceSegment * REDUCE_MAX), ("count", ctypes.c_int64)]
+
+
 RELAYOUT_PLANES_TO_PIXELS, RELAYOUT_PIXELS_TO_BLOCKED = 0, 1
 
 _SIGNATURES = {
@@ -341,6 +392,9 @@ _SIGNATURES = {
     "gnn_trimul_proj_bwd": (ctypes.c_int, [ctypes.POINTER(TrimulProjBwdArgs), ctypes.c_void_p]),
     "gnn_trimul_contract_bwd": (ctypes.c_int, [ctypes.POINTER(TrimulContractBwdArgs), ctypes.c_void_p]),
     "gnn_trimul_relayout": (ctypes.c_int, [ctypes.POINTER(TrimulRelayoutArgs), ctypes.c_void_p]),
+    "gnn_rows_product_slices": (ctypes.c_int64, [ctypes.POINTER(RowsProductArgs)]),
+    "gnn_rows_product": (ctypes.c_int, [ctypes.POINTER(RowsProductArgs), ctypes.c_void_p]),
+    "gnn_reduce_parts": (ctypes.c_int, [ctypes.POINTER(ReduceArgs), ctypes.c_void_p]),
     "gnn_last_error": (ctypes.c_char_p, []),
     "gnn_version": (ctypes.c_char_p, []),
 }

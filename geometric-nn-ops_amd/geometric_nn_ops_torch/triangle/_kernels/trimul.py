@@ -315,14 +315,15 @@ def trimul_wide_hip(x, direction, mask, eps, weights):
 # gnn_trimul_gate_bwd), and for 16-bit types so do the contraction's two N^3 products per
 # channel (gnn_trimul_contract_bwd, reading a and b in place in the forward's workspace) and
 # the moves between pixel-major tensors and per-channel planes (gnn_trimul_relayout). The
-# other matrix products (the three input projections as one [4 Ch + C, C] linear, p_out, the
-# weight gradients, and fp32's contraction products) go to the vendor GEMM through torch.
+# other matrix products (the three input projections as one [4 Ch + C, C] linear, p_out, and
+# fp32's contraction products) go to the vendor GEMM through torch; the weight gradients run on
+# gnn_rows_product, and gnn_reduce_parts adds every parameter's partial sums in one launch.
 # a, b and o come from the forward's workspace.
 
-def layernorm_rows_hip(x2d, weight=None, bias=None, eps=1e-5, *, dy=None, partials=False):
+def layernorm_rows_hip(x2d, weight=None, bias=None, eps=1e-5, *, dy=None, partials=False, raw=False):
     """Row LayerNorm of ``x2d`` ``[R, K]`` (columns contiguous): ``LN(x)`` when ``dy`` is
     None, else ``dx`` and, with ``partials``, ``(dweight, dbias)`` in fp32 summed over the
-    kernel's per-workgroup partial rows."""
+    kernel's per-workgroup partial rows (``raw``: those rows themselves, ``[parts, 2, K]``)."""
     lib = _lib.load()
     R, K = x2d.shape
     out = torch.empty((R, K), device=x2d.device, dtype=x2d.dtype)
@@ -344,18 +345,20 @@ def layernorm_rows_hip(x2d, weight=None, bias=None, eps=1e-5, *, dy=None, partia
     _lib.call("gnn_layernorm_rows", a, x2d.device)
     if part is None:
         return out
+    if raw:
+        return out, part
     sums = part.sum(0)
     return out, sums[0], sums[1]
 
 
 def gate_bwd_hip(grad, value, gate_pre, mask_rows=None, *, d_value=None, d_gate_pre=None, sums=False,
-                 gate_is_sigmoid=False):
+                 gate_is_sigmoid=False, raw=False):
     """Backward of ``value * sigmoid(gate_pre) * mask_rows[:, None]`` for ``[R, K]`` row
     views (columns contiguous); writes into ``d_value`` / ``d_gate_pre`` (allocated when
     None) and returns them, followed with ``sums`` by their fp32 column sums (the bias
     gradients of the layers behind value and gate_pre), from the kernel's per-workgroup
-    partial rows where K allows it. With ``gate_is_sigmoid`` the third operand is the saved
-    ``sigmoid(gate_pre)`` itself."""
+    partial rows where K allows it (``raw``: followed by the partial rows, ``[parts, 2, K]``). With
+    ``gate_is_sigmoid`` the third operand is the saved ``sigmoid(gate_pre)`` itself."""
     lib = _lib.load()
     R, K = grad.shape
     if d_value is None:
@@ -378,6 +381,10 @@ def gate_bwd_hip(grad, value, gate_pre, mask_rows=None, *, d_value=None, d_gate_
     _lib.call("gnn_trimul_gate_bwd", a, grad.device)
     if not sums:
         return d_value, d_gate_pre
+    if raw:
+        if part is None:
+            part = torch.stack((d_value.sum(0, dtype=torch.float32), d_gate_pre.sum(0, dtype=torch.float32)))[None]
+        return d_value, d_gate_pre, part
     if part is not None:
         colsum = part.sum(0)
         return d_value, d_gate_pre, colsum[0], colsum[1]
@@ -391,8 +398,8 @@ def proj_bwd_supported(dtype, C, Ch):
 
 def proj_bwd_hip(xk, w, mask_rows, dab, d_p, d_g, eps):
     """gnn_trimul_proj_bwd: z = LN_in(x) and the backward of a|b = p * sigmoid(g) * mask
-    with p / g recomputed on the fly; writes ``d_p`` / ``d_g`` (row views) and returns
-    ``(z, p_in bias gradient, g_in bias gradient)``, the latter two fp32."""
+    with p / g recomputed on the fly; writes ``d_p`` / ``d_g`` (row views) and returns ``z`` and the
+    per-workgroup rows ``[parts, 2, 2 Ch]`` (fp32) whose sums are the p_in and g_in bias gradients."""
     lib = _lib.load()
     M, C = xk.shape
     Ch = w["p_in_weight"].shape[0] // 2
@@ -412,8 +419,7 @@ def proj_bwd_hip(xk, w, mask_rows, dab, d_p, d_g, eps):
     a.x_ld, a.dab_ld, a.dl_ld = xk.stride(0), dab.stride(0), d_p.stride(0)
     a.eps, a.dtype = float(eps), _lib.DTYPE_CODE[xk.dtype]
     _lib.call("gnn_trimul_proj_bwd", a, xk.device)
-    sums = part.sum(0)
-    return z, sums[0], sums[1]
+    return z, part
 
 
 def out_bwd_supported(dtype, C, Ch):
@@ -423,10 +429,10 @@ def out_bwd_supported(dtype, C, Ch):
 
 def out_bwd_hip(o_cm, w, gate_pm, dout2, d_go, B, N, eps):
     """gnn_trimul_out_bwd: from the channel-major ``o_cm`` [B, Ch, N, NP], the saved gate and
-    the output gradient (pixel-major rows), ``(on, dy, d_o, sums)`` with on = LN_out(o), dy the
-    gradient of p_out's output, d_o that of o (pixel-major) and ``sums`` [4, 128] fp32 (the
-    p_out / g_out bias and the LN_out weight / bias gradients, each from column 0); d(g_out
-    pre-activation) goes into ``d_go`` (a row view)."""
+    the output gradient (pixel-major rows), ``(on, dy, d_o, part)`` with on = LN_out(o), dy the
+    gradient of p_out's output, d_o that of o (pixel-major) and ``part`` ``[parts, 4, 128]`` fp32 rows
+    whose sums are the p_out / g_out bias and the LN_out weight / bias gradients, each from column
+    0; d(g_out pre-activation) goes into ``d_go`` (a row view)."""
     lib = _lib.load()
     M, C = dout2.shape
     Ch = o_cm.shape[1]
@@ -446,19 +452,38 @@ def out_bwd_hip(o_cm, w, gate_pm, dout2, d_go, B, N, eps):
     a.dgo_ld = d_go.stride(0)
     a.eps, a.dtype = float(eps), _lib.DTYPE_CODE[dt]
     _lib.call("gnn_trimul_out_bwd", a, dev)
-    return on, dy, d_o, part.sum(0)
+    return on, dy, d_o, part
 
 
-def _wgrad(d, t, slices=64):
-    """``d^T t`` for ``[M, O]`` / ``[M, I]`` with M in the hundreds of thousands: the sum
-    over M split into batched slices (one GEMM each, summed in fp32 in slice order), since a
-    single product with an O x I output leaves most of the GPU idle."""
-    M = d.shape[0]
-    while slices > 1 and M % slices:
-        slices //= 2
-    ds = d.reshape(slices, M // slices, d.shape[1])
-    ts = t.reshape(slices, M // slices, t.shape[1])
-    return torch.bmm(ds.transpose(1, 2), ts).sum(0, dtype=torch.float32)  # [O, I], contiguous
+def rows_products_hip(pairs):
+    """Partials of ``d^T t`` for up to ``_lib.ROWS_PRODUCT_MAX`` pairs of ``[M, O]`` / ``[M, I]`` row
+    views over the same M rows (columns contiguous): one fp32 ``[slices, O, I]`` tensor per pair,
+    to be added with ``reduce_parts_hip``."""
+    lib = _lib.load()
+    a = _lib.RowsProductArgs()
+    d0 = pairs[0][0]
+    a.rows, a.count, a.dtype = d0.shape[0], len(pairs), _lib.DTYPE_CODE[d0.dtype]
+    for p, (d, t) in zip(a.p, pairs):
+        p.d, p.t, p.d_ld, p.t_ld, p.O, p.I = (d.data_ptr(), t.data_ptr(), d.stride(0), t.stride(0), d.shape[1],
+                                              t.shape[1])
+    slices = lib.gnn_rows_product_slices(ctypes.byref(a))
+    parts = [torch.empty((slices, d.shape[1], t.shape[1]), device=d0.device, dtype=torch.float32) for d, t in pairs]
+    for p, part in zip(a.p, parts):
+        p.partial = part.data_ptr()
+    _lib.call("gnn_rows_product", a, d0.device)
+    return parts
+
+
+def reduce_parts_hip(segments, device):
+    """Ordered sums of partial results in one launch: ``segments`` are ``(src, offset, n, dst)`` with
+    ``src`` an fp32 ``[parts, ...]`` tensor, the segment being elements ``offset .. offset + n`` of
+    each part, and ``dst`` a contiguous tensor of n elements."""
+    a = _lib.ReduceArgs()
+    a.count = len(segments)
+    for g, (src, offset, n, dst) in zip(a.seg, segments):
+        g.src, g.dst = src.data_ptr() + 4 * offset, dst.data_ptr()
+        g.parts, g.stride, g.n, g.dtype = src.shape[0], src.stride(0), n, _lib.DTYPE_CODE[dst.dtype]
+    _lib.call("gnn_reduce_parts", a, device)
 
 
 def _operand(ws, off, B, Ch, N, NP, dtype):
@@ -551,9 +576,9 @@ def trimul_bwd_hip(x, direction, mask, eps, weights, workspace, offsets, dout, g
     grads = {}
     if use_fused and out_bwd_supported(dt, C, Ch):
         # the output side in one kernel, from the channel-major o and the saved gate
-        on, dy, do_pm, sums = out_bwd_hip(o_cm, w, gate_pm, dout2, dlin[:, 4 * Ch:], B, N, eps)
-        db_pout, db_gout = sums[0, :C], sums[1, :C]
-        grads["norm_out_weight"], grads["norm_out_bias"] = sums[2, :Ch], sums[3, :Ch]
+        on, dy, do_pm, part = out_bwd_hip(o_cm, w, gate_pm, dout2, dlin[:, 4 * Ch:], B, N, eps)
+        for i, key in enumerate(("p_out_bias", "g_out_bias", "norm_out_weight", "norm_out_bias")):
+            grads[key] = part, 128 * i
     else:
         if x.element_size() == 2:
             o_pm = relayout_hip(o_cm, torch.empty((M, Ch), device=dev, dtype=dt), _lib.RELAYOUT_PLANES_TO_PIXELS,
@@ -563,15 +588,14 @@ def trimul_bwd_hip(x, direction, mask, eps, weights, workspace, offsets, dout, g
         on = layernorm_rows_hip(o_pm, w["norm_out_weight"], w["norm_out_bias"], eps)
         y = torch.nn.functional.linear(on, w["p_out_weight"], w["p_out_bias"])
         if use_fused:  # torch's sigmoid backward reads the saved output as well
-            dy, _, db_pout, db_gout = gate_bwd_hip(dout2, y, gate_pm, d_gate_pre=dlin[:, 4 * Ch:], sums=True,
-                                                   gate_is_sigmoid=True)
+            dy, _, part = gate_bwd_hip(dout2, y, gate_pm, d_gate_pre=dlin[:, 4 * Ch:], sums=True,
+                                       gate_is_sigmoid=True, raw=True)
         else:
-            dy, _, db_pout, db_gout = gate_bwd_hip(dout2, y, gopre, d_gate_pre=dlin[:, 4 * Ch:], sums=True)
+            dy, _, part = gate_bwd_hip(dout2, y, gopre, d_gate_pre=dlin[:, 4 * Ch:], sums=True, raw=True)
+        grads["p_out_bias"], grads["g_out_bias"] = (part, 0), (part, C)
         don = dy @ w["p_out_weight"]
-        do_pm, dlnw, dlnb = layernorm_rows_hip(o_pm, w["norm_out_weight"], eps=eps, dy=don, partials=True)
-        grads["norm_out_weight"], grads["norm_out_bias"] = dlnw, dlnb
-    grads["p_out_weight"] = _wgrad(dy, on)
-    grads["p_out_bias"] = db_pout
+        do_pm, part = layernorm_rows_hip(o_pm, w["norm_out_weight"], eps=eps, dy=don, partials=True, raw=True)
+        grads["norm_out_weight"], grads["norm_out_bias"] = (part, 0), (part, Ch)
     # contraction: o_c = A_c B_c^T per (batch, channel) plane; dO_c[i, j] is pixel (i, j).
     # dA / dB planes go back to the pixel layout of a / b (plane [i, k] is pixel (i, k)
     # outgoing, (k, i) incoming), into the two halves of dab.
@@ -595,31 +619,33 @@ def trimul_bwd_hip(x, direction, mask, eps, weights, workspace, offsets, dout, g
     if mask is not None:
         m_rows = mask.to(device=dev, dtype=dt).expand(*x.shape[:-1]).reshape(M).contiguous()
     if use_fused:
-        z, db_pin, db_gin = proj_bwd_hip(xk, w, m_rows, dab, dlin[:, :2 * Ch], dlin[:, 2 * Ch:4 * Ch], eps)
+        z, part = proj_bwd_hip(xk, w, m_rows, dab, dlin[:, :2 * Ch], dlin[:, 2 * Ch:4 * Ch], eps)
     else:
-        _, _, db_pin, db_gin = gate_bwd_hip(dab, p, gpre, m_rows, d_value=dlin[:, :2 * Ch],
-                                            d_gate_pre=dlin[:, 2 * Ch:4 * Ch], sums=True)
-    dwcat = _wgrad(dlin, z)
-    dbcat = torch.cat([db_pin, db_gin, db_gout])
+        _, _, part = gate_bwd_hip(dab, p, gpre, m_rows, d_value=dlin[:, :2 * Ch],
+                                  d_gate_pre=dlin[:, 2 * Ch:4 * Ch], sums=True, raw=True)
+    grads["p_in_bias"], grads["g_in_bias"] = (part, 0), (part, 2 * Ch)
+    dwcat, dwout = rows_products_hip([(dlin, z), (dy, on)])
     grads["p_in_weight"], grads["g_in_weight"], grads["g_out_weight"] = (
-        dwcat[:2 * Ch], dwcat[2 * Ch:4 * Ch], dwcat[4 * Ch:])
-    grads["p_in_bias"], grads["g_in_bias"], grads["g_out_bias"] = (
-        dbcat[:2 * Ch], dbcat[2 * Ch:4 * Ch], dbcat[4 * Ch:])
+        (dwcat, 0), (dwcat, 2 * Ch * C), (dwcat, 4 * Ch * C))
+    grads["p_out_weight"] = dwout, 0
     dz = dlin @ wcat
-    dx, dlnw, dlnb = layernorm_rows_hip(xk, w["norm_in_weight"], eps=eps, dy=dz, partials=True)
-    grads["norm_in_weight"], grads["norm_in_bias"] = dlnw, dlnb
-    # every parameter gradient is fp32 here: one concatenation and one conversion per
-    # parameter dtype instead of a small conversion launch per parameter
+    dx, part = layernorm_rows_hip(xk, w["norm_in_weight"], eps=eps, dy=dz, partials=True, raw=True)
+    grads["norm_in_weight"], grads["norm_in_bias"] = (part, 0), (part, C)
+    # every parameter gradient is a sum of fp32 partials here: one launch adds and converts them
+    # all, into one flat tensor per parameter dtype
+    keys = [k for k in _WEIGHT_KEYS if weights.get(k) is not None]
     out = dict.fromkeys(_WEIGHT_KEYS)
-    by_dtype = {}
-    for key in _WEIGHT_KEYS:
-        if weights.get(key) is not None:
-            by_dtype.setdefault(weights[key].dtype, []).append(key)
-    for pdt, keys in by_dtype.items():
-        flat = torch.cat([grads[k].reshape(-1) for k in keys]).to(pdt)
-        off = 0
-        for k in keys:
-            n = weights[k].numel()
-            out[k] = flat[off:off + n].view(weights[k].shape)
-            off += n
+    segments = []
+    for pdt in {weights[k].dtype for k in keys}:
+        mine = [k for k in keys if weights[k].dtype == pdt]
+        sizes = [weights[k].numel() for k in mine]
+        kdt = pdt if pdt in _lib.DTYPE_CODE else torch.float32
+        views = torch.empty(sum(sizes), device=dev, dtype=kdt).split(sizes)
+        segments += [(*grads[k], n, v) for k, n, v in zip(mine, sizes, views)]
+        for k, v in zip(mine, views):
+            out[k] = v.view(weights[k].shape)
+    reduce_parts_hip(segments, dev)
+    for k in keys:
+        if out[k].dtype != weights[k].dtype:
+            out[k] = out[k].to(weights[k].dtype)
     return dx.reshape(x.shape), out

@@ -511,6 +511,51 @@ typedef struct gnn_trimul_relayout_args {
  * autograd through trimul_torch (triangle/_reference/trimul.py:57-97). */
 int gnn_trimul_relayout(const gnn_trimul_relayout_args* args, void* stream);
 
+/* C[o][i] = sum over the rows m of d[m][o] * t[m][i]: the weight gradient of a linear layer whose
+ * output gradient is d [rows, O] and whose input is t [rows, I]. Up to GNN_ROWS_PRODUCT_MAX products
+ * over the same number of rows run in one launch. Each leaves fp32 partials [slices][O][I] in
+ * `partial` (slices = gnn_rows_product_slices of the same arguments; the pointers need not be set
+ * for that call), to be added with gnn_reduce_parts. O and I are multiples of 8, the pitches
+ * multiples of 8 elements and at least O / I, and d and t 16-byte aligned. fp32 products are full
+ * precision. */
+#define GNN_ROWS_PRODUCT_MAX 4
+typedef struct gnn_rows_product_item {
+  const void* d;
+  const void* t;
+  float* partial;
+  int64_t d_ld, t_ld;
+  int64_t O, I;
+} gnn_rows_product_item;
+typedef struct gnn_rows_product_args {
+  gnn_rows_product_item p[GNN_ROWS_PRODUCT_MAX];
+  int64_t rows;
+  int32_t count;
+  int32_t dtype; /* enum gnn_dtype of d and t */
+} gnn_rows_product_args;
+
+/* Replaces the weight gradients of autograd through F.linear (geometric_nn_ops_torch/triangle/
+ * _reference/trimul.py:86-97); the reference has no kernel for them. */
+int64_t gnn_rows_product_slices(const gnn_rows_product_args* args);
+int gnn_rows_product(const gnn_rows_product_args* args, void* stream);
+
+/* dst[e] = sum over p < parts of src[p * stride + e] (e < n), in a fixed order, for up to
+ * GNN_REDUCE_MAX segments in one launch; dst is in the segment's dtype. Adds the partials that
+ * gnn_rows_product, gnn_layernorm_rows, gnn_trimul_gate_bwd, gnn_trimul_proj_bwd and
+ * gnn_trimul_out_bwd leave. No counterpart in the reference (autograd's own sums). */
+#define GNN_REDUCE_MAX 16
+typedef struct gnn_reduce_segment {
+  const float* src;
+  void* dst;
+  int64_t parts, stride, n;
+  int32_t dtype; /* enum gnn_dtype of dst */
+  int32_t reserved;
+} gnn_reduce_segment;
+typedef struct gnn_reduce_args {
+  gnn_reduce_segment seg[GNN_REDUCE_MAX];
+  int64_t count;
+} gnn_reduce_args;
+int gnn_reduce_parts(const gnn_reduce_args* args, void* stream);
+
 /* Message for the last failing call on this thread ("" if none). */
 const char* gnn_last_error(void);
 

@@ -11,6 +11,7 @@ from oracle import triangle_oracle as O
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
+DEV_T = torch.device(DEV)
 DTYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
 TOL = {torch.bfloat16: 1e-2, torch.float16: 2e-3, torch.float32: 1e-5}
 
@@ -101,3 +102,56 @@ def test_fp32_contraction_tiles(N, direction):
     (torch.float32, 135, 64, 128, 1)])
 def test_projection_dispatch(dtype, N, C, Ch, B, direction):
     assert _trimul_forward_error(N, C, Ch, dtype, direction, B) <= TOL[dtype]
+
+
+# ------------------------------------------------------- products over rows, ordered sums
+@DTYPES
+@pytest.mark.parametrize(("M", "shapes"), [
+    (1, [(8, 8)]), (15, [(32, 24), (8, 136)]), (33, [(128, 128)]), (255, [(640, 128), (128, 128)]),
+    (1000, [(136, 72), (64, 256), (8, 8), (192, 64)]), (40401, [(192, 64), (64, 32)])])
+def test_rows_product(M, shapes, dtype):
+    """Rows short of a stage and of a slice, output blocks part empty, one to four products a launch,
+    operands inside wider rows. The products are exact in fp32, so the sum of M of them errs by at
+    most M 2^-24 of the sum of magnitudes, far below the bound for these sizes (random signs)."""
+    from geometric_nn_ops_torch.triangle._kernels.trimul import reduce_parts_hip, rows_products_hip
+
+    g = torch.Generator(device=DEV).manual_seed(M)
+    pairs = []
+    for O_, I_ in shapes:
+        d = torch.randn(M, O_ + 16, generator=g, device=DEV).to(dtype)
+        t = torch.randn(M, I_ + 8, generator=g, device=DEV).to(dtype)
+        pairs.append((d[:, 16:], t[:, :I_]) if dtype != torch.float32 else (d[:, 8:O_ + 8], t[:, 8:]))
+    parts = rows_products_hip(pairs)
+    sums = [torch.empty(d.shape[1] * t.shape[1], device=DEV) for d, t in pairs]
+    reduce_parts_hip([(p, 0, s.numel(), s) for p, s in zip(parts, sums)], DEV_T)
+    for (d, t), s in zip(pairs, sums):
+        want = d.double().t().contiguous() @ t.double()
+        assert (s.view_as(want).double() - want).norm() <= 2e-6 * want.norm()
+
+
+def test_rows_product_ignores_what_lies_past_the_rows():
+    """The rows behind the last one (of a larger tensor) hold NaN; the result does not."""
+    from geometric_nn_ops_torch.triangle._kernels.trimul import rows_products_hip
+
+    for dtype in TOL:
+        d, t = (torch.randn(64, 128, device=DEV).to(dtype) for _ in range(2))
+        d[37:], t[37:] = float("nan"), float("nan")
+        (part,) = rows_products_hip([(d[:37], t[:37])])
+        want = d[:37].double().t().contiguous() @ t[:37].double()
+        assert (part.sum(0).double() - want).norm() <= 2e-6 * want.norm()
+
+
+@DTYPES
+@pytest.mark.parametrize(("parts", "n"), [(1, 1), (7, 300), (128, 257), (129, 9), (1024, 31)])
+def test_reduce_parts(parts, n, dtype):
+    """Both ways of adding (up to 128 parts a thread adds an element alone), element counts that leave a
+    block part empty, a segment inside wider parts, results in each dtype, the same bits twice."""
+    from geometric_nn_ops_torch.triangle._kernels.trimul import reduce_parts_hip
+
+    src = torch.randn(parts, n + 5, device=DEV)
+    out = [torch.empty(n, device=DEV, dtype=dtype) for _ in range(2)]
+    for o in out:
+        reduce_parts_hip([(src, 3, n, o)], DEV_T)
+    want = src[:, 3:3 + n].double().sum(0)
+    assert torch.equal(out[0], out[1])
+    assert (out[0].double() - want).norm() <= TOL[dtype] * want.norm()
