@@ -289,13 +289,37 @@ int gnn_trimul_contract_bwd(const gnn_trimul_contract_bwd_args* args, void* stre
   return hip_status((hipError_t)rc, "trimul_contract_bwd");
 }
 
+int gnn_relayout_f32(const gnn_trimul_relayout_args* args, void* stream) {
+  if (!args) return set_error(GNN_ERR_ARG, "relayout_f32: args is NULL");
+  const gnn_trimul_relayout_args& a = *args;
+  if (!a.src || !a.dst) return set_error(GNN_ERR_ARG, "relayout_f32: src and dst are required");
+  if (a.dtype != GNN_F32) return set_error(GNN_ERR_UNSUPPORTED, "relayout_f32: fp32 only");
+  const bool to_pixels = a.mode == GNN_RELAYOUT_PLANES_TO_PIXELS;
+  if (!to_pixels && a.mode != GNN_RELAYOUT_PIXELS_TO_PLANES)
+    return set_error(GNN_ERR_ARG, "relayout_f32: unknown mode");
+  if (a.B < 1 || a.N < 1 || a.Ch < 1) return set_error(GNN_ERR_ARG, "relayout_f32: B, N and Ch must be positive");
+  if (a.Ch % 4 || a.src_ld % 4 || a.dst_ld % 4 || a.src_c0 % 4 || a.dst_c0 % 4 || a.src_c0 < 0 || a.dst_c0 < 0)
+    return set_error(GNN_ERR_ARG, "relayout_f32: Ch, row pitches and channel offsets must be multiples of 4");
+  if (!aligned(a.src, 16) || !aligned(a.dst, 16))
+    return set_error(GNN_ERR_ARG, "relayout_f32: src and dst must be 16-byte aligned");
+  if (a.plane_rows != 0 && a.plane_rows < a.N)
+    return set_error(GNN_ERR_ARG, "relayout_f32: plane_rows must be 0 or at least N");
+  const int64_t N4 = (a.N + 3) / 4 * 4;
+  if (to_pixels ? (a.src_ld < N4 || a.dst_c0 + a.Ch > a.dst_ld) : (a.dst_ld < N4 || a.src_c0 + a.Ch > a.src_ld))
+    return set_error(GNN_ERR_ARG, "relayout_f32: a row pitch is too small for its rows");
+  int rc = relayout_f32(a, (hipStream_t)stream);
+  if (rc < 0) return rc;
+  return hip_status((hipError_t)rc, "relayout_f32");
+}
+
 static int check_rows_product(const gnn_rows_product_args* args, bool pointers) {
   if (!args) return set_error(GNN_ERR_ARG, "rows_product: args is NULL");
   const gnn_rows_product_args& a = *args;
   if (a.dtype != GNN_BF16 && a.dtype != GNN_F16 && a.dtype != GNN_F32)
     return set_error(GNN_ERR_ARG, "rows_product: unknown dtype");
-  if (a.count < 1 || a.count > GNN_ROWS_PRODUCT_MAX || a.rows < 1)
-    return set_error(GNN_ERR_ARG, "rows_product: rows must be positive and count in 1 .. GNN_ROWS_PRODUCT_MAX");
+  if (a.count < 1 || a.count > GNN_ROWS_PRODUCT_MAX || a.rows < 1 || a.slice_rows < 0)
+    return set_error(GNN_ERR_ARG, "rows_product: rows must be positive, slice_rows not negative and count in 1 .. "
+                                  "GNN_ROWS_PRODUCT_MAX");
   for (int i = 0; i < a.count; ++i) {
     const gnn_rows_product_item& p = a.p[i];
     if (p.O < 8 || p.I < 8 || p.O % 8 || p.I % 8 || p.O > (1 << 20) || p.I > (1 << 20))

@@ -59,6 +59,7 @@ int trimul_out_bwd(const gnn_trimul_out_bwd_args& a, hipStream_t stream);
 int trimul_proj_bwd(const gnn_trimul_proj_bwd_args& a, hipStream_t stream);
 int trimul_contract_bwd(const gnn_trimul_contract_bwd_args& a, hipStream_t stream);
 int trimul_relayout(const gnn_trimul_relayout_args& a, hipStream_t stream);
+int relayout_f32(const gnn_trimul_relayout_args& a, hipStream_t stream);
 int64_t rows_product_slices(const gnn_rows_product_args& a);
 int rows_product(const gnn_rows_product_args& a, hipStream_t stream);
 int reduce_parts(const gnn_reduce_args& a, hipStream_t stream);

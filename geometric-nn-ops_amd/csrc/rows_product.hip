@@ -93,7 +93,7 @@ __device__ __forceinline__ void read_stage16(const uint32_t (&ax)[2], const uint
 struct RowsProductGrid {
   int nb[GNN_ROWS_PRODUCT_MAX];  // output blocks of each product
   int total;                     // of all
-  int64_t rps;                   // rows per slice, a multiple of 32
+  int64_t rps;                   // rows per slice
 };
 
 template <typename T>
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(RP_NT, RP_WGS) void rows_product_kernel(const gnn_r
     asm volatile("s_barrier" ::: "memory");
     unsigned char* sx = smem + (kt % Cfg::STAGES) * Cfg::STAGE_BYTES;
     const int valid = (int)min<int64_t>(Cfg::RS, m1 - m0 - (int64_t)kt * Cfg::RS);
-    if (valid < Cfg::RS) {  // uniform; the last stage of the last slice: rows past the end are zeros
+    if (valid < Cfg::RS) {  // uniform; the last stage of a slice: rows past its end are zeros
       typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
       for (int b = valid * Cfg::ROWB + 16 * tid; b < Cfg::OP_BYTES; b += 16 * RP_NT) {
         *reinterpret_cast<u32x4_t*>(sx + b) = u32x4_t{0u, 0u, 0u, 0u};
@@ -234,6 +234,10 @@ RowsProductGrid rows_product_grid(const gnn_rows_product_args& a) {
   for (int i = 0; i < a.count; ++i) {
     G.nb[i] = (int)(((a.p[i].O + RP_BLK - 1) / RP_BLK) * ((a.p[i].I + RP_BLK - 1) / RP_BLK));
     G.total += G.nb[i];
+  }
+  if (a.slice_rows > 0) {
+    G.rps = a.slice_rows;
+    return G;
   }
   const int64_t want = std::max<int64_t>(1, (int64_t)RP_WGS * compute_units() / G.total);
   const int64_t rows =

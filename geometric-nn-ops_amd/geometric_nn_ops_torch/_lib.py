@@ -309,7 +309,7 @@ class TrimulRelayoutArgs(ctypes.Structure):
         ("mode", ctypes.c_int32),
         ("transposed", ctypes.c_int32),
         ("dtype", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("plane_rows", ctypes.c_int32),
     ]
 
 
@@ -336,6 +336,7 @@ class RowsProductArgs(ctypes.Structure):
     _fields_ = [
         ("p", RowsProductItem * ROWS_PRODUCT_MAX),
         ("rows", ctypes.c_int64),
+        ("slice_rows", ctypes.c_int64),
         ("count", ctypes.c_int32),
         ("dtype", ctypes.c_int32),
     ]
@@ -364,7 +365,7 @@ class ReduceArgs(ctypes.Structure):
     _fields_ = [("seg", ReduceSegment * REDUCE_MAX), ("count", ctypes.c_int64)]
 
 
-RELAYOUT_PLANES_TO_PIXELS, RELAYOUT_PIXELS_TO_BLOCKED = 0, 1
+RELAYOUT_PLANES_TO_PIXELS, RELAYOUT_PIXELS_TO_BLOCKED, RELAYOUT_PIXELS_TO_PLANES = 0, 1, 2
 
 _SIGNATURES = {
     "gnn_triattn_fwd": (ctypes.c_int, [ctypes.POINTER(TriAttnArgs), ctypes.c_void_p]),
@@ -392,6 +393,7 @@ _SIGNATURES = {
     "gnn_trimul_proj_bwd": (ctypes.c_int, [ctypes.POINTER(TrimulProjBwdArgs), ctypes.c_void_p]),
     "gnn_trimul_contract_bwd": (ctypes.c_int, [ctypes.POINTER(TrimulContractBwdArgs), ctypes.c_void_p]),
     "gnn_trimul_relayout": (ctypes.c_int, [ctypes.POINTER(TrimulRelayoutArgs), ctypes.c_void_p]),
+    "gnn_relayout_f32": (ctypes.c_int, [ctypes.POINTER(TrimulRelayoutArgs), ctypes.c_void_p]),
     "gnn_rows_product_slices": (ctypes.c_int64, [ctypes.POINTER(RowsProductArgs)]),
     "gnn_rows_product": (ctypes.c_int, [ctypes.POINTER(RowsProductArgs), ctypes.c_void_p]),
     "gnn_reduce_parts": (ctypes.c_int, [ctypes.POINTER(ReduceArgs), ctypes.c_void_p]),

@@ -455,14 +455,15 @@ def out_bwd_hip(o_cm, w, gate_pm, dout2, d_go, B, N, eps):
     return on, dy, d_o, part
 
 
-def rows_products_hip(pairs):
+def rows_products_hip(pairs, slice_rows=0):
     """Partials of ``d^T t`` for up to ``_lib.ROWS_PRODUCT_MAX`` pairs of ``[M, O]`` / ``[M, I]`` row
     views over the same M rows (columns contiguous): one fp32 ``[slices, O, I]`` tensor per pair,
-    to be added with ``reduce_parts_hip``."""
+    to be added with ``reduce_parts_hip``; with ``slice_rows``, slice s is the product over rows
+    ``s slice_rows .. (s + 1) slice_rows``."""
     lib = _lib.load()
     a = _lib.RowsProductArgs()
     d0 = pairs[0][0]
-    a.rows, a.count, a.dtype = d0.shape[0], len(pairs), _lib.DTYPE_CODE[d0.dtype]
+    a.rows, a.slice_rows, a.count, a.dtype = d0.shape[0], slice_rows, len(pairs), _lib.DTYPE_CODE[d0.dtype]
     for p, (d, t) in zip(a.p, pairs):
         p.d, p.t, p.d_ld, p.t_ld, p.O, p.I = (d.data_ptr(), t.data_ptr(), d.stride(0), t.stride(0), d.shape[1],
                                               t.shape[1])
@@ -486,27 +487,15 @@ def reduce_parts_hip(segments, device):
     _lib.call("gnn_reduce_parts", a, device)
 
 
-def _operand(ws, off, B, Ch, N, NP, dtype):
-    """The contraction operand of the workspace as ``[B * Ch, N, N]`` (row = output index,
-    column = contraction index), contiguous."""
-    el = torch.empty((), dtype=dtype).element_size()
-    n = B * Ch * N * NP
-    flat = ws[off:off + n * el].view(dtype)
-    if el == 2:  # k-blocked [B, Ch, NP / 32, N, 32]
-        t = flat.view(B * Ch, NP // 32, N, 32).permute(0, 2, 1, 3).reshape(B * Ch, N, NP)
-    else:  # row-major [B, Ch, N, NP]
-        t = flat.view(B * Ch, N, NP)
-    return t[..., :N].contiguous()
-
-
-def relayout_hip(src, dst, mode, B, N, Ch, *, src_ld, dst_ld, src_c0=0, dst_c0=0, transposed=False):
-    """gnn_trimul_relayout (16-bit) between pixel-major rows and per-channel planes."""
+def relayout_hip(src, dst, mode, B, N, Ch, *, src_ld, dst_ld, src_c0=0, dst_c0=0, transposed=False, plane_rows=0):
+    """gnn_trimul_relayout (16-bit) or gnn_relayout_f32 between pixel-major rows and per-channel
+    planes."""
     a = _lib.TrimulRelayoutArgs()
     a.src, a.dst = src.data_ptr(), dst.data_ptr()
     a.B, a.N, a.Ch = B, N, Ch
     a.src_ld, a.dst_ld, a.src_c0, a.dst_c0 = src_ld, dst_ld, src_c0, dst_c0
-    a.mode, a.transposed, a.dtype = mode, int(transposed), _lib.DTYPE_CODE[src.dtype]
-    _lib.call("gnn_trimul_relayout", a, src.device)
+    a.mode, a.transposed, a.dtype, a.plane_rows = mode, int(transposed), _lib.DTYPE_CODE[src.dtype], plane_rows
+    _lib.call("gnn_relayout_f32" if src.dtype == torch.float32 else "gnn_trimul_relayout", a, src.device)
     return dst
 
 
@@ -531,6 +520,20 @@ def contract_bwd_hip(workspace, offsets, do_pm, B, Ch, N):
     a.planes, a.N, a.dtype = B * Ch, N, _lib.DTYPE_CODE[dt]
     _lib.call("gnn_trimul_contract_bwd", a, dev)
     return da, db
+
+
+def contract_bwd_f32_hip(workspace, offsets, do_pm, B, Ch, N):
+    """``contract_bwd_hip`` for fp32: ``(dA, dB)`` ``[B, Ch, N8, N8]`` (N8 = round_up(N, 8); rows and
+    columns past N hold nothing), as batches of products over the rows of the planes, with A and B
+    ``[N, NP]`` read in place and dO brought into planes in both orientations:
+    ``dA[i][k] = sum_j dO[i][j] B[j][k]``, ``dB[j][k] = sum_i dO[i][j] A[i][k]``."""
+    dev, planes, NP, N8 = do_pm.device, B * Ch, _pad32(N), (N + 7) // 8 * 8
+    d = torch.empty((2, planes * N, N8), device=dev, dtype=torch.float32)
+    for t, transposed in ((d[0], False), (d[1], True)):
+        relayout_hip(do_pm, t, _lib.RELAYOUT_PIXELS_TO_PLANES, B, N, Ch, src_ld=do_pm.stride(0), dst_ld=N8,
+                     transposed=transposed)
+    ab = [workspace[o:o + planes * N * NP * 4].view(torch.float32).view(planes * N, NP)[:, :N8] for o in offsets[:2]]
+    return rows_products_hip([(d[1], ab[1]), (d[0], ab[0])], slice_rows=N)
 
 
 def trimul_bwd_hip(x, direction, mask, eps, weights, workspace, offsets, dout, gate=None, fused=None):
@@ -580,11 +583,8 @@ def trimul_bwd_hip(x, direction, mask, eps, weights, workspace, offsets, dout, g
         for i, key in enumerate(("p_out_bias", "g_out_bias", "norm_out_weight", "norm_out_bias")):
             grads[key] = part, 128 * i
     else:
-        if x.element_size() == 2:
-            o_pm = relayout_hip(o_cm, torch.empty((M, Ch), device=dev, dtype=dt), _lib.RELAYOUT_PLANES_TO_PIXELS,
-                                B, N, Ch, src_ld=NP, dst_ld=Ch)
-        else:
-            o_pm = o_cm[..., :N].permute(0, 2, 3, 1).reshape(M, Ch).contiguous()
+        o_pm = relayout_hip(o_cm, torch.empty((M, Ch), device=dev, dtype=dt), _lib.RELAYOUT_PLANES_TO_PIXELS,
+                            B, N, Ch, src_ld=NP, dst_ld=Ch)
         on = layernorm_rows_hip(o_pm, w["norm_out_weight"], w["norm_out_bias"], eps)
         y = torch.nn.functional.linear(on, w["p_out_weight"], w["p_out_bias"])
         if use_fused:  # torch's sigmoid backward reads the saved output as well
@@ -600,21 +600,11 @@ def trimul_bwd_hip(x, direction, mask, eps, weights, workspace, offsets, dout, g
     # dA / dB planes go back to the pixel layout of a / b (plane [i, k] is pixel (i, k)
     # outgoing, (k, i) incoming), into the two halves of dab.
     dab = torch.empty((M, 2 * Ch), device=dev, dtype=dt)
-    if x.element_size() == 2:  # this library's kernels, reading A and B in the workspace
-        dA, dB = contract_bwd_hip(workspace, offsets, do_pm, B, Ch, N)
-        for t, c0 in ((dA, 0), (dB, Ch)):
-            relayout_hip(t, dab, _lib.RELAYOUT_PLANES_TO_PIXELS, B, N, Ch, src_ld=NP, dst_ld=2 * Ch, dst_c0=c0,
-                         transposed=not outgoing)
-    else:  # fp32: the vendor GEMM
-        A = _operand(workspace, offsets[0], B, Ch, N, NP, dt)
-        Bm = _operand(workspace, offsets[1], B, Ch, N, NP, dt)
-        do_cm = do_pm.view(B, N, N, Ch).permute(0, 3, 1, 2).reshape(B * Ch, N, N).contiguous()
-        dA4 = torch.bmm(do_cm, Bm).view(B, Ch, N, N)                                   # dO B
-        dB4 = torch.bmm(A.transpose(1, 2), do_cm).view(B, Ch, N, N).transpose(-1, -2)  # dO^T A
-        perm = (0, 2, 3, 1) if outgoing else (0, 3, 2, 1)
-        dab4 = dab.view(B, N, N, 2 * Ch)
-        dab4[..., :Ch] = dA4.permute(*perm)
-        dab4[..., Ch:] = dB4.permute(*perm)
+    contract = contract_bwd_f32_hip if dt == torch.float32 else contract_bwd_hip
+    dA, dB = contract(workspace, offsets, do_pm, B, Ch, N)
+    for t, c0 in ((dA, 0), (dB, Ch)):
+        relayout_hip(t, dab, _lib.RELAYOUT_PLANES_TO_PIXELS, B, N, Ch, src_ld=t.shape[-1], dst_ld=2 * Ch, dst_c0=c0,
+                     transposed=not outgoing, plane_rows=t.shape[-2])
     m_rows = None
     if mask is not None:
         m_rows = mask.to(device=dev, dtype=dt).expand(*x.shape[:-1]).reshape(M).contiguous()

@@ -491,8 +491,17 @@ int gnn_trimul_contract_bwd(const gnn_trimul_contract_bwd_args* args, void* stre
  *       ((i / 32) NP + j) 32 + i % 32, or at ((j / 32) NP + i) 32 + j % 32 when `transposed`;
  *       every element with i >= N or j >= N is written as zero (the dO operands of
  *       gnn_trimul_contract_bwd: do_i untransposed, do_j transposed).
- * Ch, the row pitches and channel offsets multiples of 8; pointers 16-byte aligned. */
-enum gnn_relayout_mode { GNN_RELAYOUT_PLANES_TO_PIXELS = 0, GNN_RELAYOUT_PIXELS_TO_BLOCKED = 1 };
+ * Ch, the row pitches and channel offsets multiples of 8; pointers 16-byte aligned.
+ * fp32 has an entry of its own (gnn_relayout_f32, multiples of 4) with
+ *   GNN_RELAYOUT_PLANES_TO_PIXELS, src_ld >= round_up(N, 4), and
+ *   GNN_RELAYOUT_PIXELS_TO_PLANES:  src[pixel (i, j)][src_c0 + c] -> dst = planes
+ *       [B * Ch][N][dst_ld], row i and column j, or row j and column i when `transposed`; columns
+ *       N .. round_up(N, 4) - 1 are written as zeros. dst_ld >= round_up(N, 4). */
+enum gnn_relayout_mode {
+  GNN_RELAYOUT_PLANES_TO_PIXELS = 0,
+  GNN_RELAYOUT_PIXELS_TO_BLOCKED = 1,
+  GNN_RELAYOUT_PIXELS_TO_PLANES = 2
+};
 
 typedef struct gnn_trimul_relayout_args {
   const void* src;
@@ -502,14 +511,15 @@ typedef struct gnn_trimul_relayout_args {
   int64_t src_c0, dst_c0;
   int32_t mode;       /* enum gnn_relayout_mode */
   int32_t transposed;
-  int32_t dtype;      /* GNN_BF16 or GNN_F16 */
-  int32_t reserved;
+  int32_t dtype;      /* GNN_BF16 or GNN_F16 (GNN_F32 for gnn_relayout_f32) */
+  int32_t plane_rows; /* gnn_relayout_f32: rows that a plane holds, 0 = N */
 } gnn_trimul_relayout_args;
 
 /* Replaces the strided copies (permute / contiguous) between the trimul backward's pixel-major
  * tensors and the contraction's planes; no counterpart in the reference, whose backward is
  * autograd through trimul_torch (triangle/_reference/trimul.py:57-97). */
 int gnn_trimul_relayout(const gnn_trimul_relayout_args* args, void* stream);
+int gnn_relayout_f32(const gnn_trimul_relayout_args* args, void* stream);
 
 /* C[o][i] = sum over the rows m of d[m][o] * t[m][i]: the weight gradient of a linear layer whose
  * output gradient is d [rows, O] and whose input is t [rows, I]. Up to GNN_ROWS_PRODUCT_MAX products
@@ -517,7 +527,8 @@ int gnn_trimul_relayout(const gnn_trimul_relayout_args* args, void* stream);
  * `partial` (slices = gnn_rows_product_slices of the same arguments; the pointers need not be set
  * for that call), to be added with gnn_reduce_parts. O and I are multiples of 8, the pitches
  * multiples of 8 elements and at least O / I, and d and t 16-byte aligned. fp32 products are full
- * precision. */
+ * precision. With slice_rows set, slice s is the product over rows [s slice_rows, (s + 1) slice_rows):
+ * a batch of products over consecutive planes of slice_rows rows. */
 #define GNN_ROWS_PRODUCT_MAX 4
 typedef struct gnn_rows_product_item {
   const void* d;
@@ -529,6 +540,7 @@ typedef struct gnn_rows_product_item {
 typedef struct gnn_rows_product_args {
   gnn_rows_product_item p[GNN_ROWS_PRODUCT_MAX];
   int64_t rows;
+  int64_t slice_rows; /* rows per slice; 0: chosen by the library */
   int32_t count;
   int32_t dtype; /* enum gnn_dtype of d and t */
 } gnn_rows_product_args;

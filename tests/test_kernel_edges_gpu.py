@@ -155,3 +155,25 @@ def test_reduce_parts(parts, n, dtype):
     want = src[:, 3:3 + n].double().sum(0)
     assert torch.equal(out[0], out[1])
     assert (out[0].double() - want).norm() <= TOL[dtype] * want.norm()
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+@pytest.mark.parametrize(("N", "C", "Ch", "B"), [(1, 32, 32, 1), (5, 64, 32, 2), (33, 32, 96, 1), (130, 64, 64, 1)])
+def test_fp32_backward_planes(N, C, Ch, B, direction):
+    """Full-precision backward: plane rows short of and past a vector, a stage and an output block,
+    every gradient against the fp64 oracle."""
+    from geometric_nn_ops_torch.triangle import triangle_multiplicative_update
+
+    w = trimul_weights(C, Ch, torch.float32, seed=N, biases=True, ln_random=True)
+    x, mask = pair_input(B, N, C, torch.float32, seed=N + 1)
+    dout = torch.randn(x.shape, generator=gen(N + 2))
+    xg = x.to(DEV).requires_grad_()
+    wg = {k: v.to(DEV).requires_grad_() for k, v in w.items()}
+    out = triangle_multiplicative_update(xg, direction, mask.to(DEV), **wg)
+    got = torch.autograd.grad(out, [xg, *wg.values()], dout.to(DEV))
+    want = O.trimul_grad(to_np(x), direction, to_np(mask), to_np(dout), **np_weights(w))
+    # a LayerNorm divides by the spread of its row, at least sqrt(eps) = 3e-3: 2^-24 / 3e-3 = 2e-5
+    scale = max(float(abs(want[k]).max()) for k in wg)
+    assert O.rel_fro(to_np(got[0]), want["x"]) <= 1e-4
+    for k, g in zip(wg, got[1:]):
+        assert abs(to_np(g) - want[k]).max() <= 1e-4 * max(float(abs(want[k]).max()), 1e-2 * scale), k
