@@ -20,6 +20,7 @@
 //   bwd_dkdv_row  Q' = bf16(q * scale) (through registers: the product is rounded) and dO
 //                 (global_load_lds) of the row, with its lse and Delta; the waves take
 //                 32-key blocks round robin and sweep every query tile.
+// These two serve N_res above BWD_FUSED_MAX_N; below it bwd_fused_row does the work of both.
 // The pair-bias fragments of the next step are requested from global memory (L2: a bias
 // plane is shared by every N_seq row) while the current one is computed. The reference's
 // correction for rows whose keys are all masked (P of a masked key divided by N_res, which
@@ -452,8 +453,362 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dkdv_row_kernel(const gnn_triattn_
   }
 }
 
+// ------------------------------------------------------------------- dQ, dK and dV together
+// Up to BWD_FUSED_MAX_N one workgroup takes a (b, s, h) row whole, so the logits and their exponents
+// are formed once instead of once for dq and once for dk / dv: 10 products and 1 exponential per
+// element pair of 32-blocks instead of 14 and 2 (QK^T, dO V^T and the bias count once).
+//
+// Q' = bf16(q * scale) and dO of the row sit in LDS (with -lse log2(e) and -Delta, which is formed
+// here while o and dO pass through the staging registers), dQ accumulates in LDS in fp32, in the
+// MFMA accumulator's own layout (16-byte reads and writes, the read being the product's initial
+// accumulator). A wave owns KB blocks of 32 keys: K and V as B operands, K once more read transposed
+// (the B operand of dQ += dS K), and the dK / dV accumulators, all in registers. Step t of wave w
+// takes the queries of block (KB w + t) mod nb: the waves of a step update different dQ blocks, a
+// barrier (which leaves the bias loads in flight) separates the steps, and so every sum has one fixed
+// order. dS has its keys on the lanes, as dK's A operand needs it; dQ's A operand needs the queries
+// there, so each 32 x 32 tile passes through a wave-private LDS tile and is read back transposed.
+//
+// KB = 2 (8 waves at N = 512, two workgroups of 4 at 256: two waves per SIMD, 256 registers) reads each
+// Q' / dO fragment and updates dQ once for 64 keys; 256 < N <= 384, one workgroup per CU, takes KB = 1,
+// whose 9 to 12 waves fill the SIMDs better than 5 or 6 (bf16, bias, H = 4, the call without the bias
+// gradient: N = 320 121 against 142 us, 384 185 against 206; N = 128 41 against 33, 256 83 against 69).
+// LDS bounds N: 264 bytes per query and 2 KB per wave.
+// The same call on the two kernels: N = 256 104 -> 74 us, 384 247 -> 185, 512 537 -> 372. At N = 512 the
+// vector ALU is busy 39% of the cycles (exponentials, conversions), the matrix unit 25% and LDS 35%; the
+// rest is the chain of a tile (fragments, products, exponentials, the tile's way through LDS, dQ), which
+// two waves per SIMD do not hide. Interleaved with the tile's C++ accesses (ordered by the compiler) and
+// with the mask's branches inside the loop it took 453 us.
+constexpr int BWD_FUSED_MAX_N = 512;
+
+__host__ __device__ inline int fused_kb(int N) { return N > 256 && N <= 384 ? 1 : 2; }
+__host__ __device__ inline int fused_waves(int N) {
+  const int nb = (N + 31) / 32, kb = fused_kb(N);
+  return (nb + kb - 1) / kb;
+}
+// LDS of a 32-query block: Q' and dO images, dQ in accumulator layout ([4][64 lanes] f32x4), then
+// -lse log2(e) (lse itself in a row whose keys are all masked; queries past N: p = 0) and -Delta
+struct FusedBlock {
+  unsigned char q[32 * RROW];
+  unsigned char d[32 * RROW];
+  f32x4 dq[4 * 64];
+  float nl[32];
+  float ndelta[32];
+};
+inline size_t fused_lds(int N) { return (size_t)((N + 31) / 32) * sizeof(FusedBlock) + fused_waves(N) * 2048; }
+
+// A 32 x 32 16-bit tile through LDS: write4 stores a lane's 16 values (row = lane % 32, columns
+// 8 rg + 4 g .. + 3 in words 2 rg, 2 rg + 1) and read_tr reads both k-steps' transposed fragments,
+// waiting for the data. In assembly, so that the compiler does not order its other LDS accesses
+// (none of which touches the tile) around them; assembly blocks keep their order among themselves
+// and a wave's LDS operations execute in order.
+__device__ __forceinline__ void tile_write(const uint32_t (&o)[4], const uint64_t (&w)[4]) {
+  asm volatile("ds_write_b64 %0, %4\n\tds_write_b64 %1, %5\n\tds_write_b64 %2, %6\n\tds_write_b64 %3, %7"
+               :
+               : "v"(o[0]), "v"(o[1]), "v"(o[2]), "v"(o[3]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]));
+}
+template <typename V8>
+__device__ __forceinline__ void tile_read_tr(uint32_t o0, uint32_t o1, V8 (&f)[2]) {
+  typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
+  uint64_t r[4];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %5\n\t"
+      "ds_read_b64_tr_b16 %2, %4 offset:1024\n\tds_read_b64_tr_b16 %3, %5 offset:1024\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+      : "v"(o0), "v"(o1));
+  f[0] = __builtin_bit_cast(V8, (u64x2_t{r[0], r[1]}));
+  f[1] = __builtin_bit_cast(V8, (u64x2_t{r[2], r[3]}));
+}
+
+// Sum over the 4 lanes of a quad (every lane gets it)
+__device__ __forceinline__ float quad_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+}
+
+template <typename T, bool HAS_BIAS, int KB>
+__global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fused_row_kernel(
+    const gnn_triattn_bwd_args a) {
+  typedef typename TypeOps<T>::V8 V8;
+  typedef typename TypeOps<T>::V4 V4;
+  extern __shared__ __align__(256) unsigned char smem_raw[];
+  const int N = (int)a.N, H = (int)a.H, S = (int)a.S;
+  const int nb = (N + 31) / 32, nrows = 32 * nb, nth = (int)blockDim.x;
+  FusedBlock* blk = reinterpret_cast<FusedBlock*>(smem_raw);
+  int b, s, h;
+  row_coords(xcd_remap(blockIdx.x, gridDim.x), S, H, b, s, h);
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned char* tile = smem_raw + nb * sizeof(FusedBlock) + wave * 2048;  // this wave's dS tile [key][query]
+  const int64_t lrow = (((int64_t)b * S + s) * H + h) * N;
+  const float pl2 = dead_row_log2(a, a.lse[lrow]);  // query 0 exists (N >= 1)
+  const bool dead = pl2 != 0.f;                     // every query shares the row's keys
+
+  // ---- this wave's keys: K and V as B operands (lane = key, 8 consecutive d), and the key-side
+  // mask term (-inf for keys past N: p = 0)
+  const int kb0 = KB * wave;
+  V8 kf[KB][2], vf[KB][2];
+  float kbias[KB];
+  bool masked = false;
+#pragma unroll
+  for (int u = 0; u < KB; ++u) {
+    const int key = 32 * (kb0 + u) + l32;
+    const bool kok = key < N;
+    const T* kr = (const T*)a.k + b * a.k_stride[0] + s * a.k_stride[1] + h * a.k_stride[3] +
+                  (int64_t)(kok ? key : 0) * a.k_stride[2];
+    const T* vr = (const T*)a.v + b * a.v_stride[0] + s * a.v_stride[1] + h * a.v_stride[3] +
+                  (int64_t)(kok ? key : 0) * a.v_stride[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      kf[u][kk] = kok ? load8(kr + 16 * kk + 8 * g) : zero8<T>();
+      vf[u][kk] = kok ? load8(vr + 16 * kk + 8 * g) : zero8<T>();
+    }
+    kbias[u] = 0.f;
+    if (!kok)
+      kbias[u] = -INFINITY;
+    else if (a.mask && a.mask[b * a.mask_stride[0] + s * a.mask_stride[1] + (int64_t)key * a.mask_stride[2]] == 0)
+      kbias[u] = a.mask_value;
+    masked |= kbias[u] != 0.f;
+    if (!dead) kbias[u] *= LOG2E_R;  // joins the exponent there, the logit in a fully masked row
+  }
+  const int mode = dead ? 2 : __any(masked) ? 1 : 0;  // uniform over the wave
+
+  // ---- stage Q' and dO (rows past N are zero), form Delta, clear dQ
+  {
+    const T* qp = (const T*)a.q + b * a.q_stride[0] + s * a.q_stride[1] + h * a.q_stride[3];
+    const T* dp = (const T*)a.dout + b * a.do_stride[0] + s * a.do_stride[1] + h * a.do_stride[3];
+    const T* op = (const T*)a.o + b * a.o_stride[0] + s * a.o_stride[1] + h * a.o_stride[3];
+    constexpr int U = 2;
+    for (int base = 0; base < nrows * 4; base += nth * U) {
+      V8 xq[U], xd[U], xo[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = base + u * nth + tid, r = c >> 2, d0 = 8 * (c & 3);
+        const bool in = r < N;  // (N <= nrows, so chunks past the staged rows read nothing)
+        xq[u] = in ? load8(qp + (int64_t)r * a.q_stride[2] + d0) : zero8<T>();
+        xd[u] = in ? load8(dp + (int64_t)r * a.do_stride[2] + d0) : zero8<T>();
+        xo[u] = in ? load8(op + (int64_t)r * a.o_stride[2] + d0) : zero8<T>();
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = base + u * nth + tid, r = c >> 2;
+        const f32x8 x = TypeOps<T>::to_f32(xo[u]), y = TypeOps<T>::to_f32(xd[u]);
+        float part = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part = __builtin_fmaf(x[e], y[e], part);
+        const float delta = quad_sum(part);
+        if (c < nrows * 4) {
+          FusedBlock& B = blk[r >> 5];
+          *reinterpret_cast<V8*>(B.q + rswz(r & 31, c & 3)) =
+              TypeOps<T>::from_f32(TypeOps<T>::to_f32(xq[u]) * a.scale);
+          *reinterpret_cast<V8*>(B.d + rswz(r & 31, c & 3)) = xd[u];
+          if ((c & 3) == 0) {
+            B.ndelta[r & 31] = -delta;
+            if (r < N) a.delta[lrow + r] = delta;
+          }
+        }
+      }
+    }
+    for (int r = tid; r < nrows; r += nth) {
+      const float l = a.lse[lrow + (r < N ? r : 0)];
+      blk[r >> 5].nl[r & 31] = dead ? (r < N ? l : INFINITY) : (r < N ? -l * LOG2E_R : -INFINITY);
+    }
+    for (int c = tid; c < nb * 256; c += nth) blk[c >> 8].dq[c & 255] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // per-lane byte offsets inside a block's images and the tile: row fragments (row l32, chunks
+  // 2 kk + g), transposed reads (rows 16 kk + 8 hh + 4 g + .., see rtr_frag; kk adds 1024), tile rows
+  const int o_row0 = rswz(l32, g), o_row1 = rswz(l32, 2 + g);
+  const int r16 = lane & 15, tcol = 16 * ((lane >> 4) & 1) + 4 * (r16 & 3);
+  const int o_tr0 = rswz(4 * g + (r16 >> 2), tcol >> 3) + 2 * (tcol & 7);
+  const int o_tr1 = rswz(8 + 4 * g + (r16 >> 2), tcol >> 3) + 2 * (tcol & 7);
+  const uint32_t t0 = lds_addr(tile);
+  const uint32_t t_tr0 = t0 + o_tr0, t_tr1 = t0 + o_tr1;
+  const uint32_t t_wr[4] = {t0 + rswz(l32, 0) + 8 * g, t0 + rswz(l32, 1) + 8 * g, t0 + rswz(l32, 2) + 8 * g,
+                            t0 + rswz(l32, 3) + 8 * g};
+  auto tr = [&](const unsigned char* img, int kk) -> V8 {  // rtr_frag(img, 0, kk, lane)
+    const V4 x = rtr4<T>(img + o_tr0 + 1024 * kk), y = rtr4<T>(img + o_tr1 + 1024 * kk);
+    return V8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  };
+  // K transposed (B operand of dQ: k = key in the accumulator's row order, n = d), through the tile
+  V8 ktr[KB][2];
+#pragma unroll
+  for (int u = 0; u < KB; ++u) {
+    *reinterpret_cast<V8*>(tile + o_row0) = kf[u][0];
+    *reinterpret_cast<V8*>(tile + o_row1) = kf[u][1];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) ktr[u][kk] = tr(tile, kk);
+    __builtin_amdgcn_wave_barrier();
+  }
+  V8 idf[2];
+  ridentity<T>(idf, l32, g);
+  // bias rows of a query block: A = bias[query][key] (lane = query, 8 keys); queries past N read
+  // row N - 1 (their p is 0). The wave that holds the row's end zeroes the values of keys past N
+  // (the identity product multiplies them with zeros: they may be NaN), chunks past N read chunk 0.
+  const T* bias_plane = HAS_BIAS ? (const T*)a.bias + b * a.bias_stride[0] + h * a.bias_stride[1] : nullptr;
+  const uint32_t bpitch = HAS_BIAS ? (uint32_t)a.bias_stride[2] : 0;
+  const bool ktail = 32 * (kb0 + KB) > N;  // uniform; such a wave is a masked one
+  V8 bb[KB][2];
+  auto load_bias = [&](int u, int qb) {
+    const uint32_t row = (uint32_t)min(32 * qb + l32, N - 1) * bpitch;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int k0 = 32 * (kb0 + u) + 16 * t + 8 * g;
+      bb[u][t] = load8(bias_plane + (row + (k0 < N ? k0 : 0)));
+    }
+  };
+  auto cut_bias = [&](int u) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int nv = N - (32 * (kb0 + u) + 16 * t + 8 * g);  // values of the chunk that are keys
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e >= nv) bb[u][t][e] = TypeOps<T>::from_f32(0.f);
+    }
+  };
+  if constexpr (HAS_BIAS) {
+#pragma unroll
+    for (int u = 0; u < KB; ++u) load_bias(u, kb0);
+  }
+  f32x16 dk[KB], dv[KB];
+#pragma unroll
+  for (int u = 0; u < KB; ++u)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dk[u][i] = dv[u][i] = 0.f;
+  __syncthreads();
+
+  // MODE 0: no masked key in the wave's blocks and none past N. 1: the key-side term joins the
+  // exponent. 2: a row whose keys are all masked.
+  auto sweep = [&](auto mode_) {
+    constexpr int MODE = decltype(mode_)::value;
+    int qb = kb0;
+    for (int t = 0; t < nb; ++t) {
+      FusedBlock& B = blk[qb];
+      const int qn = qb + 1 == nb ? 0 : qb + 1;
+      f32x16 dq;
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        const f32x4 v = B.dq[64 * rg + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dq[4 * rg + e] = v[e];
+      }
+#pragma unroll
+      for (int u = 0; u < KB; ++u) {
+        if (MODE > 0 && u > 0 && kb0 + u >= nb) continue;  // uniform; no key there
+        // S[q][key] = Q' K^T (+ bias) and dP[q][key] - Delta_q = dO V^T - Delta (the accumulator
+        // starts at -Delta): rows = queries 32 qb + 8 (i / 4) + 4 g + i % 4, column = key
+        f32x16 sc, dp;
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const f32x4 nd4 = *reinterpret_cast<const f32x4*>(&B.ndelta[8 * rg + 4 * g]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sc[4 * rg + e] = 0.f;
+            dp[4 * rg + e] = nd4[e];
+          }
+        }
+        if constexpr (HAS_BIAS) {
+          if (MODE > 0 && ktail) cut_bias(u);
+#pragma unroll
+          for (int t2 = 0; t2 < 2; ++t2) Mma<T, PREC_NATIVE>::step(sc, bb[u][t2], idf[t2]);
+          load_bias(u, qn);
+        }
+        Mma<T, PREC_NATIVE>::step(sc, *reinterpret_cast<const V8*>(B.q + o_row0), kf[u][0]);
+        Mma<T, PREC_NATIVE>::step(dp, *reinterpret_cast<const V8*>(B.d + o_row0), vf[u][0]);
+        Mma<T, PREC_NATIVE>::step(sc, *reinterpret_cast<const V8*>(B.q + o_row1), kf[u][1]);
+        Mma<T, PREC_NATIVE>::step(dp, *reinterpret_cast<const V8*>(B.d + o_row1), vf[u][1]);
+        // P = exp2(S log2 e - lse log2 e [+ mask]); in a row whose keys are all masked S and lse
+        // both sit near the sentinel and are subtracted first
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const f32x4 l4 = *reinterpret_cast<const f32x4*>(&B.nl[8 * rg + 4 * g]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = 4 * rg + e;
+            const float x = MODE == 0   ? __builtin_fmaf(sc[i], LOG2E_R, l4[e])
+                            : MODE == 1 ? __builtin_fmaf(sc[i], LOG2E_R, l4[e] + kbias[u])
+                                        : __builtin_fmaf(sc[i] + kbias[u] - l4[e], LOG2E_R, pl2);
+            sc[i] = fast_exp2(x);
+            dp[i] *= sc[i];  // dS
+          }
+        }
+        // dS through the tile (row = key), dV += P^T dO and dK += dS^T Q' meanwhile: A = P / dS
+        // (lane = key, k = queries), B = the staged rows read transposed (k = queries, n = d)
+        const V8 dsf[2] = {racc_frag<T>(dp, 0), racc_frag<T>(dp, 1)};
+        typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
+        const u64x2_t d0 = __builtin_bit_cast(u64x2_t, dsf[0]), d1 = __builtin_bit_cast(u64x2_t, dsf[1]);
+        const uint64_t dw[4] = {d0[0], d0[1], d1[0], d1[1]};
+        tile_write(t_wr, dw);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          Mma<T, PREC_NATIVE>::step(dv[u], racc_frag<T>(sc, kk), tr(B.d, kk));
+          Mma<T, PREC_NATIVE>::step(dk[u], dsf[kk], tr(B.q, kk));
+        }
+        // dQ += dS K: A = dS (lane = query, k = keys)
+        V8 dst[2];
+        tile_read_tr(t_tr0, t_tr1, dst);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) Mma<T, PREC_NATIVE>::step(dq, dst[kk], ktr[u][kk]);
+      }
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)
+        B.dq[64 * rg + lane] = f32x4{dq[4 * rg], dq[4 * rg + 1], dq[4 * rg + 2], dq[4 * rg + 3]};
+      qb = qn;
+      // this wave's dQ block is written; after the barrier another wave takes it over
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+  };
+  if (mode == 0)
+    sweep(std::integral_constant<int, 0>{});
+  else if (mode == 1)
+    sweep(std::integral_constant<int, 1>{});
+  else
+    sweep(std::integral_constant<int, 2>{});
+
+  // dk / dv[m = key][n = d]: lane = d (l32), rows = keys 32 block + 8 (i / 4) + 4 g + i % 4
+  T* dkp = (T*)a.dk + b * a.dk_stride[0] + s * a.dk_stride[1] + h * a.dk_stride[3] + l32;
+  T* dvp = (T*)a.dv + b * a.dv_stride[0] + s * a.dv_stride[1] + h * a.dv_stride[3] + l32;
+#pragma unroll
+  for (int u = 0; u < KB; ++u)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int kj = (kb0 + u) * 32 + 8 * (i / 4) + 4 * g + (i % 4);
+      if (kj < N) {
+        dkp[(int64_t)kj * a.dk_stride[2]] = TypeOps<T>::from_f32(dk[u][i]);
+        dvp[(int64_t)kj * a.dv_stride[2]] = TypeOps<T>::from_f32(dv[u][i]);
+      }
+    }
+  // dq[m = query][n = d]: the accumulator layout of each block
+  T* dqg = (T*)a.dq + b * a.dq_stride[0] + s * a.dq_stride[1] + h * a.dq_stride[3] + l32;
+  for (int c = wave; c < nb; c += nth / 64) {
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      const f32x4 v = blk[c].dq[64 * rg + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int qq = 32 * c + 8 * rg + 4 * g + e;
+        if (qq < N) dqg[(int64_t)qq * a.dq_stride[2]] = TypeOps<T>::from_f32(v[e] * a.scale);
+      }
+    }
+  }
+}
+
+template <typename T, bool HAS_BIAS, int KB>
+int launch_bwd_fused(const gnn_triattn_bwd_args& a, hipStream_t stream) {
+  const void* fn = (const void*)bwd_fused_row_kernel<T, HAS_BIAS, KB>;
+  const size_t smem = fused_lds((int)a.N);
+  if (smem > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  hipLaunchKernelGGL((bwd_fused_row_kernel<T, HAS_BIAS, KB>), dim3((uint32_t)(a.B * a.S * a.H)),
+                     dim3(64 * fused_waves((int)a.N)), smem, stream, a);
+  return (int)hipGetLastError();
+}
+
 template <typename T, bool HAS_BIAS>
 int launch_bwd_row(const gnn_triattn_bwd_args& a, hipStream_t stream) {
+  // (the fused kernel addresses the bias plane in 32 bits)
+  if (a.N <= BWD_FUSED_MAX_N && (!HAS_BIAS || a.N * a.bias_stride[2] < ((int64_t)1 << 31)))
+    return fused_kb((int)a.N) == 2 ? launch_bwd_fused<T, HAS_BIAS, 2>(a, stream)
+                                   : launch_bwd_fused<T, HAS_BIAS, 1>(a, stream);
   const int64_t ntiles = (a.N + RT - 1) / RT;
   const dim3 grid((uint32_t)(a.B * a.S * a.H));
   const size_t smem_dq = DQ_HDR + 2 * (size_t)ntiles * RTILE;

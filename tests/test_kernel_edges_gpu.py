@@ -177,3 +177,64 @@ def test_fp32_backward_planes(N, C, Ch, B, direction):
     assert O.rel_fro(to_np(got[0]), want["x"]) <= 1e-4
     for k, g in zip(wg, got[1:]):
         assert abs(to_np(g) - want[k]).max() <= 1e-4 * max(float(abs(want[k]).max()), 1e-2 * scale), k
+
+
+# --------------------------------------------------------------------- attention, backward
+def _attention_grads(q, k, v, bias, mask, dout):
+    from geometric_nn_ops_torch.triangle import triangle_attention
+
+    leaves = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    leaves += [] if bias is None else [bias.to(DEV).requires_grad_()]
+    out = triangle_attention(*leaves[:3], None if bias is None else leaves[3], None if mask is None else mask.to(DEV))
+    return torch.autograd.grad(out, leaves, dout.to(DEV))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize(("N", "with_bias", "with_mask"), [
+    (1, True, False), (31, True, True), (32, False, True), (33, True, True), (64, True, False), (65, False, False),
+    (96, True, True), (255, True, True), (256, False, True), (257, True, True), (288, True, False),
+    (384, True, True), (385, True, True), (500, False, True), (512, True, True), (513, True, True)])
+def test_attention_backward_rows(N, with_bias, with_mask, dtype):
+    """Rows at and past a block of 32, the change of waves and blocks per wave (256, 384) and the longest
+    fused row (512); a key block of which a wave owns nothing (odd block counts); rows with no, some
+    and only masked keys side by side (fp16 without the last, whose sentinel does not swamp its
+    logits). Probabilities and their gradients are rounded once to the input dtype before each product
+    and the result once: about 3 roundings of 2^-9 (bf16) or 2^-12 (fp16)."""
+    S, H, D = 3, 2, 32
+    g = gen(300 + N)
+    q, k, v, dout = (torch.randn(1, S, N, H, D, generator=g).to(dtype) for _ in range(4))
+    bias = torch.randn(1, 1, H, N, N, generator=g).to(dtype) if with_bias else None
+    mask = None
+    if with_mask:
+        mask = torch.rand(1, S, 1, 1, N, generator=g) < 0.7
+        mask[:, 0] = True
+        mask[:, 1, ..., 0] = True
+        mask[:, 2] = dtype == torch.float16
+    got = _attention_grads(q, k, v, bias, mask, dout)
+    want = O.triangle_attention_grad(*(to_np(t) for t in (q, k, v)), None if bias is None else to_np(bias),
+                                     None if mask is None else mask.numpy(), D ** -0.5, to_np(dout))
+    for a, b in zip(got, want):
+        assert torch.isfinite(a).all()
+        # a single key's logit gradients are zeros, and rounding's leftovers have no relative error
+        assert O.rel_fro(to_np(a).reshape(b.shape), b) <= TOL[dtype] or abs(b).max() < 1e-12
+    again = _attention_grads(q, k, v, bias, mask, dout)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+def test_attention_backward_bias_padding_is_not_used():
+    """A bias view whose padding (keys past N) holds NaN, and strided q / k / v views."""
+    from geometric_nn_ops_torch.triangle import triangle_attention
+
+    N, H, D, dtype = 70, 2, 32, torch.bfloat16
+    g = gen(7)
+    q, k, v, dout = (torch.randn(1, N, N, H, D, generator=g).to(dtype) for _ in range(4))
+    wide = torch.full((1, 1, H, N, 80), float("nan"), dtype=dtype)
+    wide[..., :N] = torch.randn(1, 1, H, N, N, generator=g)
+    bias = wide.to(DEV)[..., :N].detach().requires_grad_()
+    leaves = [t.to(DEV).transpose(1, 2).detach().requires_grad_() for t in (q, k, v)]
+    out = triangle_attention(*leaves, bias)
+    got = torch.autograd.grad(out, [*leaves, bias], dout.to(DEV).transpose(1, 2))
+    want = _attention_grads(*(t.transpose(1, 2).contiguous() for t in (q, k, v)), wide[..., :N].contiguous(), None,
+                            dout.transpose(1, 2).contiguous())
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
