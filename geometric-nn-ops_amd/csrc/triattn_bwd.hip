@@ -52,6 +52,11 @@ constexpr int BNT = 256;    // threads per workgroup (4 waves)
 constexpr int ROWB = 64;    // bytes per staged row (32 x 16-bit)
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// Waves per SIMD that bwd_dq / bwd_dkdv keep registers for. Full-precision fp32 at D <= 32 fits three
+// (170 and 176 registers left to themselves; at N = 333 the two take 815 us together, with two 876).
+template <typename T, int DC, int PREC>
+constexpr int row_min_waves() { return DC > 2 ? 1 : sizeof(T) == 4 && DC == 1 && PREC == 1 ? 3 : 2; }
+
 // byte offset of (row r, 16-byte chunk c) in a [rows][32] 16-bit tile whose chunks are
 // XOR-swizzled by (r / 4) % 4: row-major fragment reads of 32 consecutive rows and the
 // transposed reads of 4-row groups both hit distinct bank groups.
@@ -154,7 +159,9 @@ struct DkdvLds {
 };
 
 template <typename T, bool HAS_BIAS, int DC, int PREC>
-__global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dkdv_kernel(const gnn_triattn_bwd_args a) {
+__global__ __launch_bounds__(BNT, (row_min_waves<T, DC, PREC>())) void bwd_dkdv_kernel(const gnn_triattn_bwd_args a) {
+  constexpr bool ADD_BIAS = HAS_BIAS && sizeof(T) == 4;
+  constexpr int NB = ADD_BIAS ? 2 : 1;
   typedef typename TypeOps<T>::V8 V8;
   __shared__ __align__(16) DkdvLds<T, DC> sm;
   const int N = (int)a.N, H = (int)a.H, D = (int)a.D;
@@ -208,9 +215,27 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dkdv_kernel(const gnn
 #pragma unroll
     for (int i = 0; i < 16; ++i) dk[dc][i] = dv[dc][i] = 0.f;
 
+  // What lies past N is not computed (a wave without keys only stages, a half tile without queries
+  // is skipped): at N = 131 a row takes 25 32 x 32 blocks instead of 48. With the bias off the
+  // matrix cores (below) dq and dk / dv in fp32 went from 1110 to 815 us at N = 333 (4 heads of 32)
+  // and from 187 to 146 at N = 160. Without gain: three or five waves a workgroup instead of four
+  // where that divides a row evenly (the SIMD that gets the extra wave sets the time).
+  const bool has_key = kb * 128 + wave * 32 < N;  // uniform
   const int ntq = (N + BT - 1) / BT;
   for (int tq = 0; tq < ntq; ++tq) {
     const int q0 = tq * BT;
+    // fp32 adds the bias itself (element i: query 8 (i / 4) + 4 g + i % 4 of the half, this lane's
+    // key; clamped into the plane, p past N is 0). As a product with identity fragments, cheap at
+    // 16-bit rates, it would be 16 of the loop's 80 fp32 MFMAs.
+    f32x16 bi[NB];
+    if constexpr (ADD_BIAS) {
+      const T* col = bias_plane + (key < N ? key : N - 1);
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          bi[sub][i] = col[(int64_t)min(q0 + 32 * sub + 8 * (i / 4) + 4 * g + (i % 4), N - 1) * a.bias_stride[2]];
+    }
     __syncthreads();  // the previous tile's reads are done
     // stage Q' = bf16(q * scale) and dO of 64 queries (256 threads: 64 rows x 4 chunks)
     {
@@ -233,9 +258,11 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dkdv_kernel(const gnn
       }
     }
     __syncthreads();
+    if (!has_key) continue;
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int r0 = sub * 32;
+      if (q0 + r0 >= N) break;  // uniform: no query there
       // S[q][key] = Q' K^T (+ bias): rows = queries r0 + 8 (i / 4) + 4 g + i % 4, column = key
       f32x16 sc, dp;
 #pragma unroll
@@ -247,7 +274,7 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dkdv_kernel(const gnn
           Mma<T, PREC>::step(sc, lds_row8<T>(sm.q[dc], r0 + l32, 2 * kk + g), kf[dc][kk]);
           Mma<T, PREC>::step(dp, lds_row8<T>(sm.d[dc], r0 + l32, 2 * kk + g), vf[dc][kk]);
         }
-      if constexpr (HAS_BIAS) {
+      if constexpr (HAS_BIAS && !ADD_BIAS) {
         // A = bias rows (lane = query, 8 consecutive keys of the wave's 32), B = identity
         const int qi = q0 + r0 + l32;
         const T* brow = bias_plane + (int64_t)(qi < N ? qi : 0) * a.bias_stride[2];
@@ -257,6 +284,10 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dkdv_kernel(const gnn
           const V8 bfr = qi < N ? load8_bias_tail<T>(brow, k0, N) : zero8<T>();
           Mma<T, PREC>::step(sc, bfr, idf[t]);
         }
+      }
+      if constexpr (ADD_BIAS) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] += bi[ADD_BIAS ? sub : 0][i];
       }
       // P and dS for this lane's key and its 16 queries
       f32x16 p, ds;
@@ -309,10 +340,14 @@ template <typename T, int DC>
 struct DqLds {
   unsigned char k[DC][BT * rowb<T>()];
   unsigned char v[DC][BT * rowb<T>()];
+  float kt[BT];  // added to the scores of a key: 0, the mask sentinel, or -inf past N
+  float km[BT];  // multiplies P: 1, or 1 / N_res for a masked key
 };
 
 template <typename T, bool HAS_BIAS, int DC, int PREC>
-__global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dq_kernel(const gnn_triattn_bwd_args a) {
+__global__ __launch_bounds__(BNT, (row_min_waves<T, DC, PREC>())) void bwd_dq_kernel(const gnn_triattn_bwd_args a) {
+  constexpr bool ADD_BIAS = HAS_BIAS && sizeof(T) == 4;
+  constexpr int NB = ADD_BIAS ? 2 : 1;
   typedef typename TypeOps<T>::V8 V8;
   __shared__ __align__(16) DqLds<T, DC> sm;
   const int N = (int)a.N, H = (int)a.H, D = (int)a.D;
@@ -375,10 +410,35 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dq_kernel(const gnn_t
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[dc][i] = 0.f;
 
+  const bool has_q = qb * 128 + wave * 32 < N;  // uniform; a wave without queries only stages
   const int ntk = (N + BT - 1) / BT;
   for (int tk = 0; tk < ntk; ++tk) {
     const int k0 = tk * BT;
+    // fp32 adds the bias itself (see bwd_dkdv_kernel): four consecutive keys a load; of a group that
+    // crosses N the padding may hold anything and is replaced below
+    f32x4 bi[NB][4];
+    if constexpr (ADD_BIAS) {
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const int key = k0 + 32 * sub + 8 * rg + 4 * g;
+          bi[sub][rg] = load4(brow + (key < N ? key : 0));
+        }
+    }
     __syncthreads();
+    if (tid < BT) {
+      const int key = k0 + tid;
+      float t = 0.f, m = 1.f;
+      if (key >= N) {
+        t = -INFINITY;
+      } else if (a.mask && a.mask[b * a.mask_stride[0] + s * a.mask_stride[1] + (int64_t)key * a.mask_stride[2]] == 0) {
+        t = a.mask_value;
+        m = 1.0f / (float)N;  // masked key: P / N_res
+      }
+      sm.kt[tid] = t;
+      sm.km[tid] = m;
+    }
     {
       const int r = tid >> 2, c = tid & 3;
       const int kj = k0 + r;
@@ -392,9 +452,11 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dq_kernel(const gnn_t
       }
     }
     __syncthreads();
+    if (!has_q) continue;
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int r0 = sub * 32;
+      if (k0 + r0 >= N) break;  // uniform: no key there
       // S^T[key][q] = K Q'^T (+ bias), dP^T[key][q] = V dO^T: rows = keys r0 + 8 (i / 4) + 4 g + i % 4
       f32x16 sc, dp;
 #pragma unroll
@@ -406,28 +468,34 @@ __global__ __launch_bounds__(BNT, DC > 2 ? 1 : 2) void bwd_dq_kernel(const gnn_t
           Mma<T, PREC>::step(sc, lds_row8<T>(sm.k[dc], r0 + l32, 2 * kk + g), qf[dc][kk]);
           Mma<T, PREC>::step(dp, lds_row8<T>(sm.v[dc], r0 + l32, 2 * kk + g), dof[dc][kk]);
         }
-      if constexpr (HAS_BIAS) {
+      if constexpr (HAS_BIAS && !ADD_BIAS) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const V8 bfr = qok ? load8_bias_tail<T>(brow, k0 + r0 + 16 * t + 8 * g, N) : zero8<T>();
           Mma<T, PREC>::step(sc, idf[t], bfr);
         }
       }
+      if constexpr (ADD_BIAS) {
+        if (k0 + r0 + 32 > N) {  // uniform
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (k0 + r0 + 8 * (i / 4) + 4 * g + (i % 4) >= N) bi[ADD_BIAS ? sub : 0][i / 4][i % 4] = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] += bi[ADD_BIAS ? sub : 0][i / 4][i % 4];
+      }
+      // subtract first: in a row whose keys are all masked both the logit and lse sit near the
+      // sentinel, and only their difference is exact
       f32x16 ds;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int kj = k0 + r0 + 8 * (i / 4) + 4 * g + (i % 4);
-        float x = sc[i], pm = 1.f;
-        if (kj >= N) {
-          x = -INFINITY;
-        } else if (a.mask && a.mask[b * a.mask_stride[0] + s * a.mask_stride[1] + (int64_t)kj * a.mask_stride[2]] == 0) {
-          x += a.mask_value;
-          pm = 1.0f / (float)N;  // masked key: P / N_res
+      for (int rg = 0; rg < 4; ++rg) {
+        const f32x4 t4 = *reinterpret_cast<const f32x4*>(&sm.kt[r0 + 8 * rg + 4 * g]);
+        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&sm.km[r0 + 8 * rg + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * rg + e;
+          ds[i] = fast_exp2((sc[i] + t4[e] - lse) * LOG2E_B) * m4[e] * (dp[i] - delta);
         }
-        // subtract first: in a row whose keys are all masked both x and lse sit near the
-        // sentinel, and only their difference is exact
-        const float pv = fast_exp2((x - lse) * LOG2E_B) * pm;
-        ds[i] = pv * (dp[i] - delta);
       }
       // dQ += dS K: A = dS^T accumulator (lane = query, k = keys), B = K read transposed
 #pragma unroll
@@ -571,6 +639,7 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_kernel(const gnn_triattn_b
     }
   };
   // one N_seq row of the tile from LDS: sum_s dS += P (dP - Delta)
+  const bool has_tile = q0 + qw < N && k0 + kw < N;  // uniform over the wave
   auto compute_row = [&]() {
     // dO fragments negated and the dP accumulator started at Delta: the MFMA yields Delta - dP
     V8 qf[DC][2], ndof[DC][2];
@@ -626,14 +695,14 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_kernel(const gnn_triattn_b
     for (; s + PF <= s_end; s += PF) {
 #pragma unroll
       for (int ph = 0; ph < PF; ++ph) {
-        compute_row();
+        if (has_tile) compute_row();
         __syncthreads();
         store_stage(ph);  // row s + ph + 1
         __syncthreads();
         load_stage(ph, min(s + ph + 1 + PF, last));
       }
     }
-    if (s < s_end) compute_row();  // PF = 2 and an odd number of rows: the last one is in LDS
+    if (s < s_end && has_tile) compute_row();  // PF = 2 and an odd number of rows: the last one is in LDS
   }
   // [B, H, N, N] fp32: the final gradient, or this split's slice of the workspace
   float* out = (splits > 1 ? a.dbias_ws + (int64_t)split * a.B * H * N * N : a.dbias) + ((int64_t)b * H + h) * N * N;

@@ -238,3 +238,37 @@ def test_attention_backward_bias_padding_is_not_used():
                             dout.transpose(1, 2).contiguous())
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize(("N", "D", "with_bias", "with_mask"), [
+    (1, 32, True, False), (31, 32, True, True), (33, 64, True, True), (64, 32, True, True), (65, 48, True, False),
+    (97, 32, False, True), (128, 64, True, True), (129, 32, True, True), (160, 32, True, True), (161, 40, True, True)])
+def test_fp32_attention_partial_tiles(N, D, with_bias, with_mask):
+    """fp32 rows that end within a half tile of 32, leave a half tile or a wave's 32 queries or keys
+    empty, and their neighbours, with NaN in the bias's padding where the view has any. Sums of at
+    most 161 products of fp32 operands against fp64: a few hundred roundings of 2^-24 at the worst."""
+    from geometric_nn_ops_torch.triangle import triangle_attention
+
+    S, H = 3, 2
+    g = gen(500 + N)
+    q, k, v, dout = (torch.randn(1, S, N, H, D, generator=g) for _ in range(4))
+    bias = torch.randn(1, 1, H, N, N, generator=g) if with_bias else None
+    mask = None
+    if with_mask:
+        mask = torch.rand(1, S, 1, 1, N, generator=g) < 0.7
+        mask[:, 0] = True
+        mask[:, 1, ..., 0] = True
+        mask[:, 2] = False
+    leaves = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    if with_bias:
+        wide = torch.full((1, 1, H, N, (N + 7) // 8 * 8), float("nan"))
+        wide[..., :N] = bias
+        leaves.append(wide.to(DEV)[..., :N].detach().requires_grad_())
+    out = triangle_attention(*leaves[:3], leaves[3] if with_bias else None, None if mask is None else mask.to(DEV))
+    got = torch.autograd.grad(out, leaves, dout.to(DEV))
+    args = (*(to_np(t) for t in (q, k, v)), None if bias is None else to_np(bias),
+            None if mask is None else mask.numpy(), D ** -0.5)
+    assert O.rel_fro(to_np(out), O.triangle_attention(*args).reshape(out.shape)) <= 3e-5
+    for a, b in zip(got, O.triangle_attention_grad(*args, to_np(dout))):
+        assert torch.isfinite(a).all()
+        assert O.rel_fro(to_np(a).reshape(b.shape), b) <= 3e-5 or abs(b).max() < 1e-12
