@@ -53,13 +53,14 @@ def _prepare_bias(bias: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """``[B, 1, H, N, N]`` bias in ``dtype``. The 16-bit row kernel reads any strides (its
     pre-pass rewrites the bias in fragment order); the tiled kernel needs unit key stride, a
     query pitch that is a multiple of 8 elements and a 16-byte aligned base, so such views
-    are copied with the pitch padded (zeros past N)."""
+    are copied with the pitch padded. No kernel uses what lies past N, so the padding is not
+    filled (the fill cost 5 us of a 145 us forward at N = 333 in fp32)."""
     bias = bias.to(dtype)
     if bias.stride(-1) == 1 and bias.stride(-2) % 8 == 0 and bias.data_ptr() % 16 == 0:
         return bias
     B, _, H, N, _ = bias.shape
     pitch = (N + 7) // 8 * 8
-    padded = torch.zeros((B, 1, H, N, pitch), device=bias.device, dtype=bias.dtype)
+    padded = torch.empty((B, 1, H, N, pitch), device=bias.device, dtype=bias.dtype)
     padded[..., :N] = bias
     return padded[..., :N]
 

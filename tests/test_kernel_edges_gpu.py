@@ -221,14 +221,18 @@ def test_attention_backward_rows(N, with_bias, with_mask, dtype):
     assert all(torch.equal(a, b) for a, b in zip(got, again))
 
 
-def test_attention_backward_bias_padding_is_not_used():
-    """A bias view whose padding (keys past N) holds NaN, and strided q / k / v views."""
+@pytest.mark.parametrize(("N", "S", "D", "dtype"), [
+    (70, 70, 32, torch.bfloat16), (70, 3, 64, torch.bfloat16), (521, 2, 32, torch.float16), (70, 3, 128, torch.float16),
+    (70, 3, 32, torch.float32), (131, 3, 64, torch.float32)])
+def test_attention_bias_padding_is_not_used(N, S, D, dtype):
+    """A bias view whose padding (keys past N) holds NaN, and strided q / k / v views: the same bits
+    as from packed tensors, forward and backward."""
     from geometric_nn_ops_torch.triangle import triangle_attention
 
-    N, H, D, dtype = 70, 2, 32, torch.bfloat16
+    H = 2
     g = gen(7)
-    q, k, v, dout = (torch.randn(1, N, N, H, D, generator=g).to(dtype) for _ in range(4))
-    wide = torch.full((1, 1, H, N, 80), float("nan"), dtype=dtype)
+    q, k, v, dout = (torch.randn(1, N, S, H, D, generator=g).to(dtype) for _ in range(4))
+    wide = torch.full((1, 1, H, N, (N + 15) // 8 * 8), float("nan"), dtype=dtype)
     wide[..., :N] = torch.randn(1, 1, H, N, N, generator=g)
     bias = wide.to(DEV)[..., :N].detach().requires_grad_()
     leaves = [t.to(DEV).transpose(1, 2).detach().requires_grad_() for t in (q, k, v)]
@@ -236,6 +240,7 @@ def test_attention_backward_bias_padding_is_not_used():
     got = torch.autograd.grad(out, [*leaves, bias], dout.to(DEV).transpose(1, 2))
     want = _attention_grads(*(t.transpose(1, 2).contiguous() for t in (q, k, v)), wide[..., :N].contiguous(), None,
                             dout.transpose(1, 2).contiguous())
+    assert torch.isfinite(out).all()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
 
