@@ -8,6 +8,7 @@ call raises RuntimeError naming the path that was tried.
 import ctypes
 import os
 import pathlib
+import struct
 import threading
 
 import torch
@@ -23,6 +24,23 @@ PRECISION_CODE = {"ieee": GNN_PREC_IEEE, "bf16x3": GNN_PREC_BF16X3}
 
 I64x3 = ctypes.c_int64 * 3
 I64x4 = ctypes.c_int64 * 4
+
+
+_FORMATS = {ctypes.c_void_p: "P", ctypes.c_int64: "q", ctypes.c_int32: "i", ctypes.c_float: "f", ctypes.c_size_t: "N"}
+
+
+def packer(cls):
+    """``pack_into(args, 0, *values)`` of an argument structure: every field in order, arrays
+    flattened, NULL as 0. One call instead of one assignment per field: calls whose kernels take
+    less than their host time are bound by it (with the raw stream handle in ``call``, attention
+    at N = 256 went from 34.8 to 29.6 us)."""
+    fmt = "@"
+    for _, typ in cls._fields_:
+        count = getattr(typ, "_length_", None)
+        fmt += f"{count}{_FORMATS[typ._type_]}" if count else _FORMATS[typ]
+    s = struct.Struct(fmt)
+    assert ctypes.sizeof(cls) - ctypes.alignment(cls) < s.size <= ctypes.sizeof(cls)
+    return s.pack_into
 
 
 class TriAttnArgs(ctypes.Structure):
@@ -55,6 +73,9 @@ class TriAttnArgs(ctypes.Structure):
         ("workspace", ctypes.c_void_p),
         ("workspace_bytes", ctypes.c_size_t),
     ]
+
+
+pack_triattn = packer(TriAttnArgs)
 
 
 class TriAttnBwdArgs(ctypes.Structure):
@@ -98,6 +119,9 @@ class TriAttnBwdArgs(ctypes.Structure):
     ]
 
 
+pack_triattn_bwd = packer(TriAttnBwdArgs)
+
+
 class TrimulArgs(ctypes.Structure):
     """Mirror of ``gnn_trimul_args``."""
 
@@ -132,6 +156,9 @@ class TrimulArgs(ctypes.Structure):
         ("ln_in_channels", ctypes.c_int64),
         ("ln_out_channels", ctypes.c_int64),
     ]
+
+
+pack_trimul = packer(TrimulArgs)
 
 
 class ApbGateOutArgs(ctypes.Structure):
@@ -456,14 +483,18 @@ def call(fn_name: str, args, device: torch.device) -> None:
     """``fn_name(&args, stream)`` on ``device``'s current stream, with ``device`` current for
     the call (the current device is switched only when it differs: the guard costs host time
     on every launch), raising on a non-zero status."""
-    fn = getattr(load(), fn_name)
+    fn = getattr(_lib or load(), fn_name)
     idx = device.index
-    if idx is None or idx == torch.cuda.current_device():
-        rc = fn(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream))
+    if idx is None or device.type != "cuda":
+        rc = fn(ctypes.byref(args), stream_handle(device))
+    elif idx == torch.cuda.current_device():
+        # the handle itself: building a torch.cuda.Stream around it takes 1.5 us a launch
+        rc = fn(ctypes.byref(args), torch._C._cuda_getCurrentRawStream(idx))
     else:
         with torch.cuda.device(idx):
-            rc = fn(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream))
-    check(rc, fn_name)
+            rc = fn(ctypes.byref(args), torch._C._cuda_getCurrentRawStream(idx))
+    if rc != GNN_OK:
+        check(rc, fn_name)
 
 
 def ptr(t) -> int | None:

@@ -25,8 +25,9 @@ HIP_ALLOWED = ("ieee", "bf16x3")
 
 def torch_precision() -> str:
     """torch's current fp32 matmul precision (reference _precision.py:44-54)."""
-    if hasattr(torch.backends.cuda.matmul, "fp32_precision"):
-        return TF32 if torch.backends.cuda.matmul.fp32_precision == TF32 else IEEE
+    setting = getattr(torch.backends.cuda.matmul, "fp32_precision", None)
+    if setting is not None:
+        return TF32 if setting == TF32 else IEEE
     return TF32 if torch.backends.cuda.matmul.allow_tf32 else IEEE
 
 

@@ -18,7 +18,7 @@ reference runs as stock torch ops. Here:
   cover and calls above ``GATE_OUT_MAX_WORK`` take torch's linear layers.
 """
 
-import ctypes
+import functools
 
 import torch
 import torch.nn.functional as F
@@ -36,16 +36,23 @@ def projection_supported(z: torch.Tensor, heads: int) -> bool:
     return zc % 8 == 0 and zc <= MAX_ZC and heads * zc <= MAX_HEADS_X_ZC
 
 
+def _ready(t, dtype):
+    """``t`` contiguous in ``dtype`` (as is when it already is: the checks cost less than the calls)."""
+    if t is None or (t.dtype == dtype and t.is_contiguous()):
+        return t
+    return t.to(dtype).contiguous()
+
+
 def pair_bias_projection_hip(z, ln_z_weight, proj_z_weight, eps=1e-5):
     """``z [B, U, V, Zc]`` -> ``[B, H, U, V]`` in z's dtype. The result is a view with a
     row pitch rounded up to 8 elements (what the attention kernel reads without a copy)."""
     B, U, V, Zc = z.shape
     H = proj_z_weight.shape[0]
     z = z.contiguous()
-    w = proj_z_weight.to(z.dtype).contiguous()
-    gamma = None if ln_z_weight is None else ln_z_weight.to(z.dtype).contiguous()
+    w = _ready(proj_z_weight, z.dtype)
+    gamma = _ready(ln_z_weight, z.dtype)
     pitch = (V + 7) // 8 * 8
-    buf = (torch.empty if pitch == V else torch.zeros)((B, H, U, pitch), device=z.device, dtype=z.dtype)
+    buf = torch.empty((B, H, U, pitch), device=z.device, dtype=z.dtype)  # nothing reads past V
     a = _lib.PairBiasArgs()
     a.z, a.proj_w, a.out = z.data_ptr(), w.data_ptr(), buf.data_ptr()
     a.ln_w = None if gamma is None else gamma.data_ptr()
@@ -90,12 +97,10 @@ def gate_out_hip(s, o, proj_g_weight, proj_g_bias, proj_o_weight, proj_o_bias):
     s2 = s.reshape(-1, cs)
     if s2.stride(-1) != 1 or (s2.stride(0) * s2.element_size()) % 16 or s2.data_ptr() % 16:
         s2 = s2.contiguous()
-    o2 = o.reshape(-1, d).to(dt).contiguous()
+    o2 = _ready(o.reshape(-1, d), dt)
     m = s2.shape[0]
-    gw = proj_g_weight.to(dt).contiguous()
-    ow = proj_o_weight.to(dt).contiguous()
-    gb = None if proj_g_bias is None else proj_g_bias.to(dt).contiguous()
-    ob = None if proj_o_bias is None else proj_o_bias.to(dt).contiguous()
+    gw, ow = _ready(proj_g_weight, dt), _ready(proj_o_weight, dt)
+    gb, ob = _ready(proj_g_bias, dt), _ready(proj_o_bias, dt)
     out = torch.empty((m, co), device=s.device, dtype=dt)
     a = _lib.ApbGateOutArgs()
     a.s, a.o, a.g_w, a.o_w, a.out = s2.data_ptr(), o2.data_ptr(), gw.data_ptr(), ow.data_ptr(), out.data_ptr()
@@ -107,6 +112,12 @@ def gate_out_hip(s, o, proj_g_weight, proj_g_bias, proj_o_weight, proj_o_bias):
     a.precision = _lib.PRECISION_CODE[_precision.matmul_precision(fp32_operands=dt == torch.float32)]
     _lib.call("gnn_apb_gate_out", a, s.device)
     return out.reshape(*lead, co)
+
+
+@functools.lru_cache(maxsize=64)
+def _rounded(value: float, dtype: torch.dtype) -> float:
+    """``value`` rounded to ``dtype`` (three tensor operations on the host)."""
+    return float(torch.tensor(value, dtype=torch.float64).to(dtype).to(torch.float32))
 
 
 def attention_pair_bias_hip(s, q, k, v, z, *, proj_g_weight, proj_o_weight, proj_z_weight=None,
@@ -140,7 +151,7 @@ def attention_pair_bias_hip(s, q, k, v, z, *, proj_g_weight, proj_o_weight, proj
         logits_dtype = torch.promote_types(q.dtype, pz.dtype)
         magnitude = mask_val(logits_dtype) if inf is None else float(inf)
         # the reference adds (keep - 1) * inf in the logits' dtype
-        mask_value = float(torch.tensor(-magnitude, dtype=torch.float64).to(logits_dtype).to(torch.float32))
+        mask_value = _rounded(-magnitude, logits_dtype)
     o = triangle_attention_hip(canon(q, U), canon(k, V), canon(v, V), bias=pz.unsqueeze(1), mask=keep,
                                scale=scale, mask_value=mask_value)
     o = o.reshape(BM, U, H * DH).to(s.dtype)

@@ -10,6 +10,7 @@ unusable), and the output is a fresh contiguous ``[B, N_seq, N_res, H, D]`` tens
 """
 
 import ctypes
+import functools
 
 import torch
 
@@ -31,9 +32,10 @@ def supports(q: torch.Tensor) -> bool:
 
 
 def _vectorizable(t: torch.Tensor) -> bool:
-    """Unit stride on the last dim, the other strides multiples of 8 elements, 16-byte base."""
-    st = t.stride()
-    return t.data_ptr() % 16 == 0 and st[-1] == 1 and all(x % 8 == 0 for x in st[:-1])
+    """Unit stride on the last of five dims, the other strides multiples of 8 elements, 16-byte
+    base."""
+    s0, s1, s2, s3, s4 = t.stride()
+    return s4 == 1 and (s0 | s1 | s2 | s3) % 8 == 0 and t.data_ptr() % 16 == 0
 
 
 def _prepare(t: torch.Tensor) -> torch.Tensor:
@@ -128,34 +130,34 @@ def triangle_attention_hip(q, k, v, bias=None, mask=None, scale=None, dynamic=Fa
     Dp = qk.shape[-1]
     o = torch.empty((B, S, N, H, Dp), device=q.device, dtype=q.dtype)
 
-    args = _lib.TriAttnArgs()
-    args.q, args.k, args.v, args.o = qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), o.data_ptr()
-    args.B, args.S, args.N, args.H, args.D = B, S, N, H, Dp
-    args.q_stride = _lib.I64x4(*qk.stride()[:4])
-    args.k_stride = _lib.I64x4(*kk.stride()[:4])
-    args.v_stride = _lib.I64x4(*vk.stride()[:4])
-    args.o_stride = _lib.I64x4(*o.stride()[:4])
-    args.dtype = _lib.DTYPE_CODE[q.dtype]
+    bias_ptr, (b0, b1, b2, b3) = 0, (0, 0, 0, 0)
     if bias is not None:
-        bias = bias_for_kernel(args, bias, q.dtype)
+        bias = bias.to(q.dtype)
+        bias_ptr, (b0, _, b1, b2, b3) = bias.data_ptr(), bias.stride()
+    mask_ptr, (m0, m1, _, _, m2) = 0, (0, 0, 0, 0, 0)
     if mask is not None:
         if mask.dtype != torch.bool:
             raise ValueError(f"mask must be bool (keep=True/mask=False), got {mask.dtype}")
-        args.mask = mask.data_ptr()
-        args.mask_stride = _lib.I64x3(mask.stride(0), mask.stride(1), mask.stride(4))
-    if lse is not None:
-        assert lse.shape == (B, S, H, N) and lse.dtype == torch.float32 and lse.is_contiguous()
-        args.lse = lse.data_ptr()
-    if row_max is not None:
-        assert row_max.shape == (B, S, H, N) and row_max.dtype == torch.float32 and row_max.is_contiguous()
-        args.row_max = row_max.data_ptr()
-    args.scale = float(scale)
-    args.mask_value = rounded_mask_value(q.dtype) if mask_value is None else float(mask_value)
+        mask_ptr, (m0, m1, _, _, m2) = mask.data_ptr(), mask.stride()
+    for t in (lse, row_max):
+        assert t is None or (t.shape == (B, S, H, N) and t.dtype == torch.float32 and t.is_contiguous())
     if precision is None:
         precision = _precision.matmul_precision(fp32_operands=q.dtype == torch.float32)
-    args.precision = _lib.PRECISION_CODE[precision]
+    args = _lib.TriAttnArgs()
+    _lib.pack_triattn(
+        args, 0, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), o.data_ptr(), bias_ptr, mask_ptr,
+        0 if lse is None else lse.data_ptr(), 0 if row_max is None else row_max.data_ptr(), B, S, N, H, Dp,
+        *qk.stride()[:4], *kk.stride()[:4], *vk.stride()[:4], *o.stride()[:4], b0, b1, b2, b3, m0, m1, m2,
+        0.0, 0.0, _lib.DTYPE_CODE[q.dtype], _lib.PRECISION_CODE[precision], 0, 0)
+    args.scale = float(scale)
+    args.mask_value = rounded_mask_value(q.dtype) if mask_value is None else float(mask_value)
 
-    ws = workspace_for(args, q.device)
+    ws = None
+    if bias is not None:  # scratch where the row-resident kernel runs, the tiled kernel's layout elsewhere
+        ws = workspace_for(args, q.device)
+        if ws is None:
+            bias = _prepare_bias(bias, q.dtype)
+            _set_bias(args, bias)
     _lib.call("gnn_triattn_fwd", args, q.device)
     del ws
     if Dp != D:
@@ -179,6 +181,7 @@ _ROW_S = 1.5e-6  # one N_seq row of a 128 x 128 tile (measured at D = 32)
 _PLANE_BPS = 5.0e12  # a partial plane is written once and read once by the ordered reduction
 
 
+@functools.lru_cache(maxsize=256)
 def dbias_splits(B: int, S: int, N: int, H: int) -> int:
     """N_seq ranges for the pair-bias gradient (at most N_seq and 64), minimising a cost
     model: the rounds of (128 x 128 tile, range) workgroups over the compute units times the
@@ -212,40 +215,32 @@ def triangle_attention_bwd_hip(q, k, v, o, dout, lse, bias=None, mask=None, scal
     dk = torch.empty_like(dq)
     dv = torch.empty_like(dq)
     delta = torch.empty((B, S, H, N), device=q.device, dtype=torch.float32)
-    a = _lib.TriAttnBwdArgs()
-    a.q, a.k, a.v, a.o, a.dout = qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), ok.data_ptr(), dk_.data_ptr()
-    a.lse = lse.contiguous().data_ptr()
-    a.dq, a.dk, a.dv, a.delta = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr()
-    a.B, a.S, a.N, a.H, a.D = B, S, N, H, D
-    a.q_stride = _lib.I64x4(*qk.stride()[:4])
-    a.k_stride = _lib.I64x4(*kk.stride()[:4])
-    a.v_stride = _lib.I64x4(*vk.stride()[:4])
-    a.o_stride = _lib.I64x4(*ok.stride()[:4])
-    a.do_stride = _lib.I64x4(*dk_.stride()[:4])
-    a.dq_stride = _lib.I64x4(*dq.stride()[:4])
-    a.dk_stride = _lib.I64x4(*dk.stride()[:4])
-    a.dv_stride = _lib.I64x4(*dv.stride()[:4])
-    dbias = None
+    lse = lse.contiguous()
+    dbias, ws, splits = None, None, 0
+    bias_ptr, (b0, b1, b2, b3) = 0, (0, 0, 0, 0)
     if bias is not None:
         bias = _prepare_bias(bias, q.dtype)
-        a.bias = bias.data_ptr()
-        a.bias_stride = _lib.I64x4(bias.stride(0), bias.stride(2), bias.stride(3), bias.stride(4))
+        bias_ptr, (b0, _, b1, b2, b3) = bias.data_ptr(), bias.stride()
         if need_dbias:
             dbias = torch.empty((B, 1, H, N, N), device=q.device, dtype=torch.float32)
-            a.dbias = dbias.data_ptr()
             splits = dbias_splits(B, S, N, H)
-            a.dbias_splits = splits
             if splits > 1:
                 ws = torch.empty((splits, B, H, N, N), device=q.device, dtype=torch.float32)
-                a.dbias_ws = ws.data_ptr()
+    mask_ptr, (m0, m1, _, _, m2) = 0, (0, 0, 0, 0, 0)
     if mask is not None:
-        a.mask = mask.data_ptr()
-        a.mask_stride = _lib.I64x3(mask.stride(0), mask.stride(1), mask.stride(4))
-    a.scale = float(scale)
-    a.mask_value = rounded_mask_value(q.dtype) if mask_value is None else float(mask_value)
-    a.dtype = _lib.DTYPE_CODE[q.dtype]
+        mask_ptr, (m0, m1, _, _, m2) = mask.data_ptr(), mask.stride()
     if precision is None:
         precision = _precision.matmul_precision(fp32_operands=q.dtype == torch.float32)
-    a.precision = _lib.PRECISION_CODE[precision]
+    grad_stride = dq.stride()[:4]  # dk and dv have it too
+    a = _lib.TriAttnBwdArgs()
+    _lib.pack_triattn_bwd(
+        a, 0, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), ok.data_ptr(), dk_.data_ptr(), bias_ptr, mask_ptr,
+        lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), 0 if dbias is None else dbias.data_ptr(),
+        delta.data_ptr(), 0 if ws is None else ws.data_ptr(), splits, B, S, N, H, D,
+        *qk.stride()[:4], *kk.stride()[:4], *vk.stride()[:4], *ok.stride()[:4], *dk_.stride()[:4],
+        *grad_stride, *grad_stride, *grad_stride, b0, b1, b2, b3, m0, m1, m2,
+        0.0, 0.0, _lib.DTYPE_CODE[q.dtype], _lib.PRECISION_CODE[precision])
+    a.scale = float(scale)
+    a.mask_value = rounded_mask_value(q.dtype) if mask_value is None else float(mask_value)
     _lib.call("gnn_triattn_bwd", a, q.device)
     return dq, dk, dv, dbias

@@ -8,6 +8,7 @@ one workspace tensor allocated here through torch's caching allocator.
 """
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -19,14 +20,6 @@ _WEIGHT_KEYS = (
     "norm_in_weight", "norm_in_bias", "p_in_weight", "p_in_bias", "g_in_weight", "g_in_bias",
     "norm_out_weight", "norm_out_bias", "p_out_weight", "p_out_bias", "g_out_weight", "g_out_bias",
 )
-_ARG_FIELD = {
-    "norm_in_weight": "ln_in_w", "norm_in_bias": "ln_in_b",
-    "p_in_weight": "p_in_w", "p_in_bias": "p_in_b",
-    "g_in_weight": "g_in_w", "g_in_bias": "g_in_b",
-    "norm_out_weight": "ln_out_w", "norm_out_bias": "ln_out_b",
-    "p_out_weight": "p_out_w", "p_out_bias": "p_out_b",
-    "g_out_weight": "g_out_w", "g_out_bias": "g_out_b",
-}
 MAX_CHANNELS = 512
 WIDE_MAX_CHANNELS = 8192  # the wide-row LayerNorm's limit (gnn_layernorm_rows forward)
 
@@ -100,11 +93,6 @@ def _parts(n, k):
     return [(i * step, (i + 1) * step) for i in range(k)]
 
 
-def _expect(name, t, shape):
-    if t is not None and t.shape != shape:
-        raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
-
-
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     t = t.contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
@@ -116,6 +104,14 @@ def _kernel_ready(t: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
     if t.dtype == like.dtype and t.device == like.device and t.is_contiguous() and t.data_ptr() % 16 == 0:
         return t
     return _aligned(t.to(device=like.device, dtype=like.dtype))
+
+
+@functools.lru_cache(maxsize=256)
+def _workspace_layout(B, N, C, Ch, dtype):
+    """(bytes, offsets of a, b, gate and o) of the forward's workspace."""
+    offsets = (ctypes.c_size_t * 4)()
+    nbytes = _lib.load().gnn_trimul_workspace_bytes(B, N, C, Ch, dtype, offsets)
+    return nbytes, tuple(offsets)
 
 
 def build_args(x, direction, mask, eps, weights, separate_gate=False):
@@ -141,7 +137,9 @@ def build_args(x, direction, mask, eps, weights, separate_gate=False):
         "g_in_bias": (2 * Ch,), "p_out_bias": (C,), "g_out_bias": (C,),
     }
     for key, shape in expected.items():
-        _expect(key, weights.get(key), shape)
+        w = weights.get(key)
+        if w is not None and w.shape != shape:
+            raise ValueError(f"{key} has shape {tuple(w.shape)}, expected {tuple(shape)}")
     lead = x.shape[:-3]
     B = math.prod(lead)
 
@@ -149,38 +147,40 @@ def build_args(x, direction, mask, eps, weights, separate_gate=False):
     out = torch.empty((B, N, N, C), device=x.device, dtype=x.dtype)
     keep = [xk]
 
-    args = _lib.TrimulArgs()
-    args.x, args.out = xk.data_ptr(), out.data_ptr()
+    mask_ptr, mask_stride = 0, (0, 0, 0)
     if mask is not None:
         m = mask.to(device=x.device, dtype=x.dtype).expand(*x.shape[:-1]).reshape(B, N, N)
         keep.append(m)
-        args.mask = m.data_ptr()
-        args.mask_stride = _lib.I64x3(*m.stride())
+        mask_ptr, mask_stride = m.data_ptr(), m.stride()
+    ptrs = []  # in _WEIGHT_KEYS order, which is the order of the structure's fields
+    xdt, xdev = x.dtype, x.device
     for key in _WEIGHT_KEYS:
         w = weights.get(key)
         if w is None:
+            ptrs.append(0)
             continue
-        w = _kernel_ready(w, x)
+        p = w.data_ptr()
+        if p % 16 or w.dtype != xdt or w.device != xdev or not w.is_contiguous():
+            w = _kernel_ready(w, x)
+            p = w.data_ptr()
         keep.append(w)
-        setattr(args, _ARG_FIELD[key], w.data_ptr())
-    dtype = _lib.DTYPE_CODE[x.dtype]
-    offsets = (ctypes.c_size_t * 4)()
-    lib = _lib.load()
-    nbytes = lib.gnn_trimul_workspace_bytes(B, N, C, Ch, dtype, offsets)
+        ptrs.append(p)
+    dtype = _lib.DTYPE_CODE[xdt]
+    nbytes, offsets = _workspace_layout(B, N, C, Ch, dtype)
+    gate_ptr = 0
     if separate_gate:  # the gate region is the workspace's last: stop before it
         nbytes = offsets[2]
         gate = torch.empty((B, N, N, C), device=x.device, dtype=x.dtype)
         keep.append(gate)
-        args.gate = gate.data_ptr()
+        gate_ptr = gate.data_ptr()
     workspace = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
-    args.workspace, args.workspace_bytes = workspace.data_ptr(), nbytes
-    args.B, args.N, args.C, args.Ch = B, N, C, Ch
-    args.eps = float(eps)
-    args.outgoing = 1 if outgoing else 0
-    args.dtype = dtype
     precision = _precision.matmul_precision(fp32_operands=x.dtype == torch.float32)
-    args.precision = _lib.PRECISION_CODE[precision]
-    return args, keep, out, workspace, tuple(offsets)
+    args = _lib.TrimulArgs()
+    _lib.pack_trimul(args, 0, xk.data_ptr(), out.data_ptr(), mask_ptr, *mask_stride, *ptrs, workspace.data_ptr(),
+                     nbytes, B, N, C, Ch, 0.0, 1 if outgoing else 0, dtype, _lib.PRECISION_CODE[precision], gate_ptr,
+                     0, 0)
+    args.eps = float(eps)
+    return args, keep, out, workspace, offsets
 
 
 def run_stage(fn_name: str, args, device) -> None:
