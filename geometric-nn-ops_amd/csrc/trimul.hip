@@ -1907,58 +1907,59 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_x3_kernel(const float* 
 // N = 384, C = c_hidden = 128).
 constexpr int PTO = 64;
 constexpr int OPC = 128;                  // output channels per pass (4 waves x 32)
-constexpr int OCH = PTO * OPC / 8 / NT;  // 8-element chunks per thread per pass
+template <int PT>
+constexpr int out_chunks() { return PT * OPC / 8 / NT; }  // 8-element chunks per thread per pass
 
 // LDS of the output stage: region 1 = the raw o tile [Ch][PTO + pad], reused after the
 // LayerNorm as the pass tile [PTO][OPC + pad]; then the normalised tile [PTO][Ch + pad] (T),
 // LN gamma / beta [Ch] and the LayerNorm partial sums [2][4][PTO] (fp32).
-__host__ __device__ inline size_t out_region1_elems(int64_t Ch, int pad) {
-  const int64_t o = Ch * (PTO + pad), y = (int64_t)PTO * (OPC + pad);
+__host__ __device__ inline size_t out_region1_elems(int64_t Ch, int pad, int pt = PTO) {
+  const int64_t o = Ch * (pt + pad), y = (int64_t)pt * (OPC + pad);
   return (size_t)(o > y ? o : y);
 }
-__host__ __device__ inline size_t out_lds_bytes(int64_t Ch, size_t elem) {
+__host__ __device__ inline size_t out_lds_bytes(int64_t Ch, size_t elem, int pt = PTO) {
   const int pad = (int)(16 / elem);
-  return (out_region1_elems(Ch, pad) + (size_t)PTO * (Ch + pad)) * elem + (2 * (size_t)Ch + 8 * PTO + OPC) * 4;
+  return (out_region1_elems(Ch, pad, pt) + (size_t)pt * (Ch + pad)) * elem + (2 * (size_t)Ch + 8 * pt + OPC) * 4;
 }
 
 // Chunk i of a thread = 8 output channels (c8) of one pixel (px) of the pass's
 // [PTO][W] sub-block, W = 8 * W8 channels; consecutive threads take consecutive chunks.
-template <typename T>
-__device__ __forceinline__ void out_load_g(typename TypeOps<T>::V8 (&gr)[OCH], const T* __restrict__ gblk,
+template <typename T, int PT>
+__device__ __forceinline__ void out_load_g(typename TypeOps<T>::V8 (&gr)[out_chunks<PT>()], const T* __restrict__ gblk,
                                            int C, int c0, int W8, int npix, int tid) {
 #pragma unroll
-  for (int i = 0; i < OCH; ++i) {
+  for (int i = 0; i < out_chunks<PT>(); ++i) {
     const int idx = tid + i * NT, px = idx / W8, c8 = idx - px * W8;
     gr[i] = zero8<T>();
-    if (idx < PTO * W8 && px < npix) gr[i] = load8(gblk + (int64_t)px * C + c0 + 8 * c8);
+    if (idx < PT * W8 && px < npix) gr[i] = load8(gblk + (int64_t)px * C + c0 + 8 * c8);
   }
 }
 
-// CK / CHK: c_z / c_hidden fixed at compile time (0 = taken from the arguments), so the
+// PT: pixels of a tile. CK / CHK: c_z / c_hidden fixed at compile time (0 = taken from the arguments), so the
 // common 128 / 128 instantiation folds its loop bounds, chunk divisions and address strides.
-template <typename T, int PREC, int CK, int CHK>
+template <typename T, int PREC, int CK, int CHK, int PT = PTO>
 __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args a, int64_t NP,
                                                            size_t off_g, size_t off_o) {
   typedef typename TypeOps<T>::V8 V8;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int C = CK ? CK : (int)a.C, Ch = CHK ? CHK : (int)a.Ch, N = (int)a.N;
-  const int OR = PTO + lds_pad<T>();  // raw o tile [Ch][OR]
-  const int ZR = Ch + lds_pad<T>();   // normalised tile [PTO][ZR]
-  const int YR = OPC + lds_pad<T>();  // pass tile [PTO][YR]
+  const int OR = PT + lds_pad<T>();  // raw o tile [Ch][OR]
+  const int ZR = Ch + lds_pad<T>();   // normalised tile [PT][ZR]
+  const int YR = OPC + lds_pad<T>();  // pass tile [PT][YR]
   T* ot = reinterpret_cast<T*>(smem_raw);
   T* ys = ot;  // the o tile is dead once the LayerNorm has written zs
-  T* zs = ot + out_region1_elems(Ch, lds_pad<T>());
-  float* lnw = reinterpret_cast<float*>(zs + (size_t)PTO * ZR);
+  T* zs = ot + out_region1_elems(Ch, lds_pad<T>(), PT);
+  float* lnw = reinterpret_cast<float*>(zs + (size_t)PT * ZR);
   float* lnb = lnw + Ch;
-  float* red = lnb + Ch;        // LayerNorm partial sums [8 * PTO]
-  float* bpo_s = red + 8 * PTO;  // p_out bias of the current pass [OPC]
+  float* red = lnb + Ch;        // LayerNorm partial sums [8 * PT]
+  float* bpo_s = red + 8 * PT;  // p_out bias of the current pass [OPC]
 
-  const int ntile = (N + PTO - 1) / PTO;
+  const int ntile = (N + PT - 1) / PT;
   const int ct = blockIdx.x % ntile;
   const int p = (blockIdx.x / ntile) % N;
   const int b = blockIdx.x / (ntile * N);
-  const int q0 = ct * PTO;
-  const int npix = N - q0 < PTO ? N - q0 : PTO;
+  const int q0 = ct * PT;
+  const int npix = N - q0 < PT ? N - q0 : PT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, g = lane >> 5;
 
   const T* __restrict__ ocm = (const T*)((const unsigned char*)a.workspace + off_o);
@@ -1967,11 +1968,12 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
       (const T*)(a.gate ? (const unsigned char*)a.gate : (const unsigned char*)a.workspace + off_g) + blk;
   T* __restrict__ oblk = (T*)a.out + blk;
 
+  constexpr int OCH = out_chunks<PT>();
   V8 gr[OCH];
-  out_load_g<T>(gr, gblk, C, 0, (C < OPC ? C : OPC) / 8, npix, tid);
+  out_load_g<T, PT>(gr, gblk, C, 0, (C < OPC ? C : OPC) / 8, npix, tid);
   // p_out fragments of this wave's first 32-channel tile, first KPF k-steps, loaded now so
   // their latency overlaps the o tile load and the LayerNorm
-  constexpr int KPF = sizeof(T) == 2 ? 8 : 4;
+  constexpr int KPF = sizeof(T) == 2 || PT < PTO ? 8 : 4;
   const T* __restrict__ wpo = (const T*)a.p_out_w;
   const int nk = Ch / 16;
   V8 wpf[KPF];
@@ -1987,72 +1989,69 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
     lnb[c] = ld_or<T>(a.ln_out_b, c, 0.f);
   }
   for (int c = tid; c < (C < OPC ? C : OPC); c += NT) bpo_s[c] = ld_or<T>(a.p_out_b, c, 0.f);
-  for (int cb = 0; cb < Ch * (PTO / 8); cb += LDB * NT) {
+  for (int cb = 0; cb < Ch * (PT / 8); cb += LDB * NT) {
     V8 v[LDB];
 #pragma unroll
     for (int i = 0; i < LDB; ++i) {
-      const int c = cb + tid + i * NT, ch = c / (PTO / 8), k0 = (c % (PTO / 8)) * 8;
+      const int c = cb + tid + i * NT, ch = c / (PT / 8), k0 = (c % (PT / 8)) * 8;
       v[i] = zero8<T>();
-      if (c < Ch * (PTO / 8) && q0 + k0 < N) v[i] = load8(ocm + (((int64_t)b * Ch + ch) * N + p) * NP + q0 + k0);
+      if (c < Ch * (PT / 8) && q0 + k0 < N) v[i] = load8(ocm + (((int64_t)b * Ch + ch) * N + p) * NP + q0 + k0);
     }
 #pragma unroll
     for (int i = 0; i < LDB; ++i) {
-      const int c = cb + tid + i * NT, ch = c / (PTO / 8), k0 = (c % (PTO / 8)) * 8;
-      if (c < Ch * (PTO / 8)) store8(&ot[ch * OR + k0], v[i]);
+      const int c = cb + tid + i * NT, ch = c / (PT / 8), k0 = (c % (PT / 8)) * 8;
+      if (c < Ch * (PT / 8)) store8(&ot[ch * OR + k0], v[i]);
     }
   }
   __syncthreads();
 
-  // ---- LayerNorm over channels. Thread = (pixel pair pp = tid % 32, channel part
-  // tid / 32 of Ch / 8 channels): 32-bit LDS reads of two neighbouring pixels, the lanes of a
-  // wave covering 64 consecutive pixels of one channel row; the parts' partial sums meet in
+  // ---- LayerNorm over channels. Thread = (PX neighbouring pixels from PX (tid % 32)
+  // on, channel part tid / 32 of Ch / 8 channels): the lanes of a wave read the PT consecutive
+  // pixels of one channel row; the parts' partial sums meet in
   // LDS. Two passes (mean, then squared deviations), as F.layer_norm.
   {
     const int pp = tid & 31, part = tid >> 5;
     const int kc = Ch / 8, k0 = part * kc;
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    auto pair = [&](int k) -> f32x2 {
-      return __builtin_convertvector(*reinterpret_cast<const T2*>(&ot[k * OR + 2 * pp]), f32x2);
+    constexpr int PX = PT / 32;
+    typedef T TP __attribute__((ext_vector_type(PX)));
+    typedef float fP __attribute__((ext_vector_type(PX)));
+    auto pixels = [&](int k) -> fP {
+      return __builtin_convertvector(*reinterpret_cast<const TP*>(&ot[k * OR + PX * pp]), fP);
     };
-    float2* red2 = reinterpret_cast<float2*>(red);  // [8 parts][32 pairs]
-    f32x2 s2 = {0.f, 0.f};
-    for (int k = k0; k < k0 + kc; ++k) s2 += pair(k);
-    red2[part * 32 + pp] = make_float2(s2[0], s2[1]);
+    fP* redp = reinterpret_cast<fP*>(red);  // [8 parts][32]
+    fP s2 = (fP)0.f;
+    for (int k = k0; k < k0 + kc; ++k) s2 += pixels(k);
+    redp[part * 32 + pp] = s2;
     __syncthreads();
-    f32x2 mean = {0.f, 0.f};
+    fP mean = (fP)0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float2 v = red2[j * 32 + pp];
-      mean += f32x2{v.x, v.y};
-    }
+    for (int j = 0; j < 8; ++j) mean += redp[j * 32 + pp];
     const LnWidth lw(a.ln_out_channels, Ch);
     mean *= lw.inv_n;
-    f32x2 q2 = {0.f, 0.f};
+    fP q2 = (fP)0.f;
     for (int k = k0; k < k0 + kc; ++k) {
-      const f32x2 d = pair(k) - mean;
+      const fP d = pixels(k) - mean;
       q2 += d * d;
     }
     __syncthreads();  // every part has read the sums
-    red2[part * 32 + pp] = make_float2(q2[0], q2[1]);
+    redp[part * 32 + pp] = q2;
     __syncthreads();
-    f32x2 var = {0.f, 0.f};
+    fP var = (fP)0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float2 v = red2[j * 32 + pp];
-      var += f32x2{v.x, v.y};
-    }
-    const float rs0 = __builtin_amdgcn_rsqf(lw.var(var[0], mean[0]) + a.eps);  // as torch's rsqrt
-    const float rs1 = __builtin_amdgcn_rsqf(lw.var(var[1], mean[1]) + a.eps);
+    for (int j = 0; j < 8; ++j) var += redp[j * 32 + pp];
+    float rs[PX];
+#pragma unroll
+    for (int i = 0; i < PX; ++i) rs[i] = __builtin_amdgcn_rsqf(lw.var(var[i], mean[i]) + a.eps);  // as torch's rsqrt
     for (int k = k0; k < k0 + kc; k += 8) {
-      f32x8 v0, v1;
+      f32x8 v[PX];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const f32x2 x = pair(k + e);
-        v0[e] = (x[0] - mean[0]) * rs0 * lnw[k + e] + lnb[k + e];
-        v1[e] = (x[1] - mean[1]) * rs1 * lnw[k + e] + lnb[k + e];
+        const fP x = pixels(k + e);
+#pragma unroll
+        for (int i = 0; i < PX; ++i) v[i][e] = (x[i] - mean[i]) * rs[i] * lnw[k + e] + lnb[k + e];
       }
-      store8(&zs[(2 * pp) * ZR + k], TypeOps<T>::from_f32(v0));
-      store8(&zs[(2 * pp + 1) * ZR + k], TypeOps<T>::from_f32(v1));
+#pragma unroll
+      for (int i = 0; i < PX; ++i) store8(&zs[(PX * pp + i) * ZR + k], TypeOps<T>::from_f32(v[i]));
     }
   }
   __syncthreads();
@@ -2076,9 +2075,9 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
         for (int r = 0; r < 16; ++r) bpo[r] = ld_or<T>(a.p_out_b, cw + 4 * g + 8 * (r / 4) + (r % 4), 0.f);
       }
       const T* wrow = wpo + (int64_t)(cw + l32) * Ch + 8 * g;
-      f32x16 acc[PTO / 32];
+      f32x16 acc[PT / 32];
 #pragma unroll
-      for (int s = 0; s < PTO / 32; ++s)
+      for (int s = 0; s < PT / 32; ++s)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[s][r] = 0.f;
       if (c0 == 0) {
@@ -2086,7 +2085,7 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
         for (int k = 0; k < KPF; ++k) {
           if (k >= nk) break;
 #pragma unroll
-          for (int s = 0; s < PTO / 32; ++s) {
+          for (int s = 0; s < PT / 32; ++s) {
             const V8 zf = load8(&zs[(32 * s + l32) * ZR + 16 * k + 8 * g]);
             Mma<T, PREC>::step(acc[s], wpf[k], zf);
           }
@@ -2095,13 +2094,13 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
       for (int k = c0 == 0 ? KPF : 0; k < nk; ++k) {
         const V8 wf = load8(wrow + 16 * k);
 #pragma unroll
-        for (int s = 0; s < PTO / 32; ++s) {
+        for (int s = 0; s < PT / 32; ++s) {
           const V8 zf = load8(&zs[(32 * s + l32) * ZR + 16 * k + 8 * g]);
           Mma<T, PREC>::step(acc[s], wf, zf);
         }
       }
 #pragma unroll
-      for (int s = 0; s < PTO / 32; ++s)
+      for (int s = 0; s < PT / 32; ++s)
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
           f32x4 v;
@@ -2115,7 +2114,7 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
 #pragma unroll
     for (int i = 0; i < OCH; ++i) {
       const int idx = tid + i * NT, px = idx / W8, c8 = idx - px * W8;
-      if (idx < PTO * W8 && px < npix) {
+      if (idx < PT * W8 && px < npix) {
         const f32x8 y = TypeOps<T>::to_f32(load8(&ys[px * YR + 8 * c8]));
         store8(oblk + (int64_t)px * C + c0 + 8 * c8, TypeOps<T>::from_f32(y * TypeOps<T>::to_f32(gr[i])));
       }
@@ -2123,7 +2122,7 @@ __global__ __launch_bounds__(NT, 2) void trimul_out_kernel(const gnn_trimul_args
     if (c0 + OPC < C) {
       __syncthreads();  // the next pass rewrites ys
       const int Wn = C - c0 - OPC < OPC ? C - c0 - OPC : OPC;
-      out_load_g<T>(gr, gblk, C, c0 + OPC, Wn / 8, npix, tid);
+      out_load_g<T, PT>(gr, gblk, C, c0 + OPC, Wn / 8, npix, tid);
     }
   }
 }
@@ -2780,6 +2779,20 @@ int launch_out_w(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st
       if (psmem > 64 * 1024) (void)hipFuncSetAttribute(pf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)psmem);
       const int64_t grid = std::min<int64_t>(a.B * a.N * ntile, persistent_grid(pf, NT, psmem));
       hipLaunchKernelGGL((trimul_out_persist_kernel<T>), dim3((uint32_t)grid), dim3(NT), psmem, st, a, NP, L.off_g,
+                         L.off_o);
+      return (int)hipGetLastError();
+    }
+  }
+  // fp32 tiles too few for the CUs are halved: each is a serial chain of loads, LayerNorm, products
+  // and stores, so its length is the time. N = 64, c_z = c_hidden = 128: 11.5 -> 8.4 us
+  if constexpr (sizeof(T) == 4 && !(PREC == PREC_BF16X3 && CK == 128)) {
+    if (a.B * a.N * ntile < compute_units()) {
+      constexpr int PT = 32;
+      const size_t hsmem = out_lds_bytes(a.Ch, sizeof(T), PT);
+      const void* hf = (const void*)trimul_out_kernel<T, PREC, CK, CHK, PT>;
+      if (hsmem > 64 * 1024) (void)hipFuncSetAttribute(hf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)hsmem);
+      hipLaunchKernelGGL((trimul_out_kernel<T, PREC, CK, CHK, PT>),
+                         dim3((uint32_t)(a.B * a.N * ((a.N + PT - 1) / PT))), dim3(NT), hsmem, st, a, NP, L.off_g,
                          L.off_o);
       return (int)hipGetLastError();
     }

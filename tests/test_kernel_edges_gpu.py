@@ -104,6 +104,15 @@ def test_projection_dispatch(dtype, N, C, Ch, B, direction):
     assert _trimul_forward_error(N, C, Ch, dtype, direction, B) <= TOL[dtype]
 
 
+@pytest.mark.parametrize(("N", "C", "Ch", "B"), [(1, 128, 128, 1), (32, 128, 128, 1), (33, 128, 128, 3),
+                                                 (97, 32, 96, 1), (127, 128, 128, 1), (128, 128, 128, 1),
+                                                 (65, 256, 32, 1), (31, 160, 256, 2)])
+def test_fp32_output_tiles(N, C, Ch, B):
+    """Output tiles of 32 and 64 pixels (below and from 256 tiles of 64 on), their row tails, and more
+    output channels than one pass."""
+    assert _trimul_forward_error(N, C, Ch, torch.float32, "outgoing", B) <= TOL[torch.float32]
+
+
 # ------------------------------------------------------- products over rows, ordered sums
 @DTYPES
 @pytest.mark.parametrize(("M", "shapes"), [
