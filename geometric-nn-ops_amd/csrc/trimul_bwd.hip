@@ -349,10 +349,15 @@ int launch_gate(const gnn_gate_bwd_args& a, hipStream_t st) {
 // wave w owns the 32 stacked channels 32 w .. 32 w + 31 of p_in and g_in (2 Ch <= 256, their
 // weight fragments in registers for the whole launch) and recomputes p and g for the tile's two
 // 32-pixel halves on MFMA as [channel][pixel] blocks (A = the weights, B = z), so that a lane
-// holds one pixel and 4 consecutive channels per register group: d_ab is read and d_p / d_g
-// written 8 bytes at a time straight from the accumulators, each pixel row's 64 bytes per wave
+// holds one pixel and twice 8 consecutive channels (acc_channel): d_ab is read and d_p / d_g
+// written 16 bytes at a time straight from the accumulators, each pixel row's 64 bytes per wave
 // covered by its two lanes. The next tile's x is requested before the current tile's MFMAs.
 // The per-channel sums of the stored d_p / d_g stay in registers until the workgroup ends.
+// A 32x32 accumulator holds rows 8 (i / 4) + 4 g + i % 4. With MFMA row r carrying channel acc_channel(r) (the order of
+// the weight rows in the A fragments), lane group g holds channels 16 q + 8 g .. + 7 in elements 8 q .. 8 q + 7:
+// 16-byte accesses, the two lanes of a pixel covering 32 consecutive bytes, instead of twice as many of 8 bytes.
+// Input side 102 -> 86 us, output side 82 -> 81 us (N = 384, c_z = c_hidden = 128, bf16).
+__device__ __forceinline__ int acc_channel(int r) { return (r & 16) + ((r & 4) << 1) + ((r & 8) >> 1) + (r & 3); }
 constexpr int PB_W = 8;              // waves
 constexpr int PB_NT = 64 * PB_W;     // threads
 constexpr int PB_TP = 64;            // pixels per tile
@@ -400,11 +405,11 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
     bias[c] = a.p_in_b ? TypeOps<T>::to_f32(((const T*)a.p_in_b)[c]) : 0.f;
     bias[256 + c] = a.g_in_b ? TypeOps<T>::to_f32(((const T*)a.g_in_b)[c]) : 0.f;
   }
-  // this wave's channels: A fragments, row = channel 32 wave + l32, k = 16 kk + 8 g + e
+  // this wave's channels: A fragments, row = channel 32 wave + acc_channel(l32), k = 16 kk + 8 g + e
   const bool has_unit = ALLU || 32 * wave < Ch2;  // uniform over the wave
   V8 wpf[NK], wgf[NK];
   {
-    const int ch = has_unit ? 32 * wave + l32 : 0;
+    const int ch = has_unit ? 32 * wave + acc_channel(l32) : 0;
     const T* wprow = (const T*)a.p_in_w + (int64_t)ch * CK + 8 * g;
     const T* wgrow = (const T*)a.g_in_w + (int64_t)ch * CK + 8 * g;
 #pragma unroll
@@ -413,7 +418,7 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
       wgf[k] = load8(wgrow + 16 * k);
     }
   }
-  float sp[16], sg[16];  // sums of the stored d_p / d_g, channel 32 wave + 8 (i / 4) + 4 g + i % 4
+  float sp[16], sg[16];  // sums of the stored d_p / d_g, channel 32 wave + 16 (i / 8) + 8 g + i % 8
 #pragma unroll
   for (int i = 0; i < 16; ++i) sp[i] = sg[i] = 0.f;
 
@@ -487,16 +492,16 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
     if (tid < PB_TP) mk[tid] = TypeOps<T>::to_f32(mraw);
   };
 
-  // d_ab of a tile: this lane's pixel of each 32-pixel half, channels 32 wave + 8 rg + 4 g
-  // .. + 3; requested a tile ahead, with the next tile's x
-  V4 dac[PB_TP / 32][4], dan[PB_TP / 32][4];
-  auto load_d = [&](int64_t t, V4 (&d)[PB_TP / 32][4]) {
+  // d_ab of a tile: this lane's pixel of each 32-pixel half, channels 32 wave + 16 q + 8 g
+  // .. + 7; requested a tile ahead, with the next tile's x
+  V8 dac[PB_TP / 32][2], dan[PB_TP / 32][2];
+  auto load_d = [&](int64_t t, V8 (&d)[PB_TP / 32][2]) {
     if (!has_unit) return;
 #pragma unroll
     for (int s = 0; s < PB_TP / 32; ++s) {
       const int64_t rr = min(t * PB_TP + 32 * s + l32, rows - 1);
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) d[s][rg] = load4((const T*)a.d_ab + rr * a.dab_ld + 32 * wave + 8 * rg + 4 * g);
+      for (int q = 0; q < 2; ++q) d[s][q] = load8((const T*)a.d_ab + rr * a.dab_ld + 32 * wave + 16 * q + 8 * g);
     }
   };
 
@@ -506,7 +511,7 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
     for (int s = 0; s < PB_TP / 32; ++s) {
       const int64_t row = t * PB_TP + 32 * s + l32;
       const bool rok = row < rows;
-      const V4 (&da)[4] = dac[s];
+      const V8 (&da)[2] = dac[s];
       f32x16 accp, accg;
 #pragma unroll
       for (int i = 0; i < 16; ++i) accp[i] = accg[i] = 0.f;
@@ -518,23 +523,23 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
       }
       const float m = mk[32 * s + l32];
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int c0 = 32 * wave + 8 * rg + 4 * g;
-        const f32x4 bp = *reinterpret_cast<const f32x4*>(&bias[c0]);
-        const f32x4 bg = *reinterpret_cast<const f32x4*>(&bias[256 + c0]);
-        const f32x4 d = TypeOps<T>::to_f32(da[rg]);
-        f32x4 dp, dg;
+      for (int q = 0; q < 2; ++q) {
+        const int c0 = 32 * wave + 16 * q + 8 * g;
+        const f32x8 bp = *reinterpret_cast<const f32x8*>(&bias[c0]);
+        const f32x8 bg = *reinterpret_cast<const f32x8*>(&bias[256 + c0]);
+        const f32x8 d = TypeOps<T>::to_f32(da[q]);
+        f32x8 dp, dg;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < 8; ++e) {
           // p and g rounded to T, as the linear layers' outputs are
-          const float p = TypeOps<T>::to_f32(TypeOps<T>::from_f32(accp[4 * rg + e] + bp[e]));
-          const float gg = TypeOps<T>::to_f32(TypeOps<T>::from_f32(accg[4 * rg + e] + bg[e]));
+          const float p = TypeOps<T>::to_f32(TypeOps<T>::from_f32(accp[8 * q + e] + bp[e]));
+          const float gg = TypeOps<T>::to_f32(TypeOps<T>::from_f32(accg[8 * q + e] + bg[e]));
           const float sgm = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gg * -1.4426950408889634f));
           const float gm = d[e] * m;
           dp[e] = gm * sgm;
           dg[e] = gm * p * sgm * (1.0f - sgm);
         }
-        const V4 dpr = TypeOps<T>::from_f32(dp), dgr = TypeOps<T>::from_f32(dg);
+        const V8 dpr = TypeOps<T>::from_f32(dp), dgr = TypeOps<T>::from_f32(dg);
         if constexpr (ALLU) {
           // ranges from the tile's first row to the end of its last valid one (the row pitch
           // is at least 2 c_hidden), so the lanes of rows past the end fall outside them
@@ -547,14 +552,14 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
         }
         if (rok) {
           if constexpr (!ALLU) {
-            store4((T*)a.d_p + row * a.dl_ld + c0, dpr);
-            store4((T*)a.d_g + row * a.dl_ld + c0, dgr);
+            store8((T*)a.d_p + row * a.dl_ld + c0, dpr);
+            store8((T*)a.d_g + row * a.dl_ld + c0, dgr);
           }
-          const f32x4 dpf = TypeOps<T>::to_f32(dpr), dgf = TypeOps<T>::to_f32(dgr);
+          const f32x8 dpf = TypeOps<T>::to_f32(dpr), dgf = TypeOps<T>::to_f32(dgr);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sp[4 * rg + e] += dpf[e];
-            sg[4 * rg + e] += dgf[e];
+          for (int e = 0; e < 8; ++e) {
+            sp[8 * q + e] += dpf[e];
+            sg[8 * q + e] += dgf[e];
           }
         }
       }
@@ -582,7 +587,7 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
 #pragma unroll
       for (int s = 0; s < PB_TP / 32; ++s)
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) dac[s][rg] = dan[s][rg];
+        for (int q = 0; q < 2; ++q) dac[s][q] = dan[s][q];
       if (has_next) ln_partial();
       __syncthreads();  // z / mask of this tile consumed, partials of the next one published
       if (has_next) ln_finish(tn);
@@ -603,7 +608,7 @@ __global__ __launch_bounds__(PB_NT, 1) void trimul_proj_bwd_kernel(const gnn_tri
       float* prow = a.partial + (int64_t)blockIdx.x * 2 * Ch2;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int c = 32 * wave + 8 * (i / 4) + 4 * g + (i % 4);
+        const int c = 32 * wave + 16 * (i / 8) + 8 * g + (i % 8);
         prow[c] = sp[i];
         prow[Ch2 + c] = sg[i];
       }
@@ -628,10 +633,13 @@ int launch_proj_bwd(const gnn_trimul_proj_bwd_args& a, hipStream_t st) {
 // the channel-major o tile is staged in LDS and normalised per pixel (LN_out, two-pass fp32
 // statistics over a pair of pixels per thread, as the forward), on written once (for the
 // p_out weight gradient); y = on p_out_w^T + p_out_b on MFMA as [output channel][pixel]
-// blocks (wave: 32 output channels x 32 pixels), so that a lane holds one pixel and 4
-// consecutive channels: dout and the saved gate are read, and d_go / dy written, 8 bytes at a
-// time straight from the accumulators; dy is also staged in LDS for d(on) = dy p_out_w, again
-// [channel][pixel] blocks, whose per-pixel LayerNorm reductions meet in LDS. Weight fragments
+// blocks (wave: 32 output channels x 32 pixels), so that a lane holds one pixel and twice 8
+// consecutive channels (acc_channel): dout and the saved gate are read, and d_go written, 16
+// bytes at a time straight from the accumulators; dy is staged in LDS, for its rows and for
+// d(on) = dy p_out_w, again [channel][pixel] blocks, whose per-pixel LayerNorm reductions meet in
+// LDS; d(o) leaves through LDS in whole rows. One workgroup fits a CU (256 registers), so nothing
+// else hides a tile's loads: o travels a tile ahead in registers, and the LayerNorm takes all 512
+// threads. With both and the whole-row stores 108 -> 82 us. Weight fragments
 // stay in registers for the whole launch; the column sums of dy, d_go, d(on) x^ and d(on) stay
 // in registers until the workgroup ends.
 constexpr int OB_W = 8;
@@ -647,14 +655,14 @@ struct ObLds {
   static constexpr size_t ot = 0;
   static constexpr size_t zs = ot + (size_t)CHK * OR * sizeof(T);
   static constexpr size_t dys = zs + (size_t)OB_TP * ZR * sizeof(T);
-  static constexpr size_t red1 = dys + (size_t)OB_TP * DR * sizeof(T);  // [8 parts][32 pairs] f32x2 sums
-  static constexpr size_t red2 = red1 + 8 * 32 * 8;                      // ... squared deviations
-  static constexpr size_t red3 = red2 + 8 * 32 * 8;                      // [CHK / 32][OB_TP] LN-bwd sums
+  static constexpr size_t red2 = dys + (size_t)OB_TP * DR * sizeof(T);  // [16 parts][32 pairs] f32x2 squared deviations
+  static constexpr size_t red3 = red2 + 16 * 32 * 8;                     // [CHK / 32][OB_TP] LN-bwd sums
   static constexpr size_t stat = red3 + (size_t)(CHK / 32) * OB_TP * 8;  // [OB_TP] (mean, rstd)
   static constexpr size_t lnw = stat + OB_TP * 8;
   static constexpr size_t lnb = lnw + CHK * 4;
   static constexpr size_t bpo = lnb + CHK * 4;
-  static constexpr size_t fin = bpo + CK * 4;  // [2 halves][4][128] final column sums
+  static constexpr size_t red1 = bpo + CK * 4;  // [16][32] f32x2 sums
+  static constexpr size_t fin = red1;           // after the tiles: [2 halves][4][128] final column sums
   static constexpr size_t total = fin + 2 * 4 * 128 * 4;
 };
 
@@ -690,23 +698,42 @@ __global__ __launch_bounds__(OB_NT, 1) void trimul_out_bwd_kernel(const gnn_trim
   }
   for (int c = tid; c < CK; c += OB_NT) bpo[c] = a.p_out_b ? TypeOps<T>::to_f32(((const T*)a.p_out_b)[c]) : 0.f;
 
-  // y: wave = (unit uy, pixel half hy); A fragments row = output channel 32 uy + l32, k = 16 kk + 8 g + e
+  // y: wave = (unit uy, pixel half hy); A fragments row = output channel 32 uy + acc_channel(l32), k = 16 kk + 8 g + e
   const int uy = wave % NUY, hy = wave / NUY;
   const bool has_y = hy < 2;  // uniform over the wave
-  // d(on): wave = (unit ud, pixel half hd); A fragments row = channel 32 ud + l32, k = output channel
+  // d(on): wave = (unit ud, pixel half hd); A fragments row = channel 32 ud + acc_channel(l32), k = output channel
   const int ud = wave % NUD, hd = wave / NUD;
   const bool has_d = hd < 2;
   const T* wpo = (const T*)a.p_out_w;
   V8 wy[NKY], wd[NKD];
 #pragma unroll
-  for (int k = 0; k < NKY; ++k) wy[k] = load8(wpo + (int64_t)((has_y ? 32 * uy : 0) + l32) * CHK + 16 * k + 8 * g);
+  for (int k = 0; k < NKY; ++k) wy[k] = load8(wpo + (int64_t)((has_y ? 32 * uy : 0) + acc_channel(l32)) * CHK + 16 * k + 8 * g);
 #pragma unroll
   for (int k = 0; k < NKD; ++k)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) wd[k][e] = wpo[(int64_t)(16 * k + 8 * g + e) * CHK + (has_d ? 32 * ud : 0) + l32];
+    for (int e = 0; e < 8; ++e) wd[k][e] = wpo[(int64_t)(16 * k + 8 * g + e) * CHK + (has_d ? 32 * ud : 0) + acc_channel(l32)];
   float s_dy[16], s_dgo[16], s_dx[16], s_db[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) s_dy[i] = s_dgo[i] = s_dx[i] = s_db[i] = 0.f;
+
+  // The o tile [CHK][64] travels a tile ahead in registers. Every chunk is loaded, from inside the
+  // padded row; columns past N become zeros where the tile is written to LDS.
+  constexpr int NCH = CHK * (OB_TP / 8);                   // 16-byte chunks of a tile
+  constexpr int OCH = (NCH + OB_NT - 1) / OB_NT;           // per thread
+  V8 onext[OCH];
+  auto load_o = [&](int64_t t) {
+    const int j0 = (int)(t % ntj) * OB_TP;
+    const int64_t rest = t / ntj;
+    const int i = (int)(rest % N);
+    const int64_t b = rest / N;
+#pragma unroll
+    for (int k = 0; k < OCH; ++k) {
+      const int c = min(tid + k * OB_NT, NCH - 1);
+      const int ch = c / (OB_TP / 8), jj = (c % (OB_TP / 8)) * 8;
+      onext[k] = load8((const T*)a.o + ((b * CHK + ch) * N + i) * NP + min(j0 + jj, (int)NP - 8));
+    }
+  };
+  if (blockIdx.x < ntiles) load_o(blockIdx.x);
 
   for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int jt = (int)(t % ntj);
@@ -716,90 +743,86 @@ __global__ __launch_bounds__(OB_NT, 1) void trimul_out_bwd_kernel(const gnn_trim
     const int j0 = jt * OB_TP;
     const int64_t pb = (b * N + i) * N + j0;  // the tile's first pixel
 
-    // ---- 1. the o tile [CHK][64] (columns past N zero), and this lane's dout / gate
-    constexpr int OCH = CHK * (OB_TP / 8) / OB_NT;  // 16-byte chunks per thread (0 when CHK < 64)
+    // ---- 1. the o tile to LDS, and this lane's dout / gate
 #pragma unroll
-    for (int k = 0; k < (OCH > 0 ? OCH : 1); ++k) {
-      const int c = tid + k * OB_NT;
-      if (c < CHK * (OB_TP / 8)) {
-        const int ch = c / (OB_TP / 8), jj = (c % (OB_TP / 8)) * 8;
-        V8 v = zero8<T>();
-        if (j0 + jj < N) {
-          v = load8((const T*)a.o + ((b * CHK + ch) * N + i) * NP + j0 + jj);
+    for (int k = 0; k < OCH; ++k) {
+      const int c = tid + k * OB_NT, ch = c / (OB_TP / 8), jj = (c % (OB_TP / 8)) * 8;
+      V8 v = onext[k];
+      if (j0 + OB_TP > N) {  // uniform
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (j0 + jj + e >= N) v[e] = TypeOps<T>::from_f32(0.f);
-        }
-        store8(&ot[ch * OR + jj], v);
+        for (int e = 0; e < 8; ++e)
+          if (j0 + jj + e >= N) v[e] = TypeOps<T>::from_f32(0.f);
       }
+      if (NCH % OB_NT == 0 || c < NCH) store8(&ot[ch * OR + jj], v);
     }
     const int pxy = 32 * hy + l32;
     const bool vy = has_y && j0 + pxy < N;
     const int64_t piy = pb + (vy ? pxy : 0);  // rows past N read the tile's first pixel
-    V4 dout4[4], gate4[4];
+    V8 dout8[2], gate8[2];
     if (has_y) {
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int c0 = 32 * uy + 8 * rg + 4 * g;
-        dout4[rg] = load4((const T*)a.dout + piy * CK + c0);
-        gate4[rg] = load4((const T*)a.gate + piy * CK + c0);
+      for (int q = 0; q < 2; ++q) {
+        const int c0 = 32 * uy + 16 * q + 8 * g;
+        dout8[q] = load8((const T*)a.dout + piy * CK + c0);
+        gate8[q] = load8((const T*)a.gate + piy * CK + c0);
       }
     }
+    load_o(t + gridDim.x < ntiles ? t + gridDim.x : t);
     __syncthreads();
 
     // ---- 2. LN_out over the CHK channels of each pixel: thread = (pixel pair pp, part of
-    // CHK / 8 channels), threads 0 .. 255
+    // CHK / 16 channels)
     typedef T T2 __attribute__((ext_vector_type(2)));
-    const int pp = tid & 31, part = (tid >> 5) & 7;
-    constexpr int KC = CHK / 8;
+    const int pp = tid & 31, part = tid >> 5;
+    constexpr int KC = CHK / 16;
+    typedef T TK __attribute__((ext_vector_type(KC)));
     const int k0 = part * KC;
-    auto pair = [&](int k) -> f32x2 {
-      return __builtin_convertvector(*reinterpret_cast<const T2*>(&ot[k * OR + 2 * pp]), f32x2);
-    };
+    f32x2 xv[KC];
+    f32x2 s2 = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+      xv[k] = __builtin_convertvector(*reinterpret_cast<const T2*>(&ot[(k0 + k) * OR + 2 * pp]), f32x2);
+      s2 += xv[k];
+    }
+    red1[tid] = make_float2(s2[0], s2[1]);
+    __syncthreads();
     f32x2 mean = {0.f, 0.f};
-    if (tid < 256) {
-      f32x2 s2 = {0.f, 0.f};
 #pragma unroll
-      for (int k = k0; k < k0 + KC; ++k) s2 += pair(k);
-      red1[part * 32 + pp] = make_float2(s2[0], s2[1]);
+    for (int j = 0; j < 16; ++j) {
+      const float2 v = red1[j * 32 + pp];
+      mean += f32x2{v.x, v.y};
     }
-    __syncthreads();
-    f32x2 rs = {0.f, 0.f};
-    if (tid < 256) {
+    mean *= 1.0f / CHK;
+    f32x2 q2 = {0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float2 v = red1[j * 32 + pp];
-        mean += f32x2{v.x, v.y};
-      }
-      mean *= 1.0f / CHK;
-      f32x2 q2 = {0.f, 0.f};
-#pragma unroll
-      for (int k = k0; k < k0 + KC; ++k) {
-        const f32x2 d = pair(k) - mean;
-        q2 += d * d;
-      }
-      red2[part * 32 + pp] = make_float2(q2[0], q2[1]);
+    for (int k = 0; k < KC; ++k) {
+      xv[k] -= mean;
+      q2 += xv[k] * xv[k];
     }
+    red2[tid] = make_float2(q2[0], q2[1]);
     __syncthreads();
-    if (tid < 256) {
+    {
       f32x2 var = {0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < 16; ++j) {
         const float2 v = red2[j * 32 + pp];
         var += f32x2{v.x, v.y};
       }
+      f32x2 rs;
       rs[0] = 1.0f / sqrtf(var[0] * (1.0f / CHK) + a.eps);
       rs[1] = 1.0f / sqrtf(var[1] * (1.0f / CHK) + a.eps);
       if (part == 0) {
         stat[2 * pp] = make_float2(mean[0], rs[0]);
         stat[2 * pp + 1] = make_float2(mean[1], rs[1]);
       }
+      TK z0, z1;
 #pragma unroll
-      for (int k = k0; k < k0 + KC; ++k) {
-        const f32x2 x = pair(k);
-        zs[(2 * pp) * ZR + k] = TypeOps<T>::from_f32((x[0] - mean[0]) * rs[0] * lnw[k] + lnb[k]);
-        zs[(2 * pp + 1) * ZR + k] = TypeOps<T>::from_f32((x[1] - mean[1]) * rs[1] * lnw[k] + lnb[k]);
+      for (int k = 0; k < KC; ++k) {
+        z0[k] = TypeOps<T>::from_f32(xv[k][0] * rs[0] * lnw[k0 + k] + lnb[k0 + k]);
+        z1[k] = TypeOps<T>::from_f32(xv[k][1] * rs[1] * lnw[k0 + k] + lnb[k0 + k]);
       }
+      *reinterpret_cast<TK*>(&zs[(2 * pp) * ZR + k0]) = z0;
+      *reinterpret_cast<TK*>(&zs[(2 * pp + 1) * ZR + k0]) = z1;
     }
     __syncthreads();
     // on to its pixel-major rows (16-byte chunks)
@@ -817,37 +840,41 @@ __global__ __launch_bounds__(OB_NT, 1) void trimul_out_bwd_kernel(const gnn_trim
       for (int k = 0; k < NKY; ++k)
         Mma<T, PREC_NATIVE>::step(acc, wy[k], load8(&zs[pxy * ZR + 16 * k + 8 * g]));
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int c0 = 32 * uy + 8 * rg + 4 * g;
-        const f32x4 b4 = *reinterpret_cast<const f32x4*>(&bpo[c0]);
-        const f32x4 d4 = TypeOps<T>::to_f32(dout4[rg]), s4 = TypeOps<T>::to_f32(gate4[rg]);
-        f32x4 dy, dg;
+      for (int q = 0; q < 2; ++q) {
+        const int c0 = 32 * uy + 16 * q + 8 * g;
+        const f32x8 b8 = *reinterpret_cast<const f32x8*>(&bpo[c0]);
+        const f32x8 d8 = TypeOps<T>::to_f32(dout8[q]), s8 = TypeOps<T>::to_f32(gate8[q]);
+        f32x8 dy, dg;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float y = TypeOps<T>::to_f32(TypeOps<T>::from_f32(acc[4 * rg + e] + b4[e]));
-          dy[e] = d4[e] * s4[e];
-          dg[e] = d4[e] * y * s4[e] * (1.0f - s4[e]);
+        for (int e = 0; e < 8; ++e) {
+          const float y = TypeOps<T>::to_f32(TypeOps<T>::from_f32(acc[8 * q + e] + b8[e]));
+          dy[e] = d8[e] * s8[e];
+          dg[e] = d8[e] * y * s8[e] * (1.0f - s8[e]);
         }
-        const V4 dyr = TypeOps<T>::from_f32(dy), dgr = TypeOps<T>::from_f32(dg);
-        store4(&dys[pxy * DR + c0], dyr);
+        const V8 dyr = TypeOps<T>::from_f32(dy), dgr = TypeOps<T>::from_f32(dg);
+        store8(&dys[pxy * DR + c0], dyr);
         if (vy) {
-          store4((T*)a.dy + piy * CK + c0, dyr);
-          store4((T*)a.d_go + piy * a.dgo_ld + c0, dgr);
-          const f32x4 dyf = TypeOps<T>::to_f32(dyr), dgf = TypeOps<T>::to_f32(dgr);
+          store8((T*)a.d_go + piy * a.dgo_ld + c0, dgr);
+          const f32x8 dyf = TypeOps<T>::to_f32(dyr), dgf = TypeOps<T>::to_f32(dgr);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            s_dy[4 * rg + e] += dyf[e];
-            s_dgo[4 * rg + e] += dgf[e];
+          for (int e = 0; e < 8; ++e) {
+            s_dy[8 * q + e] += dyf[e];
+            s_dgo[8 * q + e] += dgf[e];
           }
         }
       }
     }
     __syncthreads();
+    // dy to its pixel-major rows
+    for (int c = tid; c < OB_TP * (CK / 8); c += OB_NT) {
+      const int px = c / (CK / 8), k = (c % (CK / 8)) * 8;
+      if (j0 + px < N) store8((T*)a.dy + (pb + px) * CK + k, load8(&dys[px * DR + k]));
+    }
 
     // ---- 4. d(on) = dy p_out_w and the LN_out backward
     const int pxd = 32 * hd + l32;
     const bool vd = has_d && j0 + pxd < N;
-    f32x4 donv[4];  // d(on) rounded as the linear's output; x^ is read again after the barrier
+    f32x8 donv[2];  // d(on) rounded as the linear's output; x^ is read again after the barrier
     float2 st = make_float2(0.f, 1.f);
     if (has_d) {
       f32x16 acc;
@@ -859,20 +886,20 @@ __global__ __launch_bounds__(OB_NT, 1) void trimul_out_bwd_kernel(const gnn_trim
       st = stat[pxd];
       float sg = 0.f, sgx = 0.f;
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int c0 = 32 * ud + 8 * rg + 4 * g;
-        const f32x4 w4 = *reinterpret_cast<const f32x4*>(&lnw[c0]);
+      for (int q = 0; q < 2; ++q) {
+        const int c0 = 32 * ud + 16 * q + 8 * g;
+        const f32x8 w8 = *reinterpret_cast<const f32x8*>(&lnw[c0]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float don = TypeOps<T>::to_f32(TypeOps<T>::from_f32(acc[4 * rg + e]));
+        for (int e = 0; e < 8; ++e) {
+          const float don = TypeOps<T>::to_f32(TypeOps<T>::from_f32(acc[8 * q + e]));
           const float x = (TypeOps<T>::to_f32(ot[(c0 + e) * OR + pxd]) - st.x) * st.y;
-          donv[rg][e] = don;
-          const float gc = don * w4[e];
+          donv[q][e] = don;
+          const float gc = don * w8[e];
           sg += gc;
           sgx += gc * x;
           if (vd) {
-            s_dx[4 * rg + e] += don * x;
-            s_db[4 * rg + e] += don;
+            s_dx[8 * q + e] += don * x;
+            s_db[8 * q + e] += don;
           }
         }
       }
@@ -892,22 +919,24 @@ __global__ __launch_bounds__(OB_NT, 1) void trimul_out_bwd_kernel(const gnn_trim
       }
       mg *= 1.0f / CHK;
       mgx *= 1.0f / CHK;
-      if (vd) {
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          const int c0 = 32 * ud + 8 * rg + 4 * g;
-          const f32x4 w4 = *reinterpret_cast<const f32x4*>(&lnw[c0]);
-          f32x4 dx;
+      for (int q = 0; q < 2; ++q) {
+        const int c0 = 32 * ud + 16 * q + 8 * g;
+        const f32x8 w8 = *reinterpret_cast<const f32x8*>(&lnw[c0]);
+        f32x8 dx;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float x = (TypeOps<T>::to_f32(ot[(c0 + e) * OR + pxd]) - st.x) * st.y;
-            dx[e] = st.y * (donv[rg][e] * w4[e] - mg - x * mgx);
-          }
-          store4((T*)a.d_o + (pb + pxd) * CHK + c0, TypeOps<T>::from_f32(dx));
+        for (int e = 0; e < 8; ++e) {
+          const float x = (TypeOps<T>::to_f32(ot[(c0 + e) * OR + pxd]) - st.x) * st.y;
+          dx[e] = st.y * (donv[q][e] * w8[e] - mg - x * mgx);
         }
+        store8(&zs[pxd * ZR + c0], TypeOps<T>::from_f32(dx));
       }
     }
-    __syncthreads();  // ot / zs / dys / red3 free for the next tile
+    __syncthreads();  // ot / dys / red3 free for the next tile, which writes zs two barriers on
+    for (int c = tid; c < OB_TP * (CHK / 8); c += OB_NT) {
+      const int px = c / (CHK / 8), k = (c % (CHK / 8)) * 8;
+      if (j0 + px < N) store8((T*)a.d_o + (pb + px) * CHK + k, load8(&zs[px * ZR + k]));
+    }
   }
 
   // ---- the workgroup's column sums: over the 32 pixels of a lane group, then the two halves
@@ -926,7 +955,7 @@ __global__ __launch_bounds__(OB_NT, 1) void trimul_out_bwd_kernel(const gnn_trim
   if (l32 == 0) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int cc = 8 * (i / 4) + 4 * g + (i % 4);
+      const int cc = 16 * (i / 8) + 8 * g + (i % 8);
       if (has_y) {
         fin[(hy * 4 + 0) * 128 + 32 * uy + cc] = s_dy[i];
         fin[(hy * 4 + 1) * 128 + 32 * uy + cc] = s_dgo[i];
@@ -985,7 +1014,9 @@ int trimul_proj_bwd(const gnn_trimul_proj_bwd_args& a, hipStream_t st) {
 
 int64_t trimul_out_bwd_partials(int64_t B, int64_t N) {
   const int64_t t = B * N * ((N + OB_TP - 1) / OB_TP);
-  return t < 1 ? 1 : (t > OB_MAX_GRID ? OB_MAX_GRID : t);
+  // one workgroup fits a CU: up to 8 tiles for each of 512, a single round of 256
+  const int64_t cap = t < 8 * OB_MAX_GRID ? OB_MAX_GRID / 2 : OB_MAX_GRID;
+  return t < 1 ? 1 : (t > cap ? cap : t);
 }
 
 int trimul_out_bwd(const gnn_trimul_out_bwd_args& a, hipStream_t st) {
