@@ -999,7 +999,9 @@ int64_t gate_bwd_partials(int64_t rows, int64_t K) {
 
 int64_t trimul_proj_bwd_partials(int64_t rows) {
   const int64_t t = (rows + PB_TP - 1) / PB_TP;
-  return t < 1 ? 1 : (t > PB_MAX_GRID ? PB_MAX_GRID : t);
+  // one workgroup fits a CU, as in trimul_out_bwd_partials
+  const int64_t cap = t < 8 * PB_MAX_GRID ? PB_MAX_GRID / 2 : PB_MAX_GRID;
+  return t < 1 ? 1 : (t > cap ? cap : t);
 }
 
 int trimul_proj_bwd(const gnn_trimul_proj_bwd_args& a, hipStream_t st) {
