@@ -312,12 +312,12 @@ def trimul_wide_hip(x, direction, mask, eps, weights):
 # triangle/_reference/trimul.py:57-97). trimul_bwd_hip differentiates the same math. The
 # LayerNorms (forward recompute and backward, with deterministic per-workgroup weight-gradient
 # partials) and the two sigmoid gates run on this library's kernels (gnn_layernorm_rows,
-# gnn_trimul_gate_bwd), and for 16-bit types so do the contraction's two N^3 products per
-# channel (gnn_trimul_contract_bwd, reading a and b in place in the forward's workspace) and
-# the moves between pixel-major tensors and per-channel planes (gnn_trimul_relayout). The
-# other matrix products (the three input projections as one [4 Ch + C, C] linear, p_out, and
-# fp32's contraction products) go to the vendor GEMM through torch; the weight gradients run on
-# gnn_rows_product, and gnn_reduce_parts adds every parameter's partial sums in one launch.
+# gnn_trimul_gate_bwd), as do the contraction's two N^3 products per channel, on the forward's
+# a and b in place (gnn_trimul_contract_bwd; fp32: gnn_rows_product), the moves between
+# pixel-major tensors and per-channel planes (gnn_trimul_relayout, gnn_relayout_f32) and the
+# weight gradients (gnn_rows_product); gnn_reduce_parts adds every parameter's partial sums in
+# one launch. The remaining matrix products (the three input projections as one [4 Ch + C, C]
+# linear, p_out, and dz) go to the vendor GEMM through torch.
 # a, b and o come from the forward's workspace.
 
 def layernorm_rows_hip(x2d, weight=None, bias=None, eps=1e-5, *, dy=None, partials=False, raw=False):
