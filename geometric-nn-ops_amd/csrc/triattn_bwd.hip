@@ -31,9 +31,9 @@
 // (triangle_attention.py:753-766, :1033-1038): in a row whose keys are all masked the
 // forward's lse holds the bare sentinel (its log(l) term is below the fp32 ulp there), so
 // exp(S - lse) is 1 for every key where softmax gives 1 / N_res; in any other row a masked
-// key's P is 0 either way. dq and dk / dv divide per masked key; bwd_dbias, which sees a
-// row's keys one tile at a time, per row (its lse at the sentinel): -log2(N_res) joins the
-// exp2 argument.
+// key's P is 0 either way. In bwd_dbias -log2(N_res) joins the exp2 argument of a masked key; its
+// DMA form, which goes with the row-resident dq / dk / dv kernels, divides as they do
+// (lost_lse_bound).
 // 16-bit inputs, head dim <= 128 (a multiple of 8, ensured by the host). Every kernel is
 // templated on DC, the number of 32-column chunks of the head dim (1, 2 or 4): the staged
 // tiles are DC swizzled [rows][32] tiles, the score and dP products sum over the chunks, and
@@ -541,7 +541,6 @@ struct DbLds {  // beyond 64 KB (16-bit DC > 1, fp32): dynamic LDS
   float lse[DB_T];
   float delta[DB_T];
   float kb[DB_T];
-  float pl2;  // -log2(N_res) when the row's keys are all masked, else 0
 };
 
 template <typename T, int DC, int PREC>
@@ -634,12 +633,11 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_kernel(const gnn_triattn_b
       sm.lse[sr] = plse[set];
       sm.delta[sr] = pdel[set];
       sm.kb[sr] = k0 + sr >= N ? -INFINITY : pmk[set] == 0 ? a.mask_value : 0.f;
-      // every query of the row shares its keys' mask: the tile's first query (< N) decides
-      if (sr == 0) sm.pl2 = (a.mask && plse[set] <= 0.5f * a.mask_value) ? -__log2f((float)N) : 0.f;
     }
   };
   // one N_seq row of the tile from LDS: sum_s dS += P (dP - Delta)
   const bool has_tile = q0 + qw < N && k0 + kw < N;  // uniform over the wave
+  const float nlog2 = -__log2f((float)N);
   auto compute_row = [&]() {
     // dO fragments negated and the dP accumulator started at Delta: the MFMA yields Delta - dP
     V8 qf[DC][2], ndof[DC][2];
@@ -670,13 +668,13 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_kernel(const gnn_triattn_b
           Mma<T, PREC>::step(scv, qf[dc][kk], lds_row8<T>(sm.k[dc], kr, 2 * kk + g));
           Mma<T, PREC>::step(ndp, ndof[dc][kk], lds_row8<T>(sm.v[dc], kr, 2 * kk + g));
         }
-      const float kb = sm.kb[kr], pl2 = sm.pl2;
+      const float kb = sm.kb[kr], kpl2 = kb != 0.f ? nlog2 : 0.f;  // masked (elements past N are not stored)
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int i = 4 * rg + e;
-          const float pv = fast_exp2(__builtin_fmaf(scv[i] + kb - l4[rg][e], LOG2E_B, pl2));
+          const float pv = fast_exp2(__builtin_fmaf(scv[i] + kb - l4[rg][e], LOG2E_B, kpl2));
           acc[sub][i] -= pv * ndp[i];
         }
     }
@@ -821,7 +819,7 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_dma_kernel(const gnn_triat
 
   const float scale = a.scale;
   constexpr bool has_mask = MASK;
-  const float pl2_masked = -__log2f((float)N);
+  const float nlog2 = -__log2f((float)N), qbound = lost_lse_bound(a.mask, a.mask_value);
   auto compute_row = [&](int stage, int mrow) {
     const DbdStage& st = sm.st[stage];
     // dO fragments negated (a sign flip, exact) and the dP accumulator started at Delta: the
@@ -843,8 +841,7 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_dma_kernel(const gnn_triat
 #pragma unroll
       for (int e = 0; e < 4; ++e) dinit[4 * rg + e] = d4[e];
     }
-    // every query of the row shares its keys' mask: the tile's first query decides
-    const float pl2 = (has_mask && st.lse[0] <= 0.5f * a.mask_value) ? pl2_masked : 0.f;
+    const bool lost = has_mask && __any(st.lse[qw + l32] <= qbound);
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int kr = kw + 32 * sub + l32;
@@ -854,17 +851,23 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_dma_kernel(const gnn_triat
         Mma<T, PREC_NATIVE>::step(scv, qf[kk], lds_row8<T>(st.k, kr, 2 * kk + g));
         Mma<T, PREC_NATIVE>::step(ndp, ndof[kk], lds_row8<T>(st.v, kr, 2 * kk + g));
       }
-      const float kb = (has_mask && sm.mask[mrow][kr] == 0) ? a.mask_value : 0.f;
+      const bool masked = has_mask && sm.mask[mrow][kr] == 0;
+      const float kb = masked ? a.mask_value : 0.f, kpl2 = masked ? nlog2 : 0.f;
+      // the logit minus lse first (in a fully masked row both sit near the sentinel)
+      auto p = [&](int i, float lse, float pl2) {
+        const float x = has_mask ? scv[i] + kb - lse : scv[i] - lse;
+        return fast_exp2(has_mask ? __builtin_fmaf(x, LOG2E_B, pl2) : x * LOG2E_B);
+      };
+      if (lost) {  // uniform
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = 4 * rg + e;
-          // the logit minus lse first (in a fully masked row both sit near the sentinel)
-          const float x = has_mask ? scv[i] + kb - l4[rg][e] : scv[i] - l4[rg][e];
-          const float pv = fast_exp2(has_mask ? __builtin_fmaf(x, LOG2E_B, pl2) : x * LOG2E_B);
-          acc[sub][i] -= pv * ndp[i];
+        for (int i = 0; i < 16; ++i) {
+          const float lse = l4[i / 4][i % 4];
+          acc[sub][i] -= p(i, lse, lse <= qbound ? nlog2 : kpl2) * ndp[i];
         }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[sub][i] -= p(i, l4[i / 4][i % 4], kpl2) * ndp[i];
+      }
     }
   };
 

@@ -24,8 +24,8 @@
 // The pair-bias fragments of the next step are requested from global memory (L2: a bias
 // plane is shared by every N_seq row) while the current one is computed. The reference's
 // correction for rows whose keys are all masked (P of a masked key divided by N_res, which
-// only changes such rows: elsewhere a masked key's P is exactly 0) is applied per row, as
-// P = exp2((S - lse) log2(e) - log2(N_res)) where the row's lse sits at the mask sentinel.
+// only changes such rows: elsewhere a masked key's P is exactly 0) joins the exponent, as
+// P = exp2((S - lse) log2(e) - log2(N_res)) (see lost_lse_bound).
 #include <type_traits>
 
 #include "gnn_common.hpp"
@@ -125,18 +125,17 @@ __device__ __forceinline__ void row_coords(uint32_t w, int S, int H, int& b, int
   b = (int)(w / ((uint32_t)S * H));
 }
 
-// -log2(N_res) for a row whose keys are all masked (its lse then holds the bare mask
-// sentinel: log(l) is below the fp32 ulp there), else 0; added to the exp2 argument it
-// divides P by N_res. A live row's lse is the logsumexp of real logits, far above half the
-// sentinel.
-__device__ __forceinline__ float dead_row_log2(const gnn_triattn_bwd_args& a, float lse) {
-  return (a.mask && lse <= 0.5f * a.mask_value) ? -__log2f((float)a.N) : 0.f;
+// Whether a query's lse lies where the mask sentinel puts it: its keys are all masked, or the pair
+// bias alone holds the query down there. Its exponents then subtract lse from the logit first.
+__device__ __forceinline__ bool at_sentinel(const gnn_triattn_bwd_args& a, float lse) {
+  return a.mask && lse <= 0.5f * a.mask_value;
 }
 
 // ------------------------------------------------------------------------------- dQ
 struct DqRowHdr {
   float kterm[BWD_ROW_MAX_N];  // added to the scores of key j: 0, the mask sentinel, or -inf past N
   int plain[RMAX_TILES];       // tile t has no masked key and no key past N
+  int dead;                    // no live key
 };
 constexpr int DQ_HDR = (int)((sizeof(DqRowHdr) + 255) / 256 * 256);
 
@@ -159,6 +158,7 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
   stage_rows_dma<T>(ks, kp, a.k_stride[2], N, ntiles, wave, lane);
   stage_rows_dma<T>(vs, vp, a.v_stride[2], N, ntiles, wave, lane);
   if (wave == 0) {
+    bool live = false;
     for (int t = 0; t < ntiles; ++t) {
       const int key = t * RT + lane;
       float kt = 0.f;
@@ -169,7 +169,9 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
       hdr.kterm[key] = kt;
       const bool plain = __ballot(kt != 0.f) == 0;
       if (lane == 0) hdr.plain[t] = plain;
+      live |= __ballot(kt == 0.f) != 0;
     }
+    if (lane == 0) hdr.dead = !live;
   }
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this wave's LDS DMA has landed
   __syncthreads();
@@ -209,11 +211,11 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
       if (qok && g == 0) a.delta[lrow + qi] = delta;
     }
     const float lse = qok ? a.lse[lrow + qi] : INFINITY;  // absent queries: p = 0
-    const float pl2 = dead_row_log2(a, lse);
-    // Unless a query of the wave sits in a fully masked row, P = exp2(S log2 e - lse log2 e)
+    // Unless a query of the wave sits at the sentinel, P = exp2(S log2 e - lse log2 e)
     // takes one fma per element (lse is this lane's query's, constant along the accumulator);
-    // a fully masked row keeps S - lse formed first (both sit near the sentinel).
-    const bool dead = __any(pl2 != 0.f);
+    // there S - lse is formed first.
+    const bool first = hdr.dead || __any(at_sentinel(a, lse));
+    const float pl2 = hdr.dead || lse <= lost_lse_bound(a.mask, a.mask_value) ? -__log2f((float)N) : 0.f;
     const float nl2 = -lse * LOG2E_R;
     const T* brow = HAS_BIAS ? (const T*)a.bias + b * a.bias_stride[0] + h * a.bias_stride[1] +
                                    (int64_t)(qok ? qi : 0) * a.bias_stride[2]
@@ -252,10 +254,10 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
       // P = exp(S - lse), subtracting first: in a row whose keys are all masked both sit
       // near the sentinel, and only their difference is exact
       f32x16 ds;
-      if (plain && !dead) {
+      if (plain && !first) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) ds[i] = fast_exp2(__builtin_fmaf(sc[i], LOG2E_R, nl2)) * (dp[i] - delta);
-      } else if (!dead) {
+      } else if (!first) {
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
           const f32x4 k4 = *reinterpret_cast<const f32x4*>(&hdr.kterm[32 * st + 8 * rg + 4 * g]);
@@ -295,6 +297,7 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
 struct DkdvRowHdr {
   float lse[BWD_ROW_MAX_N];    // +inf for absent queries (p = 0)
   float ndelta[BWD_ROW_MAX_N];  // -Delta (0 for absent queries): the dP accumulators' start
+  int row[RW];                  // per wave, of what it staged: 1 a live key, 2 a query past lost_lse_bound
 };
 constexpr int DKDV_HDR = (int)((sizeof(DkdvRowHdr) + 255) / 256 * 256);
 
@@ -339,17 +342,37 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dkdv_row_kernel(const gnn_triattn_
       }
     }
     const int64_t lrow = (((int64_t)b * S + s) * H + h) * N;
+    bool live = false, lost = false;
     for (int r = tid; r < nrows; r += RNT) {
-      hdr.lse[r] = r < N ? a.lse[lrow + r] : INFINITY;
+      const float l = r < N ? a.lse[lrow + r] : INFINITY;
+      hdr.lse[r] = l;
       hdr.ndelta[r] = r < N ? -a.delta[lrow + r] : 0.f;
+      live |= r < N && (!a.mask || a.mask[b * a.mask_stride[0] + s * a.mask_stride[1] + r * a.mask_stride[2]] != 0);
+      lost |= l <= lost_lse_bound(a.mask, a.mask_value);
     }
+    const int row = (__any(live) ? 1 : 0) | (__any(lost) ? 2 : 0);
+    if (lane == 0) hdr.row[wave] = row;
   }
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this wave's LDS DMA has landed
   __syncthreads();
 
   V8 idf[2];
   ridentity<T>(idf, l32, g);
-  const float pl2 = dead_row_log2(a, hdr.lse[0]);  // query 0 exists (N >= 1)
+  // both uniform over the workgroup. A row whose keys are all masked divides P by N_res in the exponent
+  const bool dead = !__any(hdr.row[lane & (RW - 1)] & 1), lost = __any(hdr.row[lane & (RW - 1)] & 2);
+  const float pl2 = dead ? -__log2f((float)N) : 0.f;
+  if (lost && !dead) {  // a live row's queries past the bound: with dO and Delta divided, P^T dO and dS are
+    const float inv_n = 1.0f / (float)N;
+    for (int r = tid; r < N; r += RNT) {
+      if (hdr.lse[r] > lost_lse_bound(a.mask, a.mask_value)) continue;
+      hdr.ndelta[r] *= inv_n;
+      for (int c = 0; c < 4; ++c) {
+        V8* x = reinterpret_cast<V8*>(ds_ + rswz(r, c));
+        *x = TypeOps<T>::from_f32(TypeOps<T>::to_f32(*x) * inv_n);
+      }
+    }
+    __syncthreads();
+  }
   const T* bias_plane = HAS_BIAS ? (const T*)a.bias + b * a.bias_stride[0] + h * a.bias_stride[1] : nullptr;
   const int nkb = (N + 31) / 32;
   const int nsub = 2 * ntiles;  // 32-query steps
@@ -486,7 +509,7 @@ __host__ __device__ inline int fused_waves(int N) {
   return (nb + kb - 1) / kb;
 }
 // LDS of a 32-query block: Q' and dO images, dQ in accumulator layout ([4][64 lanes] f32x4), then
-// -lse log2(e) (lse itself in a row whose keys are all masked; queries past N: p = 0) and -Delta
+// -lse log2(e) (lse itself where the row subtracts first; queries past N: p = 0) and -Delta
 struct FusedBlock {
   unsigned char q[32 * RROW];
   unsigned char d[32 * RROW];
@@ -494,7 +517,11 @@ struct FusedBlock {
   float nl[32];
   float ndelta[32];
 };
-inline size_t fused_lds(int N) { return (size_t)((N + 31) / 32) * sizeof(FusedBlock) + fused_waves(N) * 2048; }
+// then a 2 KB tile and a word of row flags for each wave
+constexpr int FUSED_FLAGS = 64;
+inline size_t fused_lds(int N) {
+  return (size_t)((N + 31) / 32) * sizeof(FusedBlock) + fused_waves(N) * 2048 + FUSED_FLAGS;
+}
 
 // A 32 x 32 16-bit tile through LDS: write4 stores a lane's 16 values (row = lane % 32, columns
 // 8 rg + 4 g .. + 3 in words 2 rg, 2 rg + 1) and read_tr reads both k-steps' transposed fragments,
@@ -541,15 +568,15 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned char* tile = smem_raw + nb * sizeof(FusedBlock) + wave * 2048;  // this wave's dS tile [key][query]
   const int64_t lrow = (((int64_t)b * S + s) * H + h) * N;
-  const float pl2 = dead_row_log2(a, a.lse[lrow]);  // query 0 exists (N >= 1)
-  const bool dead = pl2 != 0.f;                     // every query shares the row's keys
+  // per wave, of its keys and the queries that it stages: 1 a live key, 2 a query at the sentinel
+  int* flags = reinterpret_cast<int*>(smem_raw + nb * sizeof(FusedBlock) + nth / 64 * 2048);
 
   // ---- this wave's keys: K and V as B operands (lane = key, 8 consecutive d), and the key-side
   // mask term (-inf for keys past N: p = 0)
   const int kb0 = KB * wave;
   V8 kf[KB][2], vf[KB][2];
   float kbias[KB];
-  bool masked = false;
+  bool masked = false, live = false, first = false;
 #pragma unroll
   for (int u = 0; u < KB; ++u) {
     const int key = 32 * (kb0 + u) + l32;
@@ -569,9 +596,8 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
     else if (a.mask && a.mask[b * a.mask_stride[0] + s * a.mask_stride[1] + (int64_t)key * a.mask_stride[2]] == 0)
       kbias[u] = a.mask_value;
     masked |= kbias[u] != 0.f;
-    if (!dead) kbias[u] *= LOG2E_R;  // joins the exponent there, the logit in a fully masked row
+    live |= kbias[u] == 0.f;
   }
-  const int mode = dead ? 2 : __any(masked) ? 1 : 0;  // uniform over the wave
 
   // ---- stage Q' and dO (rows past N are zero), form Delta, clear dQ
   {
@@ -610,9 +636,12 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
       }
     }
     for (int r = tid; r < nrows; r += nth) {
-      const float l = a.lse[lrow + (r < N ? r : 0)];
-      blk[r >> 5].nl[r & 31] = dead ? (r < N ? l : INFINITY) : (r < N ? -l * LOG2E_R : -INFINITY);
+      const float l = r < N ? a.lse[lrow + r] : INFINITY;
+      blk[r >> 5].nl[r & 31] = l;
+      first |= at_sentinel(a, l);
     }
+    const int f = (__any(live) ? 1 : 0) | (__any(first) ? 2 : 0);
+    if (lane == 0) flags[wave] = f;
     for (int c = tid; c < nb * 256; c += nth) blk[c >> 8].dq[c & 255] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // per-lane byte offsets inside a block's images and the tile: row fragments (row l32, chunks
@@ -676,9 +705,23 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
 #pragma unroll
     for (int i = 0; i < 16; ++i) dk[u][i] = dv[u][i] = 0.f;
   __syncthreads();
+  // What the row's waves found together. Unless it subtracts first, lse and the key-side term join
+  // the exponent in units of log2.
+  const int found = flags[lane % (nth / 64)];
+  const bool dead = !__any(found & 1);
+  first = dead || __any(found & 2);
+  const float nlog2 = -__log2f((float)N), qbound = lost_lse_bound(a.mask, a.mask_value);
+  const float pl2 = dead ? nlog2 : 0.f;
+  if (!first) {
+    for (int r = tid; r < nrows; r += nth) blk[r >> 5].nl[r & 31] *= -LOG2E_R;
+#pragma unroll
+    for (int u = 0; u < KB; ++u) kbias[u] *= LOG2E_R;
+    __syncthreads();
+  }
+  const int mode = first ? 2 : __any(masked) ? 1 : 0;  // uniform over the wave
 
   // MODE 0: no masked key in the wave's blocks and none past N. 1: the key-side term joins the
-  // exponent. 2: a row whose keys are all masked.
+  // exponent. 2: the row subtracts lse from the logit first.
   auto sweep = [&](auto mode_) {
     constexpr int MODE = decltype(mode_)::value;
     int qb = kb0;
@@ -727,7 +770,8 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
             const int i = 4 * rg + e;
             const float x = MODE == 0   ? __builtin_fmaf(sc[i], LOG2E_R, l4[e])
                             : MODE == 1 ? __builtin_fmaf(sc[i], LOG2E_R, l4[e] + kbias[u])
-                                        : __builtin_fmaf(sc[i] + kbias[u] - l4[e], LOG2E_R, pl2);
+                                        : __builtin_fmaf(sc[i] + kbias[u] - l4[e], LOG2E_R,
+                                                         l4[e] <= qbound ? nlog2 : pl2);
             sc[i] = fast_exp2(x);
             dp[i] *= sc[i];  // dS
           }
