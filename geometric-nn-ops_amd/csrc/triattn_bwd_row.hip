@@ -1,8 +1,7 @@
 // Triangle attention backward for gfx950, row-resident variant of dq and dk / dv: 16-bit
 // inputs, head dim 32, N_res <= BWD_ROW_MAX_N.
 //
-// Same mathematics and the same per-element arithmetic as bwd_dq_kernel and
-// bwd_dkdv_kernel (triattn_bwd.hip), so both paths give identical results:
+// Same mathematics as bwd_dq_kernel and bwd_dkdv_kernel (triattn_bwd.hip):
 //   dP_ij = dO_i . v_j,  dS_ij = P_ij (dP_ij - Delta_i),  P_ij = exp(S_ij - lse_i),
 //   dV_j = sum_i P_ij dO_i,  dK_j = sum_i dS_ij Q'_i,  dQ_i = scale * sum_j dS_ij k_j,
 // the gradient of triangle_attention_torch (geometric_nn_ops_torch/triangle/_reference/
@@ -26,6 +25,9 @@
 // correction for rows whose keys are all masked (P of a masked key divided by N_res, which
 // only changes such rows: elsewhere a masked key's P is exactly 0) joins the exponent, as
 // P = exp2((S - lse) log2(e) - log2(N_res)) (see lost_lse_bound).
+// Against the tiled kernels the results differ in their last bits: the exponent is one fma where
+// |lse| is small (subtracts_first; bwd_dkdv_row always subtracts first), and the fused kernel
+// adds dQ over the key blocks in an order that starts at the wave's own.
 #include <type_traits>
 
 #include "gnn_common.hpp"
@@ -125,10 +127,14 @@ __device__ __forceinline__ void row_coords(uint32_t w, int S, int H, int& b, int
   b = (int)(w / ((uint32_t)S * H));
 }
 
-// Whether a query's lse lies where the mask sentinel puts it: its keys are all masked, or the pair
-// bias alone holds the query down there. Its exponents then subtract lse from the logit first.
-__device__ __forceinline__ bool at_sentinel(const gnn_triattn_bwd_args& a, float lse) {
-  return a.mask && lse <= 0.5f * a.mask_value;
+// P = exp(S - lse) is exp2(fma(S, log2 e, -lse log2 e)), one fma per element, where the rounding of
+// -lse log2 e does no harm: up to FAR_LSE it is at most 2^-16, which moves P by 1.1e-5 of itself, a
+// twentieth of fp16's half ulp. It grows with |lse|; at the mask sentinel, or wherever the pair bias
+// alone puts a query, S - lse is exact and the rounded product is off by whole powers of two (bf16:
+// 0.5 at 1e7, 52 at 1e9). Queries there subtract lse from the logit first.
+constexpr float FAR_LSE = 256.f;
+__device__ __forceinline__ bool subtracts_first(const gnn_triattn_bwd_args& a, float lse) {
+  return fabsf(lse) > FAR_LSE || (a.mask && lse <= 0.5f * a.mask_value);
 }
 
 // ------------------------------------------------------------------------------- dQ
@@ -211,10 +217,9 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
       if (qok && g == 0) a.delta[lrow + qi] = delta;
     }
     const float lse = qok ? a.lse[lrow + qi] : INFINITY;  // absent queries: p = 0
-    // Unless a query of the wave sits at the sentinel, P = exp2(S log2 e - lse log2 e)
-    // takes one fma per element (lse is this lane's query's, constant along the accumulator);
-    // there S - lse is formed first.
-    const bool first = hdr.dead || __any(at_sentinel(a, lse));
+    // P = exp2(S log2 e - lse log2 e) takes one fma per element (lse is this lane's query's,
+    // constant along the accumulator) unless a query of the wave has S - lse formed first.
+    const bool first = hdr.dead || __any(qok && subtracts_first(a, lse));
     const float pl2 = hdr.dead || lse <= lost_lse_bound(a.mask, a.mask_value) ? -__log2f((float)N) : 0.f;
     const float nl2 = -lse * LOG2E_R;
     const T* brow = HAS_BIAS ? (const T*)a.bias + b * a.bias_stride[0] + h * a.bias_stride[1] +
@@ -251,8 +256,6 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dq_row_kernel(const gnn_triattn_bw
         for (int t2 = 0; t2 < 2; ++t2) Mma<T, PREC_NATIVE>::step(sc, idf[t2], bb[t2]);
         if (st + 1 < nst) load_bias(st + 1);
       }
-      // P = exp(S - lse), subtracting first: in a row whose keys are all masked both sit
-      // near the sentinel, and only their difference is exact
       f32x16 ds;
       if (plain && !first) {
 #pragma unroll
@@ -568,7 +571,7 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned char* tile = smem_raw + nb * sizeof(FusedBlock) + wave * 2048;  // this wave's dS tile [key][query]
   const int64_t lrow = (((int64_t)b * S + s) * H + h) * N;
-  // per wave, of its keys and the queries that it stages: 1 a live key, 2 a query at the sentinel
+  // per wave, of its keys and the queries that it stages: 1 a live key, 2 a query that subtracts first
   int* flags = reinterpret_cast<int*>(smem_raw + nb * sizeof(FusedBlock) + nth / 64 * 2048);
 
   // ---- this wave's keys: K and V as B operands (lane = key, 8 consecutive d), and the key-side
@@ -638,7 +641,7 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
     for (int r = tid; r < nrows; r += nth) {
       const float l = r < N ? a.lse[lrow + r] : INFINITY;
       blk[r >> 5].nl[r & 31] = l;
-      first |= at_sentinel(a, l);
+      first |= r < N && subtracts_first(a, l);
     }
     const int f = (__any(live) ? 1 : 0) | (__any(first) ? 2 : 0);
     if (lane == 0) flags[wave] = f;
@@ -760,8 +763,7 @@ __global__ __launch_bounds__(KB == 2 ? 512 : 768, KB == 2 ? 2 : 3) void bwd_fuse
         Mma<T, PREC_NATIVE>::step(dp, *reinterpret_cast<const V8*>(B.d + o_row0), vf[u][0]);
         Mma<T, PREC_NATIVE>::step(sc, *reinterpret_cast<const V8*>(B.q + o_row1), kf[u][1]);
         Mma<T, PREC_NATIVE>::step(dp, *reinterpret_cast<const V8*>(B.d + o_row1), vf[u][1]);
-        // P = exp2(S log2 e - lse log2 e [+ mask]); in a row whose keys are all masked S and lse
-        // both sit near the sentinel and are subtracted first
+        // P = exp2(S log2 e - lse log2 e [+ mask]), or with S - lse formed first (subtracts_first)
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
           const f32x4 l4 = *reinterpret_cast<const f32x4*>(&B.nl[8 * rg + 4 * g]);

@@ -1,9 +1,9 @@
 """Triangle-attention gradients where some queries' logits lie far from zero: the pair bias alone holds
 a query at the mask sentinel, or anywhere at all, next to ordinary queries and fully masked rows.
 
-The reference is the kernels' own definition in float64, from the forward's o and lse:
-P = exp(S - lse) with S rounded to fp32 (at 1e9 one ulp swallows q . k), Delta = dO . o. Held queries
-have q = 0, so that their S is the bias exactly. Tolerance: the table that the gradient tests use."""
+The backward gets o and lse as fp32 logits give them (at 1e9 one ulp swallows q . k) and is compared with
+its own definition in float64: P = exp(S - lse), Delta = dO . o. Held queries have q = 0, so that their
+S is the bias exactly. Tolerance: the table that the gradient tests use."""
 
 import pytest
 import torch
@@ -16,24 +16,32 @@ DEV = "cuda"
 MASK_VALUE = {torch.bfloat16: 1e9, torch.float16: torch.finfo(torch.float16).max / 2, torch.float32: 1e9}
 
 
+def heads_first(t):
+    return t.double().transpose(2, 3).contiguous()
+
+
+def scores(q, k, bias, mask):
+    """[B, S, H, N, N] in fp32, the mask term added last; and the scaled q."""
+    qs = heads_first((q.float() * q.shape[-1] ** -0.5).to(q.dtype))
+    s = (qs @ heads_first(k).transpose(-1, -2).contiguous() + bias.double()).float()
+    if mask is not None:
+        value = torch.tensor(-MASK_VALUE[q.dtype]).to(q.dtype).float().to(s.device)
+        s = torch.where(~mask, s + value, s)
+    return s, qs
+
+
 def gradients(q, k, v, bias, mask, o, dout, lse, *, divides_queries):
     """(dq, dk, dv, dbias). P of a masked key is divided by N, and so is, where the kernels do it, P
     of a query of a masked call whose lse has lost log(l) to the sentinel."""
-    dtype, (_, _, n, _, d) = q.dtype, q.shape
-    heads_first = lambda t: t.double().transpose(2, 3)  # noqa: E731
-    qs = heads_first((q.float() * d**-0.5).to(dtype))
+    n, d = q.shape[2], q.shape[4]
+    s, qs = scores(q, k, bias, mask)
     k, v, dout, o = (heads_first(t) for t in (k, v, dout, o))
-    # [B, S, H, N, N], added in fp32 order: the mask term last
-    s = (qs @ k.transpose(-1, -2).contiguous() + bias.double()).float()
-    factor = torch.ones_like(s, dtype=torch.float64)
+    p = torch.exp((s - lse[..., None]).double())
     if mask is not None:
-        masked = ~mask.expand(*s.shape[:2], 1, 1, n)
-        value = torch.tensor(-MASK_VALUE[dtype]).to(dtype).float().to(s.device)
-        s = torch.where(masked, s + value, s)
-        bound = min(0.5 * float(value), -(2.0**27))
-        held = (lse <= bound)[..., None] if divides_queries else torch.zeros_like(lse, dtype=torch.bool)[..., None]
-        factor = torch.where(masked | held, 1.0 / n, 1.0).double()
-    p = torch.exp((s - lse[..., None]).double()) * factor
+        divided = (~mask).expand(*s.shape[:2], 1, 1, n)
+        if divides_queries:
+            divided = divided | (lse <= min(-0.5 * MASK_VALUE[q.dtype], -(2.0**27)))[..., None]
+        p = torch.where(divided, p / n, p)
     ds = p * (dout @ v.transpose(-1, -2).contiguous() - (dout * o).sum(-1, keepdim=True))
     t = lambda x: x.transpose(-1, -2).contiguous()  # noqa: E731
     dq, dk, dv = d**-0.5 * (ds @ k), t(ds) @ qs, t(p) @ dout
@@ -49,24 +57,23 @@ def check(n, dtype, held_at, masked, *, d=32, rows=(0, 5, -1), divides_queries=T
     if masked:
         mask = key_mask(B, S, N, seed=n + 1, frac_keep=0.75, device=DEV)
         mask[:, 1] = False  # a row whose keys are all masked
-    q, bias = t["q"].clone(), t["bias"].clone()
+    q, k, v, bias = (t[x] for x in ("q", "k", "v", "bias"))
     q[:, :, list(rows)] = 0
     bias[..., list(rows), :] = held_at
-    dout = torch.randn(B, S, N, H, D, generator=gen(n + 2)).to(DEV, dtype)
-    lse = torch.empty((B, S, H, N), device=DEV, dtype=torch.float32)
-    o = K.triangle_attention_hip(q, t["k"], t["v"], bias=bias, mask=mask, lse=lse, precision="ieee")
-    got = K.triangle_attention_bwd_hip(q, t["k"], t["v"], o, dout, lse, bias=bias, mask=mask, precision="ieee")
-    want = gradients(q, t["k"], t["v"], bias, mask, o, dout, lse, divides_queries=divides_queries)
+    dout = torch.randn(*shape, generator=gen(n + 2)).to(DEV, dtype)
+    s = scores(q, k, bias, mask)[0].double()
+    lse = torch.logsumexp(s, -1).float()
+    o = (torch.softmax(s, -1) @ heads_first(v)).transpose(2, 3).to(dtype).contiguous()
+    got = K.triangle_attention_bwd_hip(q, k, v, o, dout, lse, bias=bias, mask=mask, precision="ieee")
+    want = gradients(q, k, v, bias, mask, o, dout, lse, divides_queries=divides_queries)
+    tol = TRIANGLE_ATTENTION_TOL[dtype, "ieee"]
     for name, g, w in zip(("dq", "dk", "dv", "dbias"), got, want):
-        assert torch.isfinite(g).all(), name
-        assert_close_to_oracle(name, g, to_np(w), TRIANGLE_ATTENTION_TOL[dtype, "ieee"])
+        assert_close_to_oracle(name, g, to_np(w), tol)
     # the other queries by themselves: a held one must not move them
     others = torch.ones(N, dtype=torch.bool, device=DEV)
     others[list(rows)] = False
-    assert_close_to_oracle("dq of the others", got[0][:, :, others], to_np(want[0][:, :, others]),
-                           TRIANGLE_ATTENTION_TOL[dtype, "ieee"])
-    assert_close_to_oracle("dbias of the others", got[3][..., others, :], to_np(want[3][..., others, :]),
-                           TRIANGLE_ATTENTION_TOL[dtype, "ieee"])
+    assert_close_to_oracle("dq of the others", got[0][:, :, others], to_np(want[0][:, :, others]), tol)
+    assert_close_to_oracle("dbias of the others", got[3][..., others, :], to_np(want[3][..., others, :]), tol)
 
 
 # the fused kernel with two key blocks a wave and with one, its largest N, and the two-kernel path
@@ -85,3 +92,13 @@ def test_masked_call_with_a_query_held_at_the_sentinel(n, dtype, held_at, rows):
 def test_masked_call_on_the_tiled_kernels(dtype, d):
     """Their dq, dk, dv and pair-bias gradient divide per masked key only."""
     check(130, dtype, -1e9, True, d=d, rows=(0, 128), divides_queries=False)
+
+
+@SIZES
+@pytest.mark.parametrize("masked", [False, True], ids=["plain", "masked"])
+@pytest.mark.parametrize("held_at", [-250.0, -300.0, -1e7, 1e7, -1e9, torch.finfo(torch.bfloat16).min],
+                         ids=["m250", "m300", "m1e7", "p1e7", "m1e9", "lowest"])
+def test_queries_held_far_from_zero(n, masked, held_at):
+    """On both sides of where the row kernels change from one fma to subtracting lse first, where lse
+    times log2(e) loses the exponent (1e7, 1e9), and where that product overflows."""
+    check(n, torch.bfloat16, held_at, masked, rows=(3, n // 2))
