@@ -1632,8 +1632,8 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_pp_kernel(const gnn_trimul
 
 // ============================== stage 2: per-channel contraction ==========================
 // fp32 under ieee: BM x BM output tiles, 4 waves of BM / 2 x BM / 2, one stage of 32 k held in
-// registers while the previous one multiplies. Columns N .. NP - 1 of a and b are zeros, so the
-// loads run to NP without a tail. Bound by the fp32 matrix rate (64 cycles per 32x32x2), so the
+// registers while the previous one multiplies. The loads run to NP without a tail; what lies past N
+// becomes zero on its way to LDS. Bound by the fp32 matrix rate (64 cycles per 32x32x2), so the
 // tile edge is chosen for the least padding: 64 where ceil(N / 64) is odd and at most 7 (128
 // planes, N = 64: 10.1 -> 4.9 us, 131: 30.0 -> 21.0, 300: 116 -> 90, 430: 270 -> 229), 128 otherwise
 // (half the cache bytes per flop at the same padded area; N = 690, 11 tiles of 64: 835 against 843).
@@ -1687,11 +1687,16 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restr
       }
     }
   };
-  auto store = [&]() {
+  auto store = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int c = tid + i * NT;
       const int r = c / CPR, kl = (c % CPR) * 8;
+      if (k0 + Cfg::BK > N) {  // uniform: the stage that crosses N; its padding may hold anything
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (k0 + kl + e >= N) ra[i][e] = rb[i][e] = TypeOps<T>::from_f32(0.f);
+      }
       store8(&as[r * Cfg::ROW + kl], ra[i]);
       store8(&bs[r * Cfg::ROW + kl], rb[i]);
     }
@@ -1707,7 +1712,7 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restr
 
   const int nkt = (N + Cfg::BK - 1) / Cfg::BK;
   load(0);
-  store();
+  store(0);
   __syncthreads();
   for (int kt = 0; kt < nkt; ++kt) {
     const bool has_next = kt + 1 < nkt;
@@ -1727,7 +1732,7 @@ __global__ __launch_bounds__(NT, 2) void trimul_contract_kernel(const T* __restr
         for (int y = 0; y < WT; ++y) Mma<T, PREC>::step(acc[x][y], af[x], bf[y]);
     }
     __syncthreads();
-    if (has_next) store();
+    if (has_next) store((kt + 1) * Cfg::BK);
     __syncthreads();
   }
 

@@ -91,6 +91,31 @@ def test_fp32_contraction_tiles(N, direction):
     assert _trimul_forward_error(N, 32, 32, torch.float32, direction) <= TOL[torch.float32]
 
 
+@pytest.mark.parametrize("precision", ["ieee", "bf16x3"])
+@pytest.mark.parametrize("N", [1, 33, 64, 131, 250])
+def test_fp32_contraction_ignores_the_padding(N, precision):
+    """Stage 2 by itself: fp32 a and b are specified up to column N only (16-bit types have zeros
+    there), on tiles of 64 and of 128."""
+    from geometric_nn_ops_torch import _lib
+    from geometric_nn_ops_torch.triangle._kernels import trimul as K
+
+    C, Ch = 32, 32
+    x, _ = pair_input(1, N, C, torch.float32, seed=N, device=DEV)
+    args, _keep, _out, workspace, offsets = K.build_args(x, "outgoing", None, 1e-5,
+                                                         trimul_weights(C, Ch, torch.float32, device=DEV))
+    args.precision = _lib.PRECISION_CODE[precision]
+    NP = (N + 31) // 32 * 32
+    workspace.view(torch.float32).fill_(float("nan"))
+    a, b, o = (workspace[offsets[i]:offsets[i] + 4 * Ch * N * NP].view(torch.float32).view(Ch, N, NP)
+               for i in (0, 1, 3))
+    g = gen(N)
+    for t in (a, b):
+        t[..., :N] = torch.randn(Ch, N, N, generator=g).to(DEV)
+    K.run_stage("gnn_trimul_contract", args, DEV_T)
+    want = a[..., :N].double() @ b[..., :N].double().transpose(1, 2).contiguous()
+    assert O.rel_fro(to_np(o[..., :N]), to_np(want)) <= (1e-5 if precision == "ieee" else 5e-5)
+
+
 @pytest.mark.parametrize("direction", ["outgoing", "incoming"])
 @pytest.mark.parametrize(("dtype", "N", "C", "Ch", "B"), [
     # one to four workgroups on a tile (256 compute units over N ceil(N / 64) B tiles)
