@@ -241,9 +241,11 @@ __device__ __forceinline__ float pair_sum(float x) { return x + __shfl_xor(x, 32
 // Attention backward, P = exp(S - lse): the saved lse has no room for log(l) where it holds the mask
 // sentinel, and exp(S - lse) is then 1 where softmax gives 1 / (number of keys). P of a masked key is
 // divided by N_res for that, as the reference does (only a row whose keys are all masked has a masked
-// key with P > 0). In a masked call so is P of a query of a row with live keys that the pair bias
-// alone holds there: its lse is at most this bound. 2^27 is where one ulp is 16 and swallows log(l) for any
-// l < 2900; sentinels nearer to zero (fp16's) leave log(l) in lse, and P needs no division.
+// key with P > 0). In a masked call the row-resident dq, dk and dv divide so the P of a query of a row
+// with live keys that the pair bias alone holds there: its lse is at most this bound. 2^27 is where one
+// ulp is 16 and swallows log(l) for any l < 2900; sentinels nearer to zero (fp16's) leave log(l) in
+// lse, and P needs no division. The tiled kernels and the pair-bias gradient go by the key alone (the
+// latter asking each row's lse as well took 113 us a call instead of 109 at N = 384, bf16).
 __device__ __forceinline__ float lost_lse_bound(const void* mask, float mask_value) {
   return mask ? fminf(0.5f * mask_value, -0x1p27f) : -INFINITY;
 }

@@ -31,9 +31,7 @@
 // (triangle_attention.py:753-766, :1033-1038): in a row whose keys are all masked the
 // forward's lse holds the bare sentinel (its log(l) term is below the fp32 ulp there), so
 // exp(S - lse) is 1 for every key where softmax gives 1 / N_res; in any other row a masked
-// key's P is 0 either way. In bwd_dbias -log2(N_res) joins the exp2 argument of a masked key; its
-// DMA form, which goes with the row-resident dq / dk / dv kernels, divides as they do
-// (lost_lse_bound).
+// key's P is 0 either way. In bwd_dbias -log2(N_res) joins the exp2 argument of a masked key.
 // 16-bit inputs, head dim <= 128 (a multiple of 8, ensured by the host). Every kernel is
 // templated on DC, the number of 32-column chunks of the head dim (1, 2 or 4): the staged
 // tiles are DC swizzled [rows][32] tiles, the score and dP products sum over the chunks, and
@@ -819,7 +817,7 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_dma_kernel(const gnn_triat
 
   const float scale = a.scale;
   constexpr bool has_mask = MASK;
-  const float nlog2 = -__log2f((float)N), qbound = lost_lse_bound(a.mask, a.mask_value);
+  const float nlog2 = -__log2f((float)N);
   auto compute_row = [&](int stage, int mrow) {
     const DbdStage& st = sm.st[stage];
     // dO fragments negated (a sign flip, exact) and the dP accumulator started at Delta: the
@@ -841,7 +839,6 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_dma_kernel(const gnn_triat
 #pragma unroll
       for (int e = 0; e < 4; ++e) dinit[4 * rg + e] = d4[e];
     }
-    const bool lost = has_mask && __any(st.lse[qw + l32] <= qbound);
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       const int kr = kw + 32 * sub + l32;
@@ -853,21 +850,16 @@ __global__ __launch_bounds__(DB_NT, 1) void bwd_dbias_dma_kernel(const gnn_triat
       }
       const bool masked = has_mask && sm.mask[mrow][kr] == 0;
       const float kb = masked ? a.mask_value : 0.f, kpl2 = masked ? nlog2 : 0.f;
-      // the logit minus lse first (in a fully masked row both sit near the sentinel)
-      auto p = [&](int i, float lse, float pl2) {
-        const float x = has_mask ? scv[i] + kb - lse : scv[i] - lse;
-        return fast_exp2(has_mask ? __builtin_fmaf(x, LOG2E_B, pl2) : x * LOG2E_B);
-      };
-      if (lost) {  // uniform
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float lse = l4[i / 4][i % 4];
-          acc[sub][i] -= p(i, lse, lse <= qbound ? nlog2 : kpl2) * ndp[i];
+      for (int rg = 0; rg < 4; ++rg)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * rg + e;
+          // the logit minus lse first (in a fully masked row both sit near the sentinel)
+          const float x = has_mask ? scv[i] + kb - l4[rg][e] : scv[i] - l4[rg][e];
+          const float pv = fast_exp2(has_mask ? __builtin_fmaf(x, LOG2E_B, kpl2) : x * LOG2E_B);
+          acc[sub][i] -= pv * ndp[i];
         }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[sub][i] -= p(i, l4[i / 4][i % 4], kpl2) * ndp[i];
-      }
     }
   };
 

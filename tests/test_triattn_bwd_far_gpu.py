@@ -31,21 +31,23 @@ def scores(q, k, bias, mask):
 
 
 def gradients(q, k, v, bias, mask, o, dout, lse, *, divides_queries):
-    """(dq, dk, dv, dbias). P of a masked key is divided by N, and so is, where the kernels do it, P
-    of a query of a masked call whose lse has lost log(l) to the sentinel."""
+    """(dq, dk, dv, dbias). P of a masked key is divided by N, and so is, in dq, dk and dv of the
+    row-resident kernels, P of a query of a masked call whose lse has lost log(l) to the sentinel."""
     n, d = q.shape[2], q.shape[4]
     s, qs = scores(q, k, bias, mask)
     k, v, dout, o = (heads_first(t) for t in (k, v, dout, o))
     p = torch.exp((s - lse[..., None]).double())
     if mask is not None:
-        divided = (~mask).expand(*s.shape[:2], 1, 1, n)
-        if divides_queries:
-            divided = divided | (lse <= min(-0.5 * MASK_VALUE[q.dtype], -(2.0**27)))[..., None]
-        p = torch.where(divided, p / n, p)
-    ds = p * (dout @ v.transpose(-1, -2).contiguous() - (dout * o).sum(-1, keepdim=True))
+        p = torch.where(mask, p, p / n)
+    dp = dout @ v.transpose(-1, -2).contiguous() - (dout * o).sum(-1, keepdim=True)
+    dbias = (p * dp).sum(1, keepdim=True)
+    if mask is not None and divides_queries:
+        held = (lse <= min(-0.5 * MASK_VALUE[q.dtype], -(2.0**27)))[..., None]
+        p = torch.where(held & mask, p / n, p)
+    ds = p * dp
     t = lambda x: x.transpose(-1, -2).contiguous()  # noqa: E731
     dq, dk, dv = d**-0.5 * (ds @ k), t(ds) @ qs, t(p) @ dout
-    return (*(x.transpose(2, 3) for x in (dq, dk, dv)), ds.sum(1, keepdim=True))
+    return (*(x.transpose(2, 3) for x in (dq, dk, dv)), dbias)
 
 
 def check(n, dtype, held_at, masked, *, d=32, rows=(0, 5, -1), divides_queries=True):
