@@ -41,6 +41,12 @@ static int hip_status(hipError_t e, const char* who) {
 
 static bool aligned(const void* p, size_t n) { return ((uintptr_t)p % n) == 0; }
 
+// Every row of the pair bias starts on 16 bytes and has a pitch up to round_up(N, 8), which is read
+static bool bias_rows_readable(const void* bias, const int64_t (&st)[4], int64_t B, int64_t H, int64_t N) {
+  return st[3] == 1 && st[2] % 8 == 0 && (st[2] >= N || N % 8 == 0) && (H == 1 || st[1] % 8 == 0) &&
+         (B == 1 || st[0] % 8 == 0) && aligned(bias, 16);
+}
+
 // caller_workspace: the caller provides the scratch (gnn_triattn_fwd); false for the entry
 // point whose scratch is the library's static array.
 static int check_triattn(const gnn_triattn_args& a, bool caller_workspace = true) {
@@ -61,12 +67,10 @@ static int check_triattn(const gnn_triattn_args& a, bool caller_workspace = true
       if (st[t][d] % 8 != 0)
         return set_error(GNN_ERR_ARG, "triangle_attention: q/k/v/o strides must be multiples of 8 elements");
   }
-  if (a.bias && !triattn_row_applicable(a)) {
-    if (a.bias_stride[3] != 1 || a.bias_stride[2] % 8 != 0 || !aligned(a.bias, 16))
-      return set_error(GNN_ERR_ARG,
-                       "triangle_attention: bias needs unit key stride, a query stride that is a multiple "
-                       "of 8 and 16-byte alignment");
-  }
+  if (a.bias && !triattn_row_applicable(a) && !bias_rows_readable(a.bias, a.bias_stride, a.B, a.H, a.N))
+    return set_error(GNN_ERR_ARG,
+                     "triangle_attention: bias needs unit key stride, other strides that are multiples of 8, rows "
+                     "readable to round_up(N, 8) and 16-byte alignment");
   const size_t need = triattn_row_applicable(a) ? triattn_row_workspace_bytes(a) : 0;
   if (caller_workspace && need && (!a.workspace || a.workspace_bytes < need || !aligned(a.workspace, 16)))
     return set_error(GNN_ERR_WORKSPACE,
@@ -120,9 +124,9 @@ int gnn_triattn_bwd(const gnn_triattn_bwd_args* args, void* stream) {
       if (st[t][d] % 8 != 0)
         return set_error(GNN_ERR_ARG, "triangle_attention backward: q/k/v/o/dout strides must be multiples of 8 elements");
   }
-  if (a.bias && (a.bias_stride[3] != 1 || a.bias_stride[2] % 8 != 0 || !aligned(a.bias, 16)))
-    return set_error(GNN_ERR_ARG, "triangle_attention backward: bias needs unit key stride, a query stride that is a "
-                                  "multiple of 8 and 16-byte alignment");
+  if (a.bias && !bias_rows_readable(a.bias, a.bias_stride, a.B, a.H, a.N))
+    return set_error(GNN_ERR_ARG, "triangle_attention backward: bias needs unit key stride, other strides that are "
+                                  "multiples of 8, rows readable to round_up(N, 8) and 16-byte alignment");
   int rc = triattn_bwd(a, (hipStream_t)stream);
   if (rc < 0) return rc;
   return hip_status((hipError_t)rc, "triangle_attention backward");

@@ -851,8 +851,9 @@ int launch_bwd_fused(const gnn_triattn_bwd_args& a, hipStream_t stream) {
 
 template <typename T, bool HAS_BIAS>
 int launch_bwd_row(const gnn_triattn_bwd_args& a, hipStream_t stream) {
-  // (the fused kernel addresses the bias plane in 32 bits)
-  if (a.N <= BWD_FUSED_MAX_N && (!HAS_BIAS || a.N * a.bias_stride[2] < ((int64_t)1 << 31)))
+  // (the fused kernel addresses the bias plane in unsigned 32 bits)
+  if (a.N <= BWD_FUSED_MAX_N &&
+      (!HAS_BIAS || (a.bias_stride[2] >= 0 && a.N * a.bias_stride[2] < ((int64_t)1 << 31))))
     return fused_kb((int)a.N) == 2 ? launch_bwd_fused<T, HAS_BIAS, 2>(a, stream)
                                    : launch_bwd_fused<T, HAS_BIAS, 1>(a, stream);
   const int64_t ntiles = (a.N + RT - 1) / RT;

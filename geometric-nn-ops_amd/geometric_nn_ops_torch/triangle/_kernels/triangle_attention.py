@@ -51,14 +51,28 @@ def _prepare(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
+def _bias_readable(bias: torch.Tensor) -> bool:
+    """Whether every row ``[b, 0, h, i, :]`` starts on 16 bytes, has unit stride and can be read up to
+    round_up(N, 8): inside its own pitch (a bias broadcast over the queries has none) and, for the
+    last row, inside the storage."""
+    B, _, H, N, _ = bias.shape
+    b, _, h, i, j = bias.stride()
+    if j != 1 or i % 8 or (H > 1 and h % 8) or (B > 1 and b % 8) or bias.data_ptr() % 16:
+        return False
+    if N % 8 == 0:
+        return True
+    end = bias.storage_offset() + (B - 1) * b + (H - 1) * h + (N - 1) * i + (N + 7) // 8 * 8
+    return i >= N and end * bias.element_size() <= bias.untyped_storage().nbytes()
+
+
 def _prepare_bias(bias: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """``[B, 1, H, N, N]`` bias in ``dtype``. The 16-bit row kernel reads any strides (its
-    pre-pass rewrites the bias in fragment order); the tiled kernel needs unit key stride, a
-    query pitch that is a multiple of 8 elements and a 16-byte aligned base, so such views
-    are copied with the pitch padded. No kernel uses what lies past N, so the padding is not
+    pre-pass rewrites the bias in fragment order); the tiled kernel and the backward read rows in
+    aligned groups of 8 elements, so a view whose rows cannot be read that way (``_bias_readable``)
+    is copied with the pitch padded. No kernel uses what lies past N, so the padding is not
     filled (the fill cost 5 us of a 145 us forward at N = 333 in fp32)."""
     bias = bias.to(dtype)
-    if bias.stride(-1) == 1 and bias.stride(-2) % 8 == 0 and bias.data_ptr() % 16 == 0:
+    if _bias_readable(bias):
         return bias
     B, _, H, N, _ = bias.shape
     pitch = (N + 7) // 8 * 8

@@ -90,7 +90,10 @@ typedef struct gnn_triattn_args {
   int64_t v_stride[4];
   int64_t o_stride[4];
   int64_t bias_stride[4]; /* b, h, i, j (any strides for 16-bit inputs with D <= 32 and
-                             N <= 1024; otherwise j stride 1, i stride a multiple of 8) */
+                             N <= 1024; otherwise j stride 1, the others multiples of 8 (where the
+                             dim is above 1) and every row, from a 16-byte aligned start, readable
+                             up to round_up(N, 8): an i stride of at least N unless N % 8 == 0.
+                             What lies past N may hold anything) */
   int64_t mask_stride[3]; /* b, s, j */
   float scale;
   float mask_value;
@@ -159,7 +162,8 @@ typedef struct gnn_triattn_bwd_args {
   int64_t dq_stride[4];
   int64_t dk_stride[4];
   int64_t dv_stride[4];
-  int64_t bias_stride[4]; /* b, h, i, j (j stride must be 1) */
+  int64_t bias_stride[4]; /* b, h, i, j: j stride 1, the others multiples of 8, rows readable up to
+                             round_up(N, 8), as in gnn_triattn_args */
   int64_t mask_stride[3]; /* b, s, j */
   float scale;
   float mask_value;
