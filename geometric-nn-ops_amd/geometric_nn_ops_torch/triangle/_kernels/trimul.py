@@ -468,6 +468,8 @@ def rows_products_hip(pairs, slice_rows=0):
         p.d, p.t, p.d_ld, p.t_ld, p.O, p.I = (d.data_ptr(), t.data_ptr(), d.stride(0), t.stride(0), d.shape[1],
                                               t.shape[1])
     slices = lib.gnn_rows_product_slices(ctypes.byref(a))
+    if slices and not slice_rows:  # that count depends on the device current here, the launch must not: pin its split
+        a.slice_rows = (-(-a.rows // slices) + 31) // 32 * 32
     parts = [torch.empty((slices, d.shape[1], t.shape[1]), device=d0.device, dtype=torch.float32) for d, t in pairs]
     for p, part in zip(a.p, parts):
         p.partial = part.data_ptr()

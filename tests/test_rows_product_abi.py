@@ -59,3 +59,29 @@ def test_reduce_argument_errors(bad):
     for k, v in bad.items():
         setattr(s, k, v)
     assert _lib.load().gnn_reduce_parts(ctypes.byref(a), None) == _lib.GNN_ERR_ARG
+
+
+@pytest.mark.parametrize("rows", [1, 31, 257, 5000, 40401, 147456])
+@pytest.mark.parametrize("cus", [1, 32, 256])
+def test_the_launch_is_held_to_the_slices_that_were_allocated(rows, cus, monkeypatch):
+    """The number of slices follows the compute units of whichever device is current when it is asked
+    for; the tensors' own device must not decide again. The wrapper passes the split on."""
+    import torch
+
+    from geometric_nn_ops_torch.triangle._kernels import trimul as K
+
+    per = max(-(-rows // max(1, 2 * cus)), 256)
+    chosen = -(-rows // (-(-per // 32) * 32))
+
+    class Lib:
+        def gnn_rows_product_slices(self, args):
+            return chosen
+
+    launched = []
+    monkeypatch.setattr(_lib, "load", lambda: Lib())
+    monkeypatch.setattr(_lib, "call", lambda fn, a, device: launched.append((fn, a.slice_rows)))
+    (part,) = K.rows_products_hip([(torch.empty(rows, 8, dtype=torch.bfloat16), torch.empty(rows, 8, dtype=torch.bfloat16))])
+    monkeypatch.undo()
+    assert part.shape[0] == chosen and launched[0][0] == "gnn_rows_product"
+    again = _product(rows=rows, slice_rows=launched[0][1])
+    assert launched[0][1] > 0 and _lib.load().gnn_rows_product_slices(ctypes.byref(again)) == chosen
