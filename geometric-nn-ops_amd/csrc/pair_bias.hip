@@ -55,8 +55,27 @@ struct PairBiasCfg {
   static constexpr int CHUNKS = KS * (int)sizeof(T) / 2;       // 16-byte chunks per lane
 };
 
+// fp32 products of channel pairs C0 .. C0 + N - 1, leaves of 4 or 8 pairs added as a binary tree (in order, so
+// that few of its sums are live at a time)
+template <int KS, int C0, int N>
+__device__ __forceinline__ f32x16 pair_bias_sum(const f32x8 (&w)[KS], const f32x8 (&x)[KS]) {
+  if constexpr (N > (KS > 4 ? 8 : 4)) {
+    f32x16 s = pair_bias_sum<KS, C0, N / 2>(w, x);
+    s += pair_bias_sum<KS, C0 + N / 2, N / 2>(w, x);
+    return s;
+  } else {
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int c = C0; c < C0 + N; ++c)
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(w[c / 8][c % 8], x[c / 8][c % 8], s, 0, 0, 0);
+    return s;
+  }
+}
+
 template <typename T, int KS>
-__global__ __launch_bounds__((64 * PairBiasCfg<T, KS>::NW), (sizeof(T) == 2 && KS <= 8 ? 4 : 1)) void pair_bias_proj_kernel(const gnn_pair_bias_args a) {
+__global__ __launch_bounds__((64 * PairBiasCfg<T, KS>::NW), (KS <= (sizeof(T) == 2 ? 8 : 4) ? 4 : 1)) void pair_bias_proj_kernel(const gnn_pair_bias_args a) {
   typedef typename TypeOps<T>::V8 V8;
   typedef PairBiasCfg<T, KS> Cfg;
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -149,10 +168,16 @@ __global__ __launch_bounds__((64 * PairBiasCfg<T, KS>::NW), (sizeof(T) == 2 && K
   for (int h0 = 0; h0 < H; h0 += 32) {
     if (h0 > 0) weights(h0);
     f32x16 acc;
+    if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) Mma<T, PREC>::step(acc, w[kk], x[kk]);
+      for (int kk = 0; kk < KS; ++kk) Mma<T, PREC>::step(acc, w[kk], x[kk]);
+    } else {
+      // sums over 8 channels (16 past 64), added as a tree: one sum over all 128 is 2.1e-7 off, the eight-lane
+      // dot products were 1.1e-7 (Zc = 64: 1.5e-7 and 0.95e-7)
+      acc = pair_bias_sum<KS, 0, 8 * KS>(w, x);
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int h = h0 + 8 * (i / 4) + 4 * g + i % 4;
