@@ -18,9 +18,9 @@
 // lanes, and the projection is [32 heads][Zc] x [Zc][32 pixels] with the weights as A fragments
 // (heads past H repeat the last one and are not stored; chunks past Zc are zero on both sides).
 // The result has a pixel per lane, so each head's 32 values leave as one run. Bound by HBM
-// (Zc * e bytes read per pixel against H * e written). The matrix unit replaced eight-lane dot
-// products on the vector ALU (H * Zc / 8 FMAs with an LDS read each and three shuffles per head
-// and lane): 54 -> 18.4 us at 384 x 384 pixels, Zc = 128, H = 16, bf16.
+// (Zc * e bytes read per pixel against H * e written). Against eight-lane dot products on the
+// vector ALU (H * Zc / 8 FMAs with an LDS read each and three shuffles per head and lane), which
+// few heads still take (pair_bias_dot): 54 -> 18.4 us at 384 x 384 pixels, Zc = 128, H = 16, bf16.
 //
 // Also here: the gate and output projection of attention with pair bias (apb_gate_out_kernel,
 // below), the part of the op after the attention itself.
@@ -186,8 +186,141 @@ __global__ __launch_bounds__((64 * PairBiasCfg<T, KS>::NW), (KS <= (sizeof(T) ==
   }
 }
 
+// The same with dot products on the vector ALU, where heads are few: eight lanes per pixel (a wave
+// holds 8 consecutive pixels), lane j loading the 8-channel chunks j, j + 8, ... of its row; LayerNorm
+// sums over the 8 lanes with xor shuffles; the weights as fp32 in LDS; a head's 8 partial products meet
+// through three shuffles and lane h % 8 stores it. Time grows with H, where the matrix unit forms 32
+// heads whatever their number (in fp32 at 64 cycles per channel pair).
+constexpr int PB_THREADS = 256;          // 4 waves
+constexpr int PB_PIX = PB_THREADS / 8;   // pixels per workgroup and step
+constexpr int PB_MAX_CHUNKS = PB_MAX_ZC / 64;
+
+template <typename T>
+__global__ __launch_bounds__(PB_THREADS) void pair_bias_dot_kernel(const gnn_pair_bias_args a) {
+  __shared__ float ws[PB_MAX_W];
+  __shared__ float gs[PB_MAX_CHUNKS * 64];
+  const int Zc = (int)a.Zc, H = (int)a.H, V = (int)a.V, U = (int)a.U;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < H * Zc; i += PB_THREADS) ws[i] = TypeOps<T>::to_f32(((const T*)a.proj_w)[i]);
+  for (int i = tid; i < Zc; i += PB_THREADS)
+    gs[i] = a.ln_w ? TypeOps<T>::to_f32(((const T*)a.ln_w)[i]) : 1.0f;
+  __syncthreads();
+
+  const int j = tid & 7;
+  const int nch = Zc / 8;
+  const int64_t npix = a.B * (int64_t)U * V;
+  const float inv_zc = 1.0f / (float)Zc;
+  for (int64_t p0 = (int64_t)blockIdx.x * PB_PIX; p0 < npix; p0 += (int64_t)gridDim.x * PB_PIX) {
+    const int64_t p = p0 + (tid >> 3);
+    const bool ok = p < npix;
+    const T* row = (const T*)a.z + (ok ? p : 0) * Zc;
+    f32x8 x[PB_MAX_CHUNKS];
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
+      const int ch = j + 8 * c;
+      if (ch < nch) {
+        x[c] = TypeOps<T>::to_f32(load8(row + 8 * ch));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += x[c][e];
+      }
+    }
+    s += __shfl_xor(s, 1);
+    s += __shfl_xor(s, 2);
+    s += __shfl_xor(s, 4);
+    const float mean = s * inv_zc;
+    float q = 0.f;
+#pragma unroll
+    for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
+      if (j + 8 * c < nch) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float d = x[c][e] - mean;
+          q += d * d;
+        }
+      }
+    }
+    q += __shfl_xor(q, 1);
+    q += __shfl_xor(q, 2);
+    q += __shfl_xor(q, 4);
+    const float rstd = 1.0f / sqrtf(q * inv_zc + a.eps);
+    // normalised, gamma-scaled and rounded to the input dtype (F.layer_norm's output)
+#pragma unroll
+    for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
+      const int ch = j + 8 * c;
+      if (ch < nch) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          x[c][e] = TypeOps<T>::to_f32(TypeOps<T>::from_f32((x[c][e] - mean) * rstd * gs[8 * ch + e]));
+      }
+    }
+    int64_t b = 0, u = 0, v = 0;
+    if (ok) {
+      v = p % V;
+      const int64_t r = p / V;
+      u = r % U;
+      b = r / U;
+    }
+    T* orow = (T*)a.out + b * a.out_stride[0] + u * a.out_stride[2] + v;
+    for (int h = 0; h < H; ++h) {
+      const float* wh = ws + h * Zc;
+      float acc = 0.f;
+#pragma unroll
+      for (int c = 0; c < PB_MAX_CHUNKS; ++c) {
+        const int ch = j + 8 * c;
+        if (ch < nch) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(x[c][e], wh[8 * ch + e], acc);
+        }
+      }
+      acc += __shfl_xor(acc, 1);
+      acc += __shfl_xor(acc, 2);
+      acc += __shfl_xor(acc, 4);
+      if (ok && (h & 7) == j) orow[h * a.out_stride[1]] = TypeOps<T>::from_f32(acc);
+    }
+  }
+}
+
+template <typename T>
+int launch_pb_dot(const gnn_pair_bias_args& a, hipStream_t stream) {
+  const int64_t want = (a.B * a.U * a.V + PB_PIX - 1) / PB_PIX;
+  const int64_t grid =
+      std::min<int64_t>(want, 4 * (int64_t)persistent_grid((const void*)pair_bias_dot_kernel<T>, PB_THREADS, 0));
+  hipLaunchKernelGGL(pair_bias_dot_kernel<T>, dim3((uint32_t)grid), dim3(PB_THREADS), 0, stream, a);
+  return (int)hipGetLastError();
+}
+
+#ifndef GNN_PB_DOT  // 0 / 1: never / always the dot products
+#define GNN_PB_DOT -1
+#endif
+// Whether heads are so few that the dot products are faster: their time grows with the heads, that of the
+// matrix unit with the channels, and up to 16384 pixels (a wave of the matrix kernel for each half
+// SIMD or less) the latter is its chain of loads, LDS passes and products. us, matrix unit / dot products:
+//   pixels  Zc    fp32: H = 4      8          12         16      | bf16: H = 2      6          10
+//   128^2   64    6.0 / 4.4   6.1 / 5.5   6.3 / 6.6               | 5.2 / 4.0   5.3 / 5.1   5.2 / 6.2
+//           128   9.1 / 5.0   9.1 / 6.5   9.3 / 8.0   9.2 / 9.4   | 7.6 / 4.5   7.7 / 6.1   7.7 / 7.6
+//           256   15.6 / 6.2  15.7 / 8.7  15.6 / 11.1 15.7 / 13.7 | 11.4 / 5.4  11.5 / 8.2  11.5 / 10.7
+//   160^2   64    6.2 / 4.9   6.3 / 6.5                           | 5.2 / 4.4   5.3 / 6.0
+//           128   11.6 / 6.1  11.6 / 8.7  11.8 / 11.2 11.8 / 13.7 | 7.7 / 5.1   7.7 / 7.5   7.7 / 10.0
+//           256   16.2 / 8.7  16.2 / 13.2 16.5 / 17.8             | 11.8 / 6.6  11.9 / 11.0 11.9 / 15.6
+//   256^2   64    7.9 / 8.4   8.0 / 11.3                          | 5.4 / 7.2
+//           128   13.2 / 11.5 13.8 / 16.9                         | 7.9 / 8.6
+//           256   38 / 21     39 / 28     40 / 36     40 / 44     | 13.1 / 12.3 13.5 / 20.4
+//   384^2   64    17.8 / 16.9 18.3 / 22.9                         | 8.1 / 13.2
+//           128   35 / 22     36 / 32     36 / 41     37 / 50     | 16.8 / 18.0
+//           256   87 / 35     88 / 48     89 / 65     90 / 82     | 37 / 26     37 / 39
+template <typename T, int KS>
+bool pair_bias_dot(const gnn_pair_bias_args& a) {
+  if (GNN_PB_DOT >= 0) return GNN_PB_DOT;
+  const int64_t px = a.B * a.U * a.V;
+  if (sizeof(T) == 4)
+    return a.H <= (px <= 16384 ? std::min(2 * KS, 16) : px <= 32768 ? std::min(3 * KS / 2, 10) : 3 * KS / 4);
+  return a.H <= (px <= 16384 ? std::min(3 * KS / 2, 10) : px <= 32768 ? std::min(KS / 2, 6) : KS > 8 ? 3 : 0);
+}
+
 template <typename T, int KS>
 int launch_pb(const gnn_pair_bias_args& a, hipStream_t stream) {
+  if (pair_bias_dot<T, KS>(a)) return launch_pb_dot<T>(a, stream);
   constexpr int pix = 32 * PairBiasCfg<T, KS>::NW;
   const int64_t grid = (a.B * a.U * a.V + pix - 1) / pix;
   if (grid >= ((int64_t)1 << 31)) return set_error(GNN_ERR_UNSUPPORTED, "pair_bias_proj: too many pixels");

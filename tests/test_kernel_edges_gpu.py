@@ -49,6 +49,27 @@ def test_pair_bias_projection_tiles(Zc, H, U, V, dtype):
     assert O.rel_fro(to_np(got), want) <= TOL[dtype]
 
 
+@DTYPES
+@pytest.mark.parametrize("V", [128, 129, 256, 257])
+@pytest.mark.parametrize(("Zc", "heads"), [(8, (1, 2, 3, 6, 7, 8, 9)), (64, (1, 3, 4)), (72, (4, 5, 6, 7, 10, 11, 16, 17)),
+                                           (256, (3, 4, 6, 7, 10, 11, 12, 13, 16, 17))])
+def test_pair_bias_head_counts(Zc, heads, V, dtype):
+    """Head counts on both sides of where the dot products give way to the matrix unit, at 16384 and
+    32768 pixels, where those change, and one row past them."""
+    from geometric_nn_ops_torch.triangle._kernels.attention_pair_bias import pair_bias_projection_hip
+
+    g = torch.Generator(device=DEV).manual_seed(Zc)
+    z = torch.randn(2, 64, V, Zc, generator=g, device=DEV).to(dtype)
+    lw = (1.0 + 0.1 * torch.randn(Zc, generator=g, device=DEV)).to(dtype)
+    zn = torch.nn.functional.layer_norm(z.double(), (Zc,), lw.double())
+    for H in heads:
+        w = (torch.randn(H, Zc, generator=g, device=DEV) * Zc ** -0.5).to(dtype)
+        want = torch.nn.functional.linear(zn, w.double()).permute(0, 3, 1, 2)
+        got = pair_bias_projection_hip(z, lw, w, 1e-5)
+        assert got.shape == want.shape
+        assert (got.double() - want).norm() <= TOL[dtype] * want.norm(), H
+
+
 @pytest.mark.parametrize("Zc", [64, 128, 256])
 def test_fp32_pair_bias_sums(Zc):
     """A running sum of m products of random signs is off by about 2^-24 sqrt(m / 11) of itself: sums of
@@ -58,7 +79,7 @@ def test_fp32_pair_bias_sums(Zc):
 
     g = torch.Generator(device=DEV).manual_seed(Zc)
     z = torch.randn(1, 96, 96, Zc, generator=g, device=DEV)
-    w = torch.randn(16, Zc, generator=g, device=DEV) * Zc ** -0.5
+    w = torch.randn(24, Zc, generator=g, device=DEV) * Zc ** -0.5  # heads for the matrix unit
     lw = 1.0 + 0.1 * torch.randn(Zc, generator=g, device=DEV)
     zn = torch.nn.functional.layer_norm(z.double(), (Zc,), lw.double())
     want = torch.nn.functional.linear(zn, w.double()).permute(0, 3, 1, 2)
