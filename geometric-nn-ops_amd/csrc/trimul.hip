@@ -2788,11 +2788,12 @@ int launch_out_w(const gnn_trimul_args& a, const TrimulLayout& L, hipStream_t st
       return (int)hipGetLastError();
     }
   }
-  // fp32 tiles too few for the CUs are halved: each is a serial chain of loads, LayerNorm, products
-  // and stores, so its length is the time. N = 64, c_z = c_hidden = 128: 11.5 -> 8.4 us
+  // fp32 tiles are halved while the halves have a CU each: a tile is a serial chain of loads, LayerNorm,
+  // products and stores, so its length is the time. N = 64, c_z = c_hidden = 128: 11.5 -> 8.4 us; two
+  // halves to a CU are slower than one whole tile (N = 100: 12.5 against 11.7)
   if constexpr (sizeof(T) == 4 && !(PREC == PREC_BF16X3 && CK == 128)) {
-    if (a.B * a.N * ntile < compute_units()) {
-      constexpr int PT = 32;
+    constexpr int PT = 32;
+    if (a.B * a.N * ((a.N + PT - 1) / PT) <= compute_units()) {
       const size_t hsmem = out_lds_bytes(a.Ch, sizeof(T), PT);
       const void* hf = (const void*)trimul_out_kernel<T, PREC, CK, CHK, PT>;
       if (hsmem > 64 * 1024) (void)hipFuncSetAttribute(hf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)hsmem);

@@ -169,10 +169,11 @@ def test_projection_dispatch(dtype, N, C, Ch, B, direction):
 
 @pytest.mark.parametrize(("N", "C", "Ch", "B"), [(1, 128, 128, 1), (32, 128, 128, 1), (33, 128, 128, 3),
                                                  (97, 32, 96, 1), (127, 128, 128, 1), (128, 128, 128, 1),
-                                                 (65, 256, 32, 1), (31, 160, 256, 2)])
+                                                 (65, 256, 32, 1), (31, 160, 256, 2), (85, 64, 64, 1), (86, 64, 64, 1),
+                                                 (128, 64, 64, 2)])
 def test_fp32_output_tiles(N, C, Ch, B):
-    """Output tiles of 32 and 64 pixels (below and from 256 tiles of 64 on), their row tails, and more
-    output channels than one pass."""
+    """Output tiles of 32 pixels (up to 256 of them) and 64, their row tails, and more output channels
+    than one pass."""
     assert _trimul_forward_error(N, C, Ch, torch.float32, "outgoing", B) <= TOL[torch.float32]
 
 
