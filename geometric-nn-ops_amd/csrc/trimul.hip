@@ -392,16 +392,18 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_ar
     // gated projection units: acc = [pixel][channel], row = pixel 32s + 8(r/4) + 4g + r%4,
     // col = channel 32u + l32; staged as [channel][pixel] for 128-byte row stores
     for (int j = 0;; ++j) {
-      int u, s0;  // unit, first sub-tile
+      int u, s_begin, s_end;  // unit, its sub-tiles: all of them, or one pass of a shared tile
       if constexpr (!SPLIT) {
-        u = wave + PW * (j / PGRP);
-        s0 = SPT * (j % PGRP);
+        u = wave + PW * j;
         if (u >= npg) break;
+        s_begin = 0;
+        s_end = PSUB;
       } else {
         const int it = part + split * (wave + PW * j);
         if (it >= npg * PGRP) break;
         u = it % npg;
-        s0 = SPT * (it / npg);
+        s_begin = SPT * (it / npg);
+        s_end = s_begin + SPT;
       }
       const int ch = 32 * u + l32;
       const T* wprow = wp + (int64_t)ch * C + 8 * g;
@@ -420,58 +422,60 @@ __global__ __launch_bounds__(PNT, 1) void trimul_proj_kernel(const gnn_trimul_ar
         if (nk <= KCH) load_w(0);
         wp_unit = u;
       }
+      for (int s0 = s_begin; s0 < s_end; s0 += SPT) {
 #pragma unroll
-      for (int s2 = 0; s2 < SPT; ++s2) {
-        const int s = s0 + s2;
-        f32x16 accp, accg;
+        for (int s2 = 0; s2 < SPT; ++s2) {
+          const int s = s0 + s2;
+          f32x16 accp, accg;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          accp[r] = bp;
-          accg[r] = bg;
-        }
-        for (int kc = 0; kc < nk; kc += KCH) {
-          if (nk > KCH) load_w(kc);
+          for (int r = 0; r < 16; ++r) {
+            accp[r] = bp;
+            accg[r] = bg;
+          }
+          for (int kc = 0; kc < nk; kc += KCH) {
+            if (nk > KCH) load_w(kc);
 #pragma unroll
-          for (int j = 0; j < KCH; ++j) {
-            if (kc + j >= nk) break;
-            const V8 zf = load8(&zs[(32 * s + l32) * ZR + 16 * (kc + j) + 8 * g]);
-            Mma<T, PREC>::step(accp, zf, wpf[j]);
-            Mma<T, PREC>::step(accg, zf, wgf[j]);
+            for (int j = 0; j < KCH; ++j) {
+              if (kc + j >= nk) break;
+              const V8 zf = load8(&zs[(32 * s + l32) * ZR + 16 * (kc + j) + 8 * g]);
+              Mma<T, PREC>::step(accp, zf, wpf[j]);
+              Mma<T, PREC>::step(accg, zf, wgf[j]);
+            }
+          }
+#pragma unroll
+          for (int rg = 0; rg < 4; ++rg) {
+            const int pt = 8 * rg + 4 * g;  // pixel within the sub-tile
+            const f32x4 m4 = *reinterpret_cast<const f32x4*>(&mk[32 * s + pt]);
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = accp[4 * rg + e] * sigmoid_acc(accg[4 * rg + e]) * m4[e];
+            store4(&ebuf[l32 * ER + 32 * s2 + pt], TypeOps<T>::from_f32(v));
           }
         }
+        wave_lds_sync();
+        // 16-byte stores, 4 * SPT lanes per channel row of 32 * SPT pixels
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          const int pt = 8 * rg + 4 * g;  // pixel within the sub-tile
-          const f32x4 m4 = *reinterpret_cast<const f32x4*>(&mk[32 * s + pt]);
-          f32x4 v;
+        for (int i = 0; i < 2 * SPT; ++i) {
+          const int c = lane + 64 * i;
+          const int crow = c / (4 * SPT), p0 = (c % (4 * SPT)) * 8;
+          const int chg = 32 * u + crow;
+          T* dst = chg < Ch ? a_cm : b_cm;
+          const int chh = chg < Ch ? chg : chg - Ch;
+          const int pl = 32 * s0 + p0;
+          T* drow = dst + ab_offset<T>((int64_t)tl.b * Ch + chh, tl.row, tl.c0 + pl, N, NP);
+          const V8 val = load8(&ebuf[crow * ER + p0]);
+          if (tl.c0 + pl + 8 <= N) {
+            store8(drow, val);
+          } else if (tl.c0 + pl < NP) {  // row tail: pixels N .. NP-1 are written as zeros
+            V8 v = val;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = accp[4 * rg + e] * sigmoid_acc(accg[4 * rg + e]) * m4[e];
-          store4(&ebuf[l32 * ER + 32 * s2 + pt], TypeOps<T>::from_f32(v));
+            for (int e = 0; e < 8; ++e)
+              if (tl.c0 + pl + e >= N) v[e] = TypeOps<T>::from_f32(0.f);
+            store8(drow, v);
+          }
         }
+        wave_lds_sync();
       }
-      wave_lds_sync();
-      // 16-byte stores, 4 * SPT lanes per channel row of 32 * SPT pixels
-#pragma unroll
-      for (int i = 0; i < 2 * SPT; ++i) {
-        const int c = lane + 64 * i;
-        const int crow = c / (4 * SPT), p0 = (c % (4 * SPT)) * 8;
-        const int chg = 32 * u + crow;
-        T* dst = chg < Ch ? a_cm : b_cm;
-        const int chh = chg < Ch ? chg : chg - Ch;
-        const int pl = 32 * s0 + p0;
-        T* drow = dst + ab_offset<T>((int64_t)tl.b * Ch + chh, tl.row, tl.c0 + pl, N, NP);
-        const V8 val = load8(&ebuf[crow * ER + p0]);
-        if (tl.c0 + pl + 8 <= N) {
-          store8(drow, val);
-        } else if (tl.c0 + pl < NP) {  // row tail: pixels N .. NP-1 are written as zeros
-          V8 v = val;
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (tl.c0 + pl + e >= N) v[e] = TypeOps<T>::from_f32(0.f);
-          store8(drow, v);
-        }
-      }
-      wave_lds_sync();
     }
     // output-gate items (unit uo, sub-tile s): acc = [channel][pixel], row = channel
     // 32uo + 8(r/4) + 4g + r%4, col = pixel 32s + l32; staged as [pixel][channel]
