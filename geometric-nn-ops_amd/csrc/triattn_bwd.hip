@@ -50,8 +50,9 @@ constexpr int BNT = 256;    // threads per workgroup (4 waves)
 constexpr int ROWB = 64;    // bytes per staged row (32 x 16-bit)
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Waves per SIMD that bwd_dq / bwd_dkdv keep registers for. Full-precision fp32 at D <= 32 fits three
-// (170 and 176 registers left to themselves; at N = 333 the two take 815 us together, with two 876).
+// Waves per SIMD that bwd_dq / bwd_dkdv keep registers for. Full-precision fp32 at D <= 32 takes three: held
+// to 168 registers, the kernels with a bias spill 2 (dq) and 5 (dk / dv) of the 170 and 176 that they
+// take otherwise (at N = 333 the two take 815 us together, with two waves 876).
 template <typename T, int DC, int PREC>
 constexpr int row_min_waves() { return DC > 2 ? 1 : sizeof(T) == 4 && DC == 1 && PREC == 1 ? 3 : 2; }
 

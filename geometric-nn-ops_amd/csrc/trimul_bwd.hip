@@ -637,7 +637,8 @@ int launch_proj_bwd(const gnn_trimul_proj_bwd_args& a, hipStream_t st) {
 // consecutive channels (acc_channel): dout and the saved gate are read, and d_go written, 16
 // bytes at a time straight from the accumulators; dy is staged in LDS, for its rows and for
 // d(on) = dy p_out_w, again [channel][pixel] blocks, whose per-pixel LayerNorm reductions meet in
-// LDS; d(o) leaves through LDS in whole rows. One workgroup fits a CU (256 registers), so nothing
+// LDS; d(o) leaves through LDS in whole rows. One workgroup fits a CU (256 registers; at 128 / 128
+// channels 5 spill in bf16 and 9 in fp16), so nothing
 // else hides a tile's loads: o travels a tile ahead in registers, and the LayerNorm takes all 512
 // threads. With both and the whole-row stores 108 -> 82 us. Weight fragments
 // stay in registers for the whole launch; the column sums of dy, d_go, d(on) x^ and d(on) stay
@@ -999,7 +1000,8 @@ int64_t gate_bwd_partials(int64_t rows, int64_t K) {
 
 int64_t trimul_proj_bwd_partials(int64_t rows) {
   const int64_t t = (rows + PB_TP - 1) / PB_TP;
-  // one workgroup fits a CU, as in trimul_out_bwd_partials
+  // as in trimul_out_bwd_partials (us with 256 / 512: N = 160 24.5 / 32.9, 384 78.5 / 86.6, 512 125 / 137, 768
+  // 262 / 264)
   const int64_t cap = t < 8 * PB_MAX_GRID ? PB_MAX_GRID / 2 : PB_MAX_GRID;
   return t < 1 ? 1 : (t > cap ? cap : t);
 }
@@ -1016,7 +1018,10 @@ int trimul_proj_bwd(const gnn_trimul_proj_bwd_args& a, hipStream_t st) {
 
 int64_t trimul_out_bwd_partials(int64_t B, int64_t N) {
   const int64_t t = B * N * ((N + OB_TP - 1) / OB_TP);
-  // one workgroup fits a CU: up to 8 tiles for each of 512, a single round of 256
+  // One workgroup fits a CU, so that a second round only repeats the first one's prologue: 256 for 256 CUs
+  // (a constant: the count is asked for without a device). From 4096 tiles on it stays at the 512 rows
+  // that callers of this count have been given; the round costs less there, if not nothing (us with
+  // 256 / 512, c_z = c_hidden = 128, bf16: N = 160 28.2 / 39.1, 384 82.5 / 92.5, 512 133 / 145, 768 274 / 285).
   const int64_t cap = t < 8 * OB_MAX_GRID ? OB_MAX_GRID / 2 : OB_MAX_GRID;
   return t < 1 ? 1 : (t > cap ? cap : t);
 }
