@@ -267,8 +267,9 @@ class AttnCall:
         a.dtype = _lib.DTYPE_CODE[q.dtype]
         a.precision = _lib.PRECISION_CODE["bf16x3" if precision == "tf32" else "ieee"]
         if bias is not None:
-            bias = TA.bias_for_kernel(a, bias, q.dtype)  # the layout the library's kernel reads
-        self.ws = TA.workspace_for(a, q.device)
+            bias = bias.to(q.dtype)
+            a.bias, a.bias_stride = bias.data_ptr(), _lib.I64x4(*(bias.stride(i) for i in (0, 2, 3, 4)))
+        bias, self.ws = TA.bias_and_workspace(a, bias, q.device)  # the layout the library's kernel reads
         self.args = a
         self.keep = (q, k, v, bias, mask)
 

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(RNT, 4) void bwd_dkdv_row_kernel(const gnn_triattn_
 // gradient: N = 320 121 against 142 us, 384 185 against 206; N = 128 41 against 33, 256 83 against 69).
 // LDS bounds N: 264 bytes per query and 2 KB per wave.
 // The same call on the two kernels: N = 256 104 -> 74 us, 384 247 -> 185, 512 537 -> 372. At N = 512 the
-// vector ALU is busy 39% of the cycles (exponentials, conversions), the matrix unit 25% and LDS 35%; the
+// vector ALU is busy 36% of the cycles (exponentials, conversions), the matrix unit 23% and LDS 33%; the
 // rest is the chain of a tile (fragments, products, exponentials, the tile's way through LDS, dQ), which
 // two waves per SIMD do not hide. Interleaved with the tile's C++ accesses (ordered by the compiler) and
 // with the mask's branches inside the loop it took 453 us.

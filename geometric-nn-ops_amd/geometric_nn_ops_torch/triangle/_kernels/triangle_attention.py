@@ -86,21 +86,6 @@ def _set_bias(args, bias: torch.Tensor) -> None:
     args.bias_stride = _lib.I64x4(bias.stride(0), bias.stride(2), bias.stride(3), bias.stride(4))
 
 
-def bias_for_kernel(args, bias: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """Points ``args`` (shapes and dtype already set) at the ``[B, 1, H, N, N]`` pair bias in
-    ``dtype`` and returns the tensor the kernel will read (the caller keeps it alive). The
-    library asks for fragment-order scratch exactly when its row-resident kernel runs, and
-    that kernel's pre-pass reads any strides; otherwise the bias is given the unit key stride
-    and aligned pitch the tiled kernel needs. Asking the library keeps this decision in one
-    place (``triattn_row_applicable`` in the C sources)."""
-    bias = bias.to(dtype)
-    _set_bias(args, bias)
-    if _lib.load().gnn_triattn_workspace_bytes(ctypes.byref(args)) == 0:
-        bias = _prepare_bias(bias, dtype)
-        _set_bias(args, bias)
-    return bias
-
-
 def workspace_for(args, device) -> torch.Tensor | None:
     """Sets ``args.workspace`` to a fresh scratch tensor of the size the library asks for
     (``None`` when the call needs none); the caller keeps the tensor alive over the launch."""
@@ -110,6 +95,21 @@ def workspace_for(args, device) -> torch.Tensor | None:
     ws = torch.empty(nbytes, device=device, dtype=torch.uint8)
     args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
     return ws
+
+
+def bias_and_workspace(args, bias, device):
+    """``(bias, workspace)`` for a forward whose ``args`` (shapes and dtype set) point at the
+    ``[B, 1, H, N, N]`` pair bias; the caller keeps both alive. The library asks for fragment-order
+    scratch exactly when its row-resident kernel runs, and that kernel's pre-pass reads any strides;
+    otherwise the bias takes the layout that the tiled kernel needs. Asking the library keeps this
+    decision in one place (``triattn_row_applicable`` in the C sources)."""
+    if bias is None:
+        return None, None
+    ws = workspace_for(args, device)
+    if ws is None:
+        bias = _prepare_bias(bias, bias.dtype)
+        _set_bias(args, bias)
+    return bias, ws
 
 
 def triangle_attention_hip(q, k, v, bias=None, mask=None, scale=None, dynamic=False, use_exp2=False,
@@ -166,12 +166,7 @@ def triangle_attention_hip(q, k, v, bias=None, mask=None, scale=None, dynamic=Fa
     args.scale = float(scale)
     args.mask_value = rounded_mask_value(q.dtype) if mask_value is None else float(mask_value)
 
-    ws = None
-    if bias is not None:  # scratch where the row-resident kernel runs, the tiled kernel's layout elsewhere
-        ws = workspace_for(args, q.device)
-        if ws is None:
-            bias = _prepare_bias(bias, q.dtype)
-            _set_bias(args, bias)
+    bias, ws = bias_and_workspace(args, bias, q.device)
     _lib.call("gnn_triattn_fwd", args, q.device)
     del ws
     if Dp != D:
